@@ -20,7 +20,21 @@
 namespace nsa {
 
 constexpr int kSelWaveCols = 16;
-constexpr int kSelMaxT = 17;  // timesteps a 16-column group can touch (hpg = 1)
+// timesteps a wave's 16 columns can touch (column groups start at multiples of 16)
+__host__ __device__ inline int sel_max_t(int hpg) {
+  return hpg % 16 == 0 ? 1 : 16 % hpg == 0 ? 16 / hpg : 15 / hpg + 2;
+}
+__host__ __device__ inline int sel_words(int nblk) { return (nblk + 31) / 32; }
+// LDS words of one wave's block bitmaps: the union's, then one per timestep
+__host__ __device__ inline int sel_wave_words(int hpg, int nblk) { return (sel_max_t(hpg) + 1) * sel_words(nblk); }
+
+// Keys per tile.  A tile's K / V fragments and their successors' loads live in registers:
+// 64 keys in bf16; in fp32, at twice the bytes, a 64-key tile spilled (dQ 134 registers at
+// dk = 64, 547 at dk = 192) while its products (32 cycles per 16 x 16 x 4) cover the
+// latency of a 32-key tile's loads several times over (B4 H16 G4 T2048 dk = dv = 64: dQ 676
+// -> 561 us, now two waves per SIMD instead of one; forward 437 -> 424 us at four).
+template <typename T>
+constexpr int kSelTile = sizeof(typename Store<T>::type) == 2 ? 64 : 32;
 
 // Workgroup id -> logical id such that each XCD (ids dispatched round-robin over 8)
 // receives a contiguous range of logical ids.
@@ -30,42 +44,38 @@ __device__ __forceinline__ int xcd_contiguous(int i, int n) {
   return (xcd < rem ? xcd * (base + 1) : rem * (base + 1) + (xcd - rem) * base) + k;
 }
 
-// Per-wave bookkeeping: the timesteps of the wave's columns, their cleaned lists and
-// the union bitmap of their blocks.
+// Per-wave bookkeeping: the timesteps of the wave's columns.
 struct SelWave {
   int t_first, nt;
 };
 
-template <typename T, bool DQ>
-__device__ __forceinline__ void sel_wave_setup(const AttnArgs& a, int bg, int f0, int* lst, uint32_t* bits,
+// The wave's block bitmaps in LDS: bits [nwords] of the union its tile cursor walks, tb
+// [nt][nwords] of each timestep's own selection.  With several timesteps per wave (fewer
+// than 16 heads per group) a column tests its block with one LDS read a tile; a scan of
+// the timestep's list took a serial chain of up to nslots LDS reads, and more time than
+// the tile's products (bf16 forward, B3 H16 G4 T1537 dk = dv = 64: 80 -> 61 us).
+__device__ __forceinline__ void sel_wave_setup(const AttnArgs& a, int bg, int f0, uint32_t* bits, uint32_t* tb,
                                                SelWave& w, int lane) {
   const int ncols = a.Tq * a.hpg;
   const int flast = min(f0 + kSelWaveCols, ncols) - 1;
   w.t_first = f0 / a.hpg;
   w.nt = flast / a.hpg - w.t_first + 1;
-  const int nwords = (a.nblk + 31) / 32;
-  for (int i = lane; i < nwords; i += 64) bits[i] = 0;
-  __builtin_amdgcn_wave_barrier();
+  const int nwords = sel_words(a.nblk);
+  for (int i = lane; i < w.nt * nwords; i += 64) tb[i] = 0;
+  wave_lds_sync();
   const int* selrow = a.sel + ((int64_t)bg * a.Tq + w.t_first) * a.nslots;
   const int total = w.nt * a.nslots;
   for (int i = lane; i < total; i += 64) {
     const int v = selrow[i];
-    lst[i] = v;
-    if (v >= 0) atomicOr(&bits[v >> 5], 1u << (v & 31));
+    if (v >= 0) atomicOr(&tb[i / a.nslots * nwords + (v >> 5)], 1u << (v & 31));
   }
-  __builtin_amdgcn_s_waitcnt(0);
-  __builtin_amdgcn_wave_barrier();
-}
-
-// does the column's timestep select block `blk`? (its list is ascending, -1 padded)
-__device__ __forceinline__ bool sel_has(const int* l, int nslots, int blk) {
-  bool has = false;
-  for (int j = 0; j < nslots; ++j) {
-    const int v = l[j];
-    if (v == blk) has = true;
-    if (v < 0 || v >= blk) break;
+  wave_lds_sync();
+  for (int i = lane; i < nwords; i += 64) {
+    uint32_t u = 0;
+    for (int t = 0; t < w.nt; ++t) u |= tb[t * nwords + i];
+    bits[i] = u;
   }
-  return has;
+  wave_lds_sync();
 }
 
 // ============================================================== forward
@@ -80,8 +90,8 @@ template <typename T, int DK, int DV>
 struct SelFwdShared {
   static constexpr int KC = Elem<T>::kKChunk;
   static constexpr int CK = CFrag<T>::kKeys;
-  static constexpr int NKF = 4 * (DK / KC);          // K rowfrags of a 64-key tile
-  static constexpr int NVF = (64 / CK) * (DV / 16);  // V^T colfrags
+  static constexpr int NKF = kSelTile<T> / 16 * (DK / KC);     // K rowfrags of a tile
+  static constexpr int NVF = (kSelTile<T> / CK) * (DV / 16);  // V^T colfrags
   static constexpr bool kOn = sizeof(typename Store<T>::type) == 2;
   static constexpr int kLdsBytes = kOn ? (NKF + NVF) * 1024 : 0;
 };
@@ -97,10 +107,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   constexpr int NKC = DK / KC;
   constexpr int CK = CFrag<T>::kKeys;
   constexpr int CT = CK / 16;
-  constexpr int NWD = kSelMaxBlocks / 32;
-  __shared__ int s_lst[4][kSelMaxT * 64];
-  __shared__ uint32_t s_bits[4][NWD];
-  extern __shared__ __attribute__((aligned(16))) uint4 sel_tile[];  // [NKF + NVF][64] (phase 1)
+  constexpr int TK = kSelTile<T>, NKS = TK / 16;
+  // [NKF + NVF][64] (phase 1), then per wave the block bitmaps, then the common blocks'
+  extern __shared__ __attribute__((aligned(16))) uint4 sel_tile[];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform control below
@@ -113,13 +122,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   const int f0 = (L % ncoltiles) * 64 + wave * kSelWaveCols;
   const bool active = f0 < ncols;  // idle waves still meet the phase-1 barriers
   const float scale2 = a.scale * kLog2e;
-  const int nwords = (a.nblk + 31) / 32;
+  const int nwords = sel_words(a.nblk);
+  const int wwords = sel_wave_words(hpg, a.nblk);
 
   SelWave w{0, 0};
-  int* lst = s_lst[wave];
-  uint32_t* bits = s_bits[wave];
+  uint32_t* maps = reinterpret_cast<uint32_t*>(sel_tile) + SH::kLdsBytes / 4;
+  uint32_t* bits = maps + wave * wwords;
+  uint32_t* tb = bits + nwords;
   if (active) {
-    sel_wave_setup<T, false>(a, bg, f0, lst, bits, w, lane);
+    sel_wave_setup(a, bg, f0, bits, tb, w, lane);
   } else if (SH::kOn) {
     for (int i = lane; i < nwords; i += 64) bits[i] = 0;
   }
@@ -129,7 +140,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   const int colt = colv ? f / hpg : w.t_first;
   const int colh = colv ? grp * hpg + f % hpg : grp * hpg;
   const int t_last = w.t_first + w.nt - 1 + a.q0;  // absolute positions: row r is at a.q0 + r
-  const int* mylst = lst + (colt - w.t_first) * a.nslots;
+  const uint32_t* mybits = tb + (colt - w.t_first) * nwords;  // the column's own selection
 
   const S* qp = reinterpret_cast<const S*>(a.q) + b * a.sq_b + (int64_t)colh * a.sq_h + (int64_t)colt * a.sq_t;
   uint4 qf[NKC];
@@ -145,22 +156,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   float m2 = -INFINITY, mtrue = -INFINITY, lsum = 0.f;  // exponent reference, true maximum, sum
   const bool one_t = w.nt == 1;
 
-  // masking and the online softmax of one tile's S^T (keys key0 .. key0 + 63 of block blk
+  // masking and the online softmax of one tile's S^T (keys key0 .. key0 + TK - 1 of block blk
   // [blk_lo, blk_hi)); returns the packed P^T fragments
-  auto softmax_tile = [&](f32x4 (&st)[4], int key0, int blk, int blk_hi, uint4 (&pf)[64 / CK])
+  auto softmax_tile = [&](f32x4 (&st)[NKS], int key0, int blk, int blk_hi, uint4 (&pf)[TK / CK])
                           __attribute__((always_inline)) {
     const int blk_lo = blk * a.lprime;
-    const bool colsel = colv && (one_t || sel_has(mylst, a.nslots, blk));
+    const bool colsel = colv && (one_t || ((mybits[blk >> 5] >> (blk & 31)) & 1));
     // end of the keys of this block the lane's column sees (blk_lo when none)
     const int kend = colsel ? max(blk_lo, a.causal ? min(blk_hi, colt + a.q0 + 1) : blk_hi) : blk_lo;
-    const bool all_visible = one_t && colv && (!a.causal || key0 + 63 <= w.t_first + a.q0) && key0 >= blk_lo &&
-                             key0 + 63 < blk_hi && f0 + kSelWaveCols <= ncols;
+    const bool all_visible = one_t && colv && (!a.causal || key0 + TK - 1 <= w.t_first + a.q0) && key0 >= blk_lo &&
+                             key0 + TK - 1 < blk_hi && f0 + kSelWaveCols <= ncols;
     float mx = -INFINITY;
     // lane-visible keys of this block: [blk_lo, kend); branch-free test per element
     const uint32_t span = all_visible ? 0xffffffffu : (uint32_t)(kend - blk_lo);
     const int kb = key0 + 4 * g4 - blk_lo;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
+    for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const bool ok = (uint32_t)(kb + ks * 16 + i) < span;
@@ -185,7 +196,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
     const float nref = m2 == -INFINITY ? 0.f : -m2;
     float rs = 0.f;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
+    for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float p = fast_exp2(mul_add_rounded(st[ks][i], scale2, nref));
@@ -194,14 +205,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
       }
     lsum += wave_sum16(rs);
 #pragma unroll
-    for (int kc2 = 0; kc2 < 64 / CK; ++kc2) pf[kc2] = CFrag<T>::pack(st[kc2 * CT], st[kc2 * CT + CT - 1]);
+    for (int kc2 = 0; kc2 < TK / CK; ++kc2) pf[kc2] = CFrag<T>::pack(st[kc2 * CT], st[kc2 * CT + CT - 1]);
   };
 
   // ---- phase 1: the workgroup's common blocks, one LDS copy per tile -----------------
-  __shared__ uint32_t s_common[SH::kOn ? NWD : 1];
+  uint32_t* s_common = maps + 4 * wwords;
   if constexpr (SH::kOn) {
     __syncthreads();  // every wave's bitmap is written
-    for (int i = threadIdx.x; i < nwords; i += 256) s_common[i] = s_bits[0][i] & s_bits[1][i] & s_bits[2][i] & s_bits[3][i];
+    for (int i = threadIdx.x; i < nwords; i += 256)
+      s_common[i] = maps[i] & maps[wwords + i] & maps[2 * wwords + i] & maps[3 * wwords + i];
     __syncthreads();
     const int t_max = (min((L % ncoltiles) * 64 + 64, ncols) - 1) / hpg + a.q0;  // the workgroup's last position
     for (int wd = 0; wd < nwords; ++wd) {
@@ -211,7 +223,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
         word &= word - 1;
         const int lo = blk * a.lprime;
         const int blk_hi = min(lo + a.lprime, a.Tkv);
-        for (int key0 = lo & ~31; key0 < blk_hi && !(a.causal && key0 > t_max); key0 += 64) {
+        for (int key0 = lo & ~31; key0 < blk_hi && !(a.causal && key0 > t_max); key0 += TK) {
           for (int fr = wave; fr < SH::NKF + SH::NVF; fr += 4) {
             const S* src;
             if (fr < SH::NKF) {
@@ -226,17 +238,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
           __builtin_amdgcn_s_waitcnt(0);
           __syncthreads();
           if (active) {
-            f32x4 st[4];
+            f32x4 st[NKS];
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
+            for (int ks = 0; ks < NKS; ++ks) {
               st[ks] = zero4();
 #pragma unroll
               for (int kc = 0; kc < NKC; ++kc) st[ks] = Mma<T>::run(st[ks], sel_tile[(ks * NKC + kc) * 64 + lane], qf[kc]);
             }
-            uint4 pf[64 / CK];
+            uint4 pf[TK / CK];
             softmax_tile(st, key0, blk, blk_hi, pf);
 #pragma unroll
-            for (int kc2 = 0; kc2 < 64 / CK; ++kc2)
+            for (int kc2 = 0; kc2 < TK / CK; ++kc2)
 #pragma unroll
               for (int j = 0; j < DV / 16; ++j)
                 oacc[j] = Mma<T>::run(oacc[j], sel_tile[(SH::NKF + kc2 * (DV / 16) + j) * 64 + lane], pf[kc2]);
@@ -250,12 +262,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
 
   // ---- phase 2: the rest of the wave's union, straight from L2 --------------------------
   // Tile cursor over the union bitmap (wave-uniform scalar state).  Tiles start on a
-  // 32-key boundary (the C-permuted chunks of vt / kn) and cover 64 keys.
+  // 32-key boundary (the C-permuted chunks of vt / kn) and cover TK keys.
   int c_wd = -1, c_blk = -1, c_key0 = 0, c_hi = 0;
   uint32_t c_word = 0;
   auto advance = [&]() -> bool {
     if (c_blk >= 0) {
-      c_key0 += 64;
+      c_key0 += TK;
       if (c_key0 < c_hi && !(a.causal && c_key0 > t_last)) return true;
     }
     while (c_word == 0) {
@@ -274,17 +286,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   // K fragments of a tile (S^T = K Q^T) and V^T fragments (O^T += V^T P^T): the next
   // tile's K is requested as soon as the current S^T is issued, its V as soon as the
   // current P V is, so the loads overlap the softmax and the products.
-  uint4 kf[4][NKC], vf[64 / CK][DV / 16];
+  uint4 kf[NKS][NKC], vf[TK / CK][DV / 16];
   auto load_k = [&](int key0) {
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
+    for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
       for (int kc = 0; kc < NKC; ++kc)
         kf[ks][kc] = ld_rowfrag<T>(krf, (key0 >> 4) + ks, kc, DK, lane);
   };
   auto load_v = [&](int key0) {
 #pragma unroll
-    for (int kc2 = 0; kc2 < 64 / CK; ++kc2)
+    for (int kc2 = 0; kc2 < TK / CK; ++kc2)
 #pragma unroll
       for (int j = 0; j < DV / 16; ++j)
         vf[kc2][j] = ld_colfrag<T>(vcf, key0 / CK + kc2, j, DV, lane);
@@ -299,19 +311,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
     const int key0 = c_key0, blk = c_blk;
     const int blk_hi = c_hi;
     // S^T[key, col] for the 64 keys of this tile
-    f32x4 st[4];
+    f32x4 st[NKS];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
+    for (int ks = 0; ks < NKS; ++ks) {
       st[ks] = zero4();
 #pragma unroll
       for (int kc = 0; kc < NKC; ++kc) st[ks] = Mma<T>::run(st[ks], kf[ks][kc], qf[kc]);
     }
     const bool have_next = advance();
     if (have_next) load_k(c_key0);
-    uint4 pf[64 / CK];
+    uint4 pf[TK / CK];
     softmax_tile(st, key0, blk, blk_hi, pf);
 #pragma unroll
-    for (int kc2 = 0; kc2 < 64 / CK; ++kc2) {
+    for (int kc2 = 0; kc2 < TK / CK; ++kc2) {
 #pragma unroll
       for (int j = 0; j < DV / 16; ++j) oacc[j] = Mma<T>::run(oacc[j], vf[kc2][j], pf[kc2]);
     }
@@ -337,15 +349,19 @@ template <typename T, int DK, int DV>
 void launch_attn_sel_fwd(const AttnArgs& a, hipStream_t s) {
   using SH = SelFwdShared<T, DK, DV>;
   const int ncoltiles = (a.Tq * a.hpg + 63) / 64;
-  if (SH::kLdsBytes > 0)
-    allow_dynamic_lds(reinterpret_cast<const void*>(&attn_sel_fwd_kernel<T, DK, DV>), SH::kLdsBytes);
-  hipLaunchKernelGGL((attn_sel_fwd_kernel<T, DK, DV>), dim3(ncoltiles * a.B * a.G), dim3(256), SH::kLdsBytes, s, a,
-                     ncoltiles);
+  // at most 40 KB of tile + 36 KB of bitmaps (hpg = 1, kSelMaxBlocks): two workgroups per CU
+  const size_t lds = SH::kLdsBytes + 4 * (size_t)(4 * sel_wave_words(a.hpg, a.nblk) + sel_words(a.nblk));
+  allow_dynamic_lds(reinterpret_cast<const void*>(&attn_sel_fwd_kernel<T, DK, DV>), lds);
+  hipLaunchKernelGGL((attn_sel_fwd_kernel<T, DK, DV>), dim3(ncoltiles * a.B * a.G), dim3(256), lds, s, a, ncoltiles);
 }
 
 // ============================================================== dQ
+// 16-byte pieces of one wave's staged K tile (bf16; fp32 stages nothing)
+template <typename T, int DK>
+constexpr int sel_dq_stage() { return sizeof(typename Store<T>::type) == 2 ? kSelTile<T> / 16 * (DK / Elem<T>::kKChunk) * 64 : 0; }
+
 template <typename T, int DK, int DV>
-__global__ __launch_bounds__(256) void attn_sel_dq_kernel(AttnArgs a, int ncoltiles) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DK <= 64 ? 2 : 1))) void attn_sel_dq_kernel(AttnArgs a, int ncoltiles) {
   using S = typename Store<T>::type;
   constexpr int EPF = Elem<T>::kPerFrag;
   constexpr int KC = Elem<T>::kKChunk;
@@ -353,10 +369,11 @@ __global__ __launch_bounds__(256) void attn_sel_dq_kernel(AttnArgs a, int ncolti
   constexpr int NVC = DV / KC;
   constexpr int CK = CFrag<T>::kKeys;
   constexpr int CT = CK / 16;
-  __shared__ int s_lst[4][kSelMaxT * 64];
-  __shared__ uint32_t s_bits[4][kSelMaxBlocks / 32];
-  // bf16: each wave's staged K rows of one 64-key tile (rowfrag order)
-  __shared__ __attribute__((aligned(16))) uint4 s_kt[4][sizeof(S) == 2 ? 4 * NKC * 64 : 1];
+  constexpr int TK = kSelTile<T>, NKS = TK / 16;
+  // bf16: each wave's staged K rows of one tile (rowfrag order); then per wave the
+  // block bitmaps
+  constexpr int NST = sel_dq_stage<T, DK>();
+  extern __shared__ __attribute__((aligned(16))) uint4 sel_dq_lds[];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform control below
@@ -371,16 +388,17 @@ __global__ __launch_bounds__(256) void attn_sel_dq_kernel(AttnArgs a, int ncolti
   const float scale2 = a.scale * kLog2e;
 
   SelWave w;
-  int* lst = s_lst[wave];
-  uint32_t* bits = s_bits[wave];
-  sel_wave_setup<T, true>(a, bg, f0, lst, bits, w, lane);
+  const int nwords = sel_words(a.nblk);
+  uint32_t* bits = reinterpret_cast<uint32_t*>(sel_dq_lds + 4 * NST) + wave * sel_wave_words(hpg, a.nblk);
+  uint32_t* tb = bits + nwords;
+  sel_wave_setup(a, bg, f0, bits, tb, w, lane);
 
   const int f = f0 + c16;
   const bool colv = f < ncols;
   const int colt = colv ? f / hpg : w.t_first;
   const int colh = colv ? grp * hpg + f % hpg : grp * hpg;
   const int t_last = w.t_first + w.nt - 1;
-  const int* mylst = lst + (colt - w.t_first) * a.nslots;
+  const uint32_t* mybits = tb + (colt - w.t_first) * nwords;  // the column's own selection
 
   uint4 qf[NKC], dof[NVC];
   {
@@ -412,7 +430,6 @@ __global__ __launch_bounds__(256) void attn_sel_dq_kernel(AttnArgs a, int ncolti
   f32x4 dqa[DK / 16];
 #pragma unroll
   for (int j = 0; j < DK / 16; ++j) dqa[j] = zero4();
-  const int nwords = (a.nblk + 31) / 32;
   const bool one_t = w.nt == 1;
 
   // wave-uniform tile cursor over the union bitmap (as in the forward)
@@ -420,7 +437,7 @@ __global__ __launch_bounds__(256) void attn_sel_dq_kernel(AttnArgs a, int ncolti
   uint32_t c_word = 0;
   auto advance = [&]() -> bool {
     if (c_blk >= 0) {
-      c_key0 += 64;
+      c_key0 += TK;
       if (c_key0 < c_hi && !(a.causal && c_key0 > t_last)) return true;
     }
     while (c_word == 0) {
@@ -445,12 +462,12 @@ __global__ __launch_bounds__(256) void attn_sel_dq_kernel(AttnArgs a, int ncolti
   // The next tile's loads are issued once this tile's S^T and dP^T are, so they overlap
   // the softmax and the dQ products.
   constexpr bool kLdsK = sizeof(S) == 2;
-  constexpr int NVL = 4 * NVC;  // V fragment loads per tile
-  uint4 kf[4][NKC], vf[4][NVC], knf[64 / CK][DK / 16];
-  uint4* kst = s_kt[wave];
+  constexpr int NVL = NKS * NVC;  // V fragment loads per tile
+  uint4 kf[NKS][NKC], vf[NKS][NVC], knf[TK / CK][DK / 16];
+  uint4* kst = sel_dq_lds + wave * NST;
   auto load_k = [&](int key0) {
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
+    for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
       for (int kc = 0; kc < NKC; ++kc) {
         if constexpr (kLdsK)
@@ -461,7 +478,7 @@ __global__ __launch_bounds__(256) void attn_sel_dq_kernel(AttnArgs a, int ncolti
   };
   auto load_v = [&](int key0) {
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
+    for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
       for (int kc = 0; kc < NVC; ++kc) vf[ks][kc] = ld_rowfrag<T>(vrf, (key0 >> 4) + ks, kc, DV, lane);
   };
@@ -489,11 +506,11 @@ __global__ __launch_bounds__(256) void attn_sel_dq_kernel(AttnArgs a, int ncolti
       __builtin_amdgcn_wave_barrier();
       asm volatile("" ::: "memory");
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks)
+      for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
         for (int kc = 0; kc < NKC; ++kc) kf[ks][kc] = kst[(ks * NKC + kc) * 64 + lane];
 #pragma unroll
-      for (int kc2 = 0; kc2 < 64 / CK; ++kc2)
+      for (int kc2 = 0; kc2 < TK / CK; ++kc2)
 #pragma unroll
         for (int j = 0; j < DK / 16; ++j) knf[kc2][j] = knf_lds(kc2, j);
       wave_lds_sync();
@@ -519,39 +536,39 @@ __global__ __launch_bounds__(256) void attn_sel_dq_kernel(AttnArgs a, int ncolti
     // the join.  bf16: the K copy goes out now, a whole tile ahead of its use.
     const int next_key0 = have_next ? c_key0 : key0;
     if (kLdsK) load_k(next_key0);
-    f32x4 st[4], dp[4];
+    f32x4 st[NKS], dp[NKS];
     // S^T first (its operands are in registers), then dP^T, whose V rows may still be
     // arriving
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
+    for (int ks = 0; ks < NKS; ++ks) {
       st[ks] = zero4();
 #pragma unroll
       for (int kc = 0; kc < NKC; ++kc) st[ks] = Mma<T>::run(st[ks], kf[ks][kc], qf[kc]);
     }
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
+    for (int ks = 0; ks < NKS; ++ks) {
       dp[ks] = zero4();
 #pragma unroll
       for (int kc = 0; kc < NVC; ++kc) dp[ks] = Mma<T>::run(dp[ks], vf[ks][kc], dof[kc]);
     }
     if constexpr (!kLdsK) {
 #pragma unroll
-      for (int kc2 = 0; kc2 < 64 / CK; ++kc2)
+      for (int kc2 = 0; kc2 < TK / CK; ++kc2)
 #pragma unroll
         for (int j = 0; j < DK / 16; ++j) knf[kc2][j] = ld_colfrag<T>(kcf, key0 / CK + kc2, j, DK, lane);
       load_k(next_key0);
     }
     load_v(next_key0);
 
-    const bool colsel = colv && (one_t || sel_has(mylst, a.nslots, blk));
+    const bool colsel = colv && (one_t || ((mybits[blk >> 5] >> (blk & 31)) & 1));
     // end of the keys of this block the lane's column sees (blk_lo when none)
     const int kend = colsel ? max(blk_lo, a.causal ? min(blk_hi, colt + 1) : blk_hi) : blk_lo;
-    const bool all_visible = one_t && colv && (!a.causal || key0 + 63 <= w.t_first) && key0 >= blk_lo &&
-                             key0 + 63 < blk_hi && f0 + kSelWaveCols <= ncols;
+    const bool all_visible = one_t && colv && (!a.causal || key0 + TK - 1 <= w.t_first) && key0 >= blk_lo &&
+                             key0 + TK - 1 < blk_hi && f0 + kSelWaveCols <= ncols;
     const uint32_t span = all_visible ? 0xffffffffu : (uint32_t)(kend - blk_lo);
     const int kb = key0 + 4 * g4 - blk_lo;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
+    for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const bool ok = (uint32_t)(kb + ks * 16 + i) < span;
@@ -559,7 +576,7 @@ __global__ __launch_bounds__(256) void attn_sel_dq_kernel(AttnArgs a, int ncolti
         st[ks][i] = p * (dp[ks][i] - dl);  // dS^T
       }
 #pragma unroll
-    for (int kc2 = 0; kc2 < 64 / CK; ++kc2) {
+    for (int kc2 = 0; kc2 < TK / CK; ++kc2) {
       const uint4 sf = CFrag<T>::pack(st[kc2 * CT], st[kc2 * CT + CT - 1]);
 #pragma unroll
       for (int j = 0; j < DK / 16; ++j) dqa[j] = Mma<T>::run(dqa[j], knf[kc2][j], sf);
@@ -731,7 +748,9 @@ void launch_attn_sel_dq(const AttnArgs& a, hipStream_t s) {
     }
   }
   const int ncoltiles = (a.Tq * a.hpg + 63) / 64;
-  hipLaunchKernelGGL((attn_sel_dq_kernel<T, DK, DV>), dim3(ncoltiles * a.B * a.G), dim3(256), 0, s, a, ncoltiles);
+  const size_t lds = (size_t)64 * sel_dq_stage<T, DK>() + (size_t)16 * sel_wave_words(a.hpg, a.nblk);
+  allow_dynamic_lds(reinterpret_cast<const void*>(&attn_sel_dq_kernel<T, DK, DV>), lds);
+  hipLaunchKernelGGL((attn_sel_dq_kernel<T, DK, DV>), dim3(ncoltiles * a.B * a.G), dim3(256), lds, s, a, ncoltiles);
 }
 
 }  // namespace nsa
