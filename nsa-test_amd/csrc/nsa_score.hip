@@ -30,6 +30,8 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <type_traits>
+
 #include "nsa_attn.h"
 #include "nsa_device.h"
 
@@ -242,6 +244,64 @@ __global__ __launch_bounds__(256) void score_logits_kernel(ScoreArgs a) {
   }
 }
 
+// The same chains for a call of few query rows (decoding: the heads of one timestep per
+// group), one 16-block x 16-row MFMA tile per wave.  A 128-row tile would be mostly padding
+// there, and its workgroup walks 64 blocks serially through LDS; here every wave loads its
+// operands straight into registers, all of its loads in flight at once.  The four lanes of
+// a row load the same 16-byte pieces (one request) and each picks the elements of its k
+// slot.  Every column tile is computed, visible or not: the rows kernel masks.
+// Up to kLgFewRows query rows of a group (four row tiles, each reading K once more; the
+// 128-row tile is at least half padding there).  Bound by launch and load latency.
+constexpr int kLgFewRows = 64;
+
+template <typename S>
+__global__ __launch_bounds__(256) void score_logits_few_kernel(ScoreArgs a) {
+  constexpr int EPL = 16 / sizeof(S);
+  const int lane = threadIdx.x & 63, li = lane & 15, kk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int bg = blockIdx.z, b = bg / a.G, g = bg % a.G;
+  const int hpg = a.hpg;
+  const int Rall = a.T * hpg;
+  const int col0 = blockIdx.x * 64 + wave * 16, row0 = blockIdx.y * 16;
+  const int r = min(row0 + li, Rall - 1);
+  const S* qrow = reinterpret_cast<const S*>(a.q) + b * a.sq_b + (int64_t)(g * hpg + r % hpg) * a.sq_h +
+                  (int64_t)(r / hpg) * a.sq_t;
+  const S* kcol = reinterpret_cast<const S*>(a.kc) + b * a.sk_b + g * a.sk_g + (int64_t)min(col0 + li, a.NB - 1) * a.sk_i;
+  // element 4 j + kk of a piece, as fp32
+  auto pick = [&](const uint4& v, int j) __attribute__((always_inline)) -> float {
+    const uint32_t x = v.x, y = v.y, z = v.z, w = v.w;
+    if constexpr (sizeof(S) == 4) {
+      const uint32_t lo = kk & 1 ? y : x, hi = kk & 1 ? w : z;
+      return __uint_as_float(kk & 2 ? hi : lo);
+    } else {
+      const uint32_t p0 = kk & 2 ? y : x, p1 = kk & 2 ? w : z;
+      const uint32_t u = j == 0 ? p0 : p1;
+      return __uint_as_float(kk & 1 ? u & 0xffff0000u : u << 16);
+    }
+  };
+  f32x4 acc = zero4();
+  auto run = [&](int e0, auto np) __attribute__((always_inline)) {
+    constexpr int NP = decltype(np)::value;  // pieces in flight per operand
+    uint4 kv[NP], qv[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      kv[p] = *reinterpret_cast<const uint4*>(kcol + e0 + p * EPL);
+      qv[p] = *reinterpret_cast<const uint4*>(qrow + e0 + p * EPL);
+    }
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int j = 0; j < EPL / 4; ++j)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(pick(kv[p], j), pick(qv[p], j), acc, 0, 0, 0);
+  };
+  int e0 = 0;  // dk is a multiple of a piece (16-byte rows)
+  for (; e0 + 8 * EPL <= a.dk; e0 += 8 * EPL) run(e0, std::integral_constant<int, 8>{});
+  for (; e0 < a.dk; e0 += EPL) run(e0, std::integral_constant<int, 1>{});
+  if (row0 + li < Rall)
+    *reinterpret_cast<float4*>(a.lg + ((int64_t)bg * Rall + row0 + li) * a.ncs + col0 + kk * 4) =
+        make_float4(acc[0] * a.scale, acc[1] * a.scale, acc[2] * a.scale, acc[3] * a.scale);
+}
+
 // ------------------------------------------------------------------ rows ----
 // One wave per (batch, group, timestep): a workgroup of NW waves takes NW consecutive
 // timesteps, and after the block ends are staged in LDS no wave waits for another.  A
@@ -262,10 +322,16 @@ __global__ __launch_bounds__(256) void score_logits_kernel(ScoreArgs a) {
 // at t are not read (the logits kernel computed every visible block, and block 0).
 constexpr int kRowsWaves = 8;
 
-template <int NQ, bool FAST9>
-__global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu(NQ == 8 ? 4 : 1))) void score_rows_kernel(ScoreArgs a) {
+//
+// HEADS: a workgroup takes one timestep and its waves the heads (head hh on wave hh % NW),
+// for calls with too few timesteps to occupy the chip with a wave each.  Every row's Eq. 9
+// scores go to LDS; wave 0 then adds them in head order and takes the top-n, so the sums
+// and the indices are those of the serial walk.
+template <int NQ, bool FAST9, bool HEADS>
+__global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu(NQ == 8 && !HEADS ? 4 : 1))) void score_rows_kernel(ScoreArgs a) {
   // LDS: sbe [NQ * 256] block ends (INT_MAX past NB); generic remap only, per wave:
-  // row copy [NQ * 256] + Eq. 10 sums [nsel rounded up to 4]
+  // row copy [NQ * 256] + Eq. 10 sums [nsel rounded up to 4]; HEADS: Eq. 9 scores [hpg][nsel
+  // rounded up to 4] at the end
   extern __shared__ float lds[];
   constexpr bool kPrefetch = NQ <= 8;  // registers for the next row's pieces
   const int tid = threadIdx.x, lane = tid & 63;
@@ -276,12 +342,14 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
   int* sbe = reinterpret_cast<int*>(lds);
   for (int i = tid; i < NQ * 256; i += blockDim.x) sbe[i] = i < NB ? a.block_ends[i] : 0x7fffffff;
   __syncthreads();
-  const int t = blockIdx.x * NW + wave;  // row; its position is ta
-  if (t >= a.T) return;  // whole wave; no barrier follows
+  const int t = HEADS ? blockIdx.x : blockIdx.x * NW + wave;  // row; its position is ta
+  if (t >= a.T) return;  // whole wave; no barrier follows (HEADS: never)
   const int ta = t + a.q0;
   const int nsel4 = (nsel + 3) & ~3;
   float* wb = lds + NQ * 256 + wave * (NQ * 256 + nsel4);  // generic remap only
   float* wag = wb + NQ * 256;
+  float* hs = lds + NQ * 256 + (FAST9 ? 0 : NW * (NQ * 256 + nsel4));  // HEADS only
+  const int h0 = HEADS ? wave : 0, hstep = HEADS ? NW : 1;
 
   int vis_hi = 0;  // 1 + the largest block index visible at t (0: none)
   int nfull = NQ;  // leading pieces whose 256 blocks are all visible (no mask needed)
@@ -320,10 +388,10 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
     for (int s = 0; s < NQ; ++s)
       if (s < nact) v[s] = *reinterpret_cast<const float4*>(row + min(256 * s + 4 * lane, ncs - 4));
   };
-  load_row(cur, 0);
-  for (int hh = 0; hh < hpg; ++hh) {
+  if (h0 < hpg) load_row(cur, h0);
+  for (int hh = h0; hh < hpg; hh += hstep) {
     if constexpr (kPrefetch)
-      if (hh + 1 < hpg) load_row(nxt, hh + 1);
+      if (hh + hstep < hpg) load_row(nxt, hh + hstep);
     const int h = g * hpg + hh;
     float v[NQ][4];
     float mx = -INFINITY;
@@ -393,8 +461,12 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
         const float nb63 = s + 1 < NQ ? __shfl(v[s + 1 < NQ ? s + 1 : s][0], 0) : 0.0f;
         if (lane == 63) nb = nb63;
         const float s9 = (((((((0.0f + v[s][0]) + v[s][1]) + v[s][1]) + v[s][2]) + v[s][2]) + v[s][3]) + v[s][3]) + nb;
-        agg[s] += s9;
         const int j = 64 * s + lane;
+        if constexpr (HEADS) {
+          if (j < nsel) hs[hh * nsel4 + j] = s9;
+        } else {
+          agg[s] += s9;
+        }
         if (psl && j < nsel) psl[j] = s9;
       }
     } else {
@@ -409,7 +481,8 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
             const int ci = a.s * j + m + nn;
             if (ci < NB) s9 += wb[ci];
           }
-        wag[j] += s9;
+        if constexpr (HEADS) hs[hh * nsel4 + j] = s9;
+        else wag[j] += s9;
         if (psl) psl[j] = s9;
       }
       wave_lds_sync();  // the copy is rewritten for the next row
@@ -417,8 +490,27 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
     if constexpr (kPrefetch) {
 #pragma unroll
       for (int s = 0; s < NQ; ++s) cur[s] = nxt[s];
-    } else if (hh + 1 < hpg) {
-      load_row(cur, hh + 1);
+    } else if (hh + hstep < hpg) {
+      load_row(cur, hh + hstep);
+    }
+  }
+  if constexpr (HEADS) {
+    __syncthreads();
+    if (wave > 0) return;
+    if constexpr (FAST9) {
+#pragma unroll
+      for (int s = 0; s < NQ; ++s) {
+        const int j = 64 * s + lane;
+        if (s < nact && j < nsel)
+          for (int hh = 0; hh < hpg; ++hh) agg[s] += hs[hh * nsel4 + j];
+      }
+    } else {
+      for (int j = lane; j < nsel; j += 64) {
+        float x = 0.0f;
+        for (int hh = 0; hh < hpg; ++hh) x += hs[hh * nsel4 + j];
+        wag[j] = x;
+      }
+      wave_lds_sync();
     }
   }
 
@@ -517,38 +609,52 @@ static size_t score_rows_lds(int nq, bool fast9, int nw, int nsel) {
   return 4 * ((size_t)nq * 256 + nw * per_wave);
 }
 
-template <int NQ, bool FAST9>
+template <int NQ, bool FAST9, bool HEADS>
 static hipError_t launch_rows_k(const ScoreArgs& a, int nw, size_t lds, hipStream_t st) {
-  auto fn = score_rows_kernel<NQ, FAST9>;
+  auto fn = score_rows_kernel<NQ, FAST9, HEADS>;
   if (lds > 64 * 1024) {  // beyond the default dynamic LDS limit
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)lds);
     if (e != hipSuccess) return e;
   }
-  dim3 grid((a.T + nw - 1) / nw, a.B * a.G);
+  dim3 grid(HEADS ? a.T : (a.T + nw - 1) / nw, a.B * a.G);
   hipLaunchKernelGGL(fn, grid, dim3(64 * nw), lds, st, a);
   return hipGetLastError();
 }
 
-template <bool FAST9>
+template <bool FAST9, bool HEADS>
 static hipError_t launch_rows_q(const ScoreArgs& a, int nq, int nw, size_t lds, hipStream_t st) {
   switch (nq) {
-    case 1: return launch_rows_k<1, FAST9>(a, nw, lds, st);
-    case 2: return launch_rows_k<2, FAST9>(a, nw, lds, st);
-    case 4: return launch_rows_k<4, FAST9>(a, nw, lds, st);
-    case 8: return launch_rows_k<8, FAST9>(a, nw, lds, st);
-    case 16: return launch_rows_k<16, FAST9>(a, nw, lds, st);
+    case 1: return launch_rows_k<1, FAST9, HEADS>(a, nw, lds, st);
+    case 2: return launch_rows_k<2, FAST9, HEADS>(a, nw, lds, st);
+    case 4: return launch_rows_k<4, FAST9, HEADS>(a, nw, lds, st);
+    case 8: return launch_rows_k<8, FAST9, HEADS>(a, nw, lds, st);
+    case 16: return launch_rows_k<16, FAST9, HEADS>(a, nw, lds, st);
   }
   return hipErrorInvalidValue;
 }
 
-// Launches the logits GEMM and the rows kernel (one wave per timestep).
+// Timesteps of a call (batches x groups x rows) up to which the rows kernel spreads one
+// timestep's heads over a workgroup's waves: a wave per timestep is at most one wave per SIMD
+// there, each walking its heads one after another.  Measured with the few-row logits where
+// they apply (call, before -> after): one timestep of B16 H32 G2, 2048 blocks 89 -> 43 us;
+// H64 G4 512 blocks 40 -> 21 us; T = 128 (512 timesteps) 35 -> 28 us; T = 256 (1024) 36 ->
+// 32 us.  With 2048 timesteps a wave each gives two waves per SIMD, and the LDS pass and
+// the idle waves of the top-n would cost what the spread saves.
+constexpr int kRowsHeadsMax = 1024;
+
+// Launches the logits GEMM and the rows kernel (one wave per timestep, or one workgroup).
 // Returns 0 on success, 1 when no configuration fits, 2 on a HIP launch error.
 int launch_score_topn(int dtype, ScoreArgs a, hipStream_t st) {
   if (a.NB > kMaxCols || a.hpg > kMaxRows) return 1;
   a.ncs = score_ncs(a.NB);
-  {
-    const int Rall = a.T * a.hpg;
+  const int Rall = a.T * a.hpg;
+  if (Rall <= kLgFewRows && a.NB > 0) {
+    const dim3 grid(a.ncs / 64, (Rall + 15) / 16, a.B * a.G);
+    if (dtype == kF32) hipLaunchKernelGGL(score_logits_few_kernel<float>, grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(score_logits_few_kernel<uint16_t>, grid, dim3(256), 0, st, a);
+    if (hipGetLastError() != hipSuccess) return 2;
+  } else {
     const dim3 grid((Rall + kLgTM - 1) / kLgTM, a.ncs / kLgTN, a.B * a.G);
     hipLaunchKernelGGL(score_tile_ncomp_kernel, dim3(grid.x), dim3(256), 0, st, a);
     if (dtype == kF32) hipLaunchKernelGGL(score_logits_kernel<float>, grid, dim3(256), 0, st, a);
@@ -557,6 +663,13 @@ int launch_score_topn(int dtype, ScoreArgs a, hipStream_t st) {
   }
   const int nq = score_rows_nq(a.ncs);
   const bool fast9 = a.a == 2 && a.s == 4;
+  hipError_t e;
+  const int nwh = min(kRowsWaves, a.hpg);
+  const size_t lds_h = score_rows_lds(nq, fast9, nwh, a.nsel) + (size_t)4 * a.hpg * ((a.nsel + 3) & ~3);
+  if (a.hpg > 1 && (int64_t)a.B * a.G * a.T <= kRowsHeadsMax && lds_h <= 156 * 1024) {
+    e = fast9 ? launch_rows_q<true, true>(a, nq, nwh, lds_h, st) : launch_rows_q<false, true>(a, nq, nwh, lds_h, st);
+    return e == hipSuccess ? 0 : 2;
+  }
   // fewer waves per workgroup when the generic remap's LDS rows do not fit, and 4 when the
   // row registers allow at most 3 waves per SIMD (a workgroup of 4 puts one on each SIMD,
   // so three workgroups share a CU where one of 8 waves would leave a third slot empty)
@@ -564,7 +677,7 @@ int launch_score_topn(int dtype, ScoreArgs a, hipStream_t st) {
   while (nw > 1 && score_rows_lds(nq, fast9, nw, a.nsel) > 80 * 1024) nw /= 2;
   const size_t lds = score_rows_lds(nq, fast9, nw, a.nsel);
   if (lds > 156 * 1024) return 1;
-  const hipError_t e = fast9 ? launch_rows_q<true>(a, nq, nw, lds, st) : launch_rows_q<false>(a, nq, nw, lds, st);
+  e = fast9 ? launch_rows_q<true, false>(a, nq, nw, lds, st) : launch_rows_q<false, false>(a, nq, nw, lds, st);
   return e == hipSuccess ? 0 : 2;
 }
 

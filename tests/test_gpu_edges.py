@@ -3,10 +3,13 @@ CPU oracle.  Tolerances as in test_gpu_branches.py (fp32 outputs 1e-5, gradients
 2e-2, the oracle fed the bf16-rounded inputs)."""
 import math
 
+import numpy as np
+import oracle
 import pytest
 import torch
 
-from nsa import _ops
+from nsa import NSAConfig, _ops
+from nsa.kernels import score_and_select
 from test_gpu_branches import _check, _make
 
 pytestmark = pytest.mark.gpu
@@ -31,3 +34,27 @@ def test_selection_bitmap_edges(dev, hpg, T, lp, n, dtype, dk, dv):
     q, kp, v, do = _make(hpg, B, G * hpg, G, T, T, dk, dv, dtype, dev)
     idx = _lists(hpg + T, B, G, T, n, (T + lp - 1) // lp).to(dev)
     _check(_ops.SELECTION, q, kp, v, do, 1 / math.sqrt(dk), dtype, indices=idx, lprime=lp)
+
+
+# scoring with few rows (one MFMA tile per wave) and few timesteps (heads across waves): rows
+# about 16 / 64 (the tile and the rule's edge), 1 / 3 / 20 heads a group, block counts at the
+# 256-block pieces and 64-block tiles, both remaps (l/d = 2, l'/d = 4 and another), dk with a
+# remainder piece; indices and scores bit for bit
+@pytest.mark.parametrize("B,G,hpg,T,N,dk,l,lp", [(1, 2, 16, 1, 255, 64, 32, 64), (2, 2, 3, 5, 257, 40, 32, 64),
+                                                 (1, 1, 16, 4, 64, 192, 32, 64), (1, 1, 13, 5, 65, 96, 32, 64),
+                                                 (1, 2, 20, 3, 1030, 64, 32, 64), (3, 1, 4, 17, 600, 128, 64, 32),
+                                                 (1, 2, 1, 64, 70, 64, 32, 64), (1, 1, 2, 1024, 100, 32, 32, 64),
+                                                 (1, 1, 2, 1025, 100, 32, 32, 64), (1, 1, 64, 1, 4096, 32, 32, 64)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_score_few_rows(dev, B, G, hpg, T, N, dk, l, lp, dtype):
+    g = torch.Generator().manual_seed(N + T)
+    q = torch.randn(B, G * hpg, T, dk, generator=g).to(dtype)
+    k = torch.randn(B, G, dk, N, generator=g).to(dtype)
+    be = torch.arange(N, dtype=torch.int32) * 16 + l - 1
+    q0 = max(0, 16 * N - 3 * T)  # the last rows see every block, the first ones do not
+    cfg = NSAConfig(head_dim_qk=dk, n_heads=G * hpg, n_kv_groups=G, l=l, l_prime=lp, n=9)
+    got = score_and_select(q.to(dev), k.to(dev), be.to(dev), 0.2, cfg, return_scores=True, q_offset=q0)
+    want = oracle.score_topn(q.float().numpy(), k.float().numpy(), be.numpy(), np.float32(0.2), l=l, d=16, lprime=lp,
+                             n=9, positions=np.arange(q0, q0 + T, dtype=np.int32), want_scores=True)
+    for a, b in zip(got, want):
+        np.testing.assert_array_equal(a.cpu().numpy(), b)
