@@ -323,7 +323,7 @@ struct IntDiv {
 // Value of lane L ^ OFF of a wave64 (OFF a power of two below 64) without the LDS
 // crossbar: v_permlane32_swap / v_permlane16_swap for 32 and 16 (each swap returns the
 // other half's values in the result the lane's own half does not keep), DPP row_ror:8
-// for 8, row_ror:4 or :12 by lane for 4, quad_perm for 2 and 1.  Equal to
+// for 8, row_shl:4 / row_shr:4 by bank for 4, quad_perm for 2 and 1.  Equal to
 // __shfl_xor(x, OFF) on every lane.
 template <int OFF>
 __device__ __forceinline__ uint32_t lane_xor_u32(uint32_t x) {
@@ -338,9 +338,9 @@ __device__ __forceinline__ uint32_t lane_xor_u32(uint32_t x) {
   } else if constexpr (OFF == 8) {
     return __builtin_amdgcn_update_dpp(0u, x, 0x128, 0xF, 0xF, false);  // row_ror:8
   } else if constexpr (OFF == 4) {
-    const uint32_t lo = __builtin_amdgcn_update_dpp(0u, x, 0x124, 0xF, 0xF, false);  // row_ror:4
-    const uint32_t hi = __builtin_amdgcn_update_dpp(0u, x, 0x12C, 0xF, 0xF, false);  // row_ror:12
-    return (lane & 4) ? lo : hi;
+    // banks 0, 2 of each row take lane + 4 (row_shl:4), banks 1, 3 lane - 4 (row_shr:4)
+    const uint32_t up = __builtin_amdgcn_update_dpp(0u, x, 0x104, 0xF, 0x5, false);
+    return __builtin_amdgcn_update_dpp(up, x, 0x114, 0xF, 0xA, false);
   } else if constexpr (OFF == 2) {
     return __builtin_amdgcn_update_dpp(0u, x, 0x4E, 0xF, 0xF, false);  // quad_perm [2,3,0,1]
   } else {
@@ -355,30 +355,53 @@ template <int OFF>
 __device__ __forceinline__ int lane_xor(int x) {
   return (int)lane_xor_u32<OFF>((uint32_t)x);
 }
+// op(x, x of lane L ^ OFF) for a commutative op.  Offsets 32 and 16: the swap of x with
+// itself leaves the low and the high half's values side by side in every lane, so op takes
+// them as they are, without the select that a lane's own "other" value would need.
+template <int OFF, typename T, typename F>
+__device__ __forceinline__ T lane_fold(T x, F op) {
+  if constexpr (OFF == 32 || OFF == 16) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, x);
+    uint32_t lo, hi;
+    if constexpr (OFF == 32) {
+      const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+      lo = r[0], hi = r[1];
+    } else {
+      const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+      lo = r[0], hi = r[1];
+    }
+    return op(__builtin_bit_cast(T, lo), __builtin_bit_cast(T, hi));
+  } else {
+    return op(x, lane_xor<OFF>(x));
+  }
+}
 // max / sum over the four lanes sharing (l & 15), lane swaps instead of LDS-crossbar
 // shuffles (same pairing order as __shfl_xor with 16, then 32)
 __device__ __forceinline__ float wave_max16(float v) {
-  v = fmaxf(v, lane_xor<16>(v));
-  v = fmaxf(v, lane_xor<32>(v));
-  return v;
+  auto mx = [](float x, float y) { return fmaxf(x, y); };
+  return lane_fold<32>(lane_fold<16>(v, mx), mx);
 }
 __device__ __forceinline__ float wave_sum16(float v) {
-  v += lane_xor<16>(v);
-  v += lane_xor<32>(v);
-  return v;
+  auto add = [](float x, float y) { return x + y; };
+  return lane_fold<32>(lane_fold<16>(v, add), add);
 }
 
-// xor butterfly over 32, 16, 8, 4, 2, 1: every lane ends with op folded over the wave,
-// pairs combined in exactly the order of the __shfl_xor loop over the same offsets
+// xor butterfly over 32, 16, 8, 4, 2, 1: every lane ends with the commutative op folded
+// over the wave, pairs combined in exactly the order of the __shfl_xor loop over the same
+// offsets
 template <typename T, typename F>
 __device__ __forceinline__ T wave_butterfly(T x, F op) {
-  x = op(x, lane_xor<32>(x));
-  x = op(x, lane_xor<16>(x));
-  x = op(x, lane_xor<8>(x));
-  x = op(x, lane_xor<4>(x));
-  x = op(x, lane_xor<2>(x));
-  x = op(x, lane_xor<1>(x));
+  x = lane_fold<32>(x, op);
+  x = lane_fold<16>(x, op);
+  x = lane_fold<8>(x, op);
+  x = lane_fold<4>(x, op);
+  x = lane_fold<2>(x, op);
+  x = lane_fold<1>(x, op);
   return x;
+}
+// Value of lane L + 1 of the wave, `last` in lane 63 (DPP wave_shl:1)
+__device__ __forceinline__ float lane_next(float x, float last) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(__float_as_uint(last), __float_as_uint(x), 0x130, 0xF, 0xF, false));
 }
 
 }  // namespace nsa

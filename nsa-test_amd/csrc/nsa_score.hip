@@ -320,13 +320,17 @@ __global__ __launch_bounds__(256) void score_logits_few_kernel(ScoreArgs a) {
 //      wave-private LDS row otherwise.
 // Then the top-n of the timestep from those sums.  Blocks past the last one visible
 // at t are not read (the logits kernel computed every visible block, and block 0).
-constexpr int kRowsWaves = 8;
-
+// Bound by vector-ALU issue (about 25 operations a block, the reductions and the top-n
+// rounds): folds without selects, the neighbour's value by a wave shift instead of the LDS
+// crossbar, top-n rounds that fold the sums alone and no scalar spills took it from 1.36 to
+// 1.25 ms (H32 G2 T32768, 2048 blocks).
 //
 // HEADS: a workgroup takes one timestep and its waves the heads (head hh on wave hh % NW),
 // for calls with too few timesteps to occupy the chip with a wave each.  Every row's Eq. 9
 // scores go to LDS; wave 0 then adds them in head order and takes the top-n, so the sums
 // and the indices are those of the serial walk.
+constexpr int kRowsWaves = 8;
+
 template <int NQ, bool FAST9, bool HEADS>
 __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu(NQ == 8 && !HEADS ? 4 : 1))) void score_rows_kernel(ScoreArgs a) {
   // LDS: sbe [NQ * 256] block ends (INT_MAX past NB); generic remap only, per wave:
@@ -438,30 +442,38 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
         for (int u = 0; u < 4; ++u) v[s][u] *= rs;  // invisible blocks: p = 0 exactly
     if (a.p_cmp) {
       float* pc = a.p_cmp + (((int64_t)b * a.H + h) * a.T + t) * NB;
+      // an opaque copy of the lane's first column: the 4 NQ store conditions depend only on
+      // it and NB, and would otherwise be kept in scalar registers through the whole head
+      // loop (115 of them spilled at NQ = 8)
+      int c0 = 4 * lane;
+      asm volatile("" : "+v"(c0));
 #pragma unroll
       for (int s = 0; s < NQ; ++s)
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const int i = 256 * s + 4 * lane + u;
+          const int i = 256 * s + c0 + u;
           if (i < NB) pc[i] = v[s][u];
         }
     }
     // Eq. 9 in the reference's (m, n) order, starting from 0; invisible blocks (and
     // blocks past NB) add an exact +0
     float* psl = a.p_slc ? a.p_slc + (((int64_t)b * a.H + h) * a.T + t) * nsel : nullptr;
+    int jl = lane;  // opaque as above: output j = 64 s + jl of this head
+    asm volatile("" : "+v"(jl));
     if constexpr (FAST9) {  // (m, n) -> 4j + {0, 1, 1, 2, 2, 3, 3, 4}
 #pragma unroll
       for (int s = 0; s < NQ; ++s) {
         if (s >= nact) {  // Eq. 9 scores of exact 0
-          const int j = 64 * s + lane;
+          const int j = 64 * s + jl;
           if (psl && j < nsel) psl[j] = 0.0f;
           continue;
         }
-        float nb = __shfl_down(v[s][0], 1);
-        const float nb63 = s + 1 < NQ ? __shfl(v[s + 1 < NQ ? s + 1 : s][0], 0) : 0.0f;
-        if (lane == 63) nb = nb63;
+        const float nb63 = s + 1 < NQ ? __uint_as_float(__builtin_amdgcn_readfirstlane(
+                                            __float_as_uint(v[s + 1 < NQ ? s + 1 : s][0])))
+                                      : 0.0f;
+        const float nb = lane_next(v[s][0], nb63);
         const float s9 = (((((((0.0f + v[s][0]) + v[s][1]) + v[s][1]) + v[s][2]) + v[s][2]) + v[s][3]) + v[s][3]) + nb;
-        const int j = 64 * s + lane;
+        const int j = 64 * s + jl;
         if constexpr (HEADS) {
           if (j < nsel) hs[hh * nsel4 + j] = s9;
         } else {
@@ -523,18 +535,21 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
       if (64 * s + lane >= nsel) agg[s] = -INFINITY;  // past nsel: never taken (kk <= nsel)
   }
   int top0 = -1, top1 = -1;  // lane c holds candidate c (top0) and c + 64 (top1)
-  for (int rk = 0; rk < kk; ++rk) {
-    float bv = -INFINITY;
-    int bi = 0x7fffffff;
+  // every lane keeps its best remaining output (largest sum, lowest index); a round folds
+  // the sums alone and finds the winner's index by a ballot (a fold over the indices only
+  // where lanes tie), and the winning lane looks for its next best
+  float bv = -INFINITY;
+  int bi = 0x7fffffff;
+  auto best = [&]() __attribute__((always_inline)) {
+    bv = -INFINITY;
+    bi = 0x7fffffff;
     if constexpr (FAST9) {
 #pragma unroll
-      for (int s = 0; s < NQ; ++s) {
-        const int j = 64 * s + lane;
-        if (agg[s] > bv || (agg[s] == bv && j < bi)) {
+      for (int s = 0; s < NQ; ++s)  // ascending outputs: an equal sum keeps the lower one
+        if (agg[s] > bv || (s == 0 && agg[s] == bv)) {
           bv = agg[s];
-          bi = j;
+          bi = 64 * s + lane;
         }
-      }
     } else {
       for (int j = lane; j < nsel; j += 64) {
         const float x = wag[j];
@@ -544,31 +559,31 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
         }
       }
     }
-    auto take = [&](float ov, int oi) __attribute__((always_inline)) {
-      if (ov > bv || (ov == bv && oi < bi)) {
-        bv = ov;
-        bi = oi;
-      }
-    };
-    take(lane_xor<32>(bv), lane_xor<32>(bi));
-    take(lane_xor<16>(bv), lane_xor<16>(bi));
-    take(lane_xor<8>(bv), lane_xor<8>(bi));
-    take(lane_xor<4>(bv), lane_xor<4>(bi));
-    take(lane_xor<2>(bv), lane_xor<2>(bi));
-    take(lane_xor<1>(bv), lane_xor<1>(bi));
-    // bi is wave-uniform: its owner marks it taken
-    if constexpr (FAST9) {
+  };
+  best();
+  for (int rk = 0; rk < kk; ++rk) {
+    const float mx = wave_butterfly(bv, [](float x, float y) { return fmaxf(x, y); });
+    const uint64_t tied = __ballot(bv == mx);
+    int win;  // wave-uniform
+    if (__builtin_popcountll(tied) == 1)
+      win = __builtin_amdgcn_readlane(bi, __builtin_ctzll(tied));
+    else
+      win = __builtin_amdgcn_readfirstlane(
+          wave_butterfly(bv == mx ? bi : 0x7fffffff, [](int x, int y) { return min(x, y); }));
+    if (lane == (win & 63)) {  // its owner marks it taken
+      if constexpr (FAST9) {
 #pragma unroll
-      for (int s = 0; s < NQ; ++s)
-        if (64 * s + lane == bi) agg[s] = -INFINITY;
-    } else {
-      if (lane == (bi & 63)) wag[bi] = -INFINITY;
-      wave_lds_sync();
+        for (int s = 0; s < NQ; ++s)
+          if (64 * s + lane == win) agg[s] = -INFINITY;
+      } else {
+        if (win < nsel) wag[win] = -INFINITY;
+      }
+      best();
     }
     const int c = nc + rk;
     if (lane == (c & 63)) {
-      if (c < 64) top0 = bi;
-      else top1 = bi;
+      if (c < 64) top0 = win;
+      else top1 = win;
     }
   }
   // candidates: fixed [0, max(0,(t-l')/l'), t/l'] then the top-k.  The top-k are
@@ -635,13 +650,14 @@ static hipError_t launch_rows_q(const ScoreArgs& a, int nq, int nw, size_t lds, 
 }
 
 // Timesteps of a call (batches x groups x rows) up to which the rows kernel spreads one
-// timestep's heads over a workgroup's waves: a wave per timestep is at most one wave per SIMD
-// there, each walking its heads one after another.  Measured with the few-row logits where
-// they apply (call, before -> after): one timestep of B16 H32 G2, 2048 blocks 89 -> 43 us;
-// H64 G4 512 blocks 40 -> 21 us; T = 128 (512 timesteps) 35 -> 28 us; T = 256 (1024) 36 ->
-// 32 us.  With 2048 timesteps a wave each gives two waves per SIMD, and the LDS pass and
-// the idle waves of the top-n would cost what the spread saves.
-constexpr int kRowsHeadsMax = 1024;
+// timestep's heads over a workgroup's waves: as many 8-wave workgroups as the chip holds at
+// once (the pieces a lane holds set the registers).  A wave per timestep is at most one
+// wave per SIMD there, each walking its heads one after another.  Measured with the few-row
+// logits where they apply (call, before -> after): one timestep of B16 H32 G2, 2048 blocks
+// 89 -> 43 us; H64 G4 512 blocks 40 -> 21 us; T = 128 (512 timesteps) 35 -> 28 us; T = 256
+// (1024) 36 -> 32 us.  Past it the idle waves of the top-n cost more than the spread saves
+// (1024 timesteps of 3000 blocks: 76 -> 119 us).
+static int64_t rows_heads_max(int nq) { return nq <= 4 ? 1024 : nq == 8 ? 512 : 256; }
 
 // Launches the logits GEMM and the rows kernel (one wave per timestep, or one workgroup).
 // Returns 0 on success, 1 when no configuration fits, 2 on a HIP launch error.
@@ -666,7 +682,7 @@ int launch_score_topn(int dtype, ScoreArgs a, hipStream_t st) {
   hipError_t e;
   const int nwh = min(kRowsWaves, a.hpg);
   const size_t lds_h = score_rows_lds(nq, fast9, nwh, a.nsel) + (size_t)4 * a.hpg * ((a.nsel + 3) & ~3);
-  if (a.hpg > 1 && (int64_t)a.B * a.G * a.T <= kRowsHeadsMax && lds_h <= 156 * 1024) {
+  if (a.hpg > 1 && (int64_t)a.B * a.G * a.T <= rows_heads_max(nq) && lds_h <= 156 * 1024) {
     e = fast9 ? launch_rows_q<true, true>(a, nq, nwh, lds_h, st) : launch_rows_q<false, true>(a, nq, nwh, lds_h, st);
     return e == hipSuccess ? 0 : 2;
   }
