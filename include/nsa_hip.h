@@ -449,6 +449,37 @@ size_t nsa_wgrad_workspace_size(int rows, int n1, int n2);
 int nsa_wgrad(const void* dY, int64_t ld_dy, const void* X, int64_t ld_x, int rows, int n1, int n2, void* dW,
               int64_t ld_dw, int dtype, void* workspace, size_t workspace_bytes, nsa_stream_t stream);
 
+/* ---- one decode step (no reference counterpart) --------------------------------------
+ * The attention of one timestep per batch entry at absolute position t (the caches hold
+ * positions 0 .. t): out[z,h] = sum over the branches (0 compression, 1 selection, 2 sliding
+ * window) of act(gates[z,h,branch]) times the branch's attention output, the branch outputs
+ * and the mix in fp32, rounded to dtype once.  The keys and values are read where they lie
+ * (unit feature stride, 16-byte aligned rows, strides (z, g, token) in elements):
+ *   branch 0  the n_cmp compressed tokens completed so far (all visible)
+ *   branch 1  the distinct blocks indices[z,g,0..n_slots-1] (contiguous int64, negative =
+ *             none; later blocks are masked) of block_size_selection keys, a multiple of 16;
+ *             a row without any block takes block t / block_size_selection
+ *   branch 2  the last window_size positions
+ * q [Z,H,dk] and out [Z,H,dv] have unit feature stride and 16-byte aligned rows; gates [Z,H,3]
+ * in dtype; gate_act as in nsa_gate_mix_fwd.  workspace: nsa_decode_workspace_size bytes. */
+typedef struct nsa_decode_args {
+  const void* q;
+  const void* k[3];
+  const void* v[3];
+  const int64_t* indices;
+  const void* gates;
+  void* out;
+  int64_t stride_qz, stride_qh, stride_oz, stride_oh;
+  int64_t stride_kz[3], stride_kg[3], stride_kt[3];
+  int64_t stride_vz[3], stride_vg[3], stride_vt[3];
+  int64_t stride_gz, stride_gh, stride_gk;
+  int Z, H, n_kv_groups, t, n_cmp, n_slots, block_size_selection, window_size;
+  int head_dim_qk, head_dim_v, gate_act, dtype;
+  float sm_scale;
+} nsa_decode_args;
+size_t nsa_decode_workspace_size(const nsa_decode_args* args);
+int nsa_decode_attn(const nsa_decode_args* args, void* workspace, size_t workspace_bytes, nsa_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -483,13 +483,43 @@ int scratch_ptr(void** out) {
   return NSA_OK;
 }
 
+// the sizes of a decode step (pointers and strides left out)
+DecodeArgs decode_shape(const nsa_decode_args& x) {
+  DecodeArgs a{};
+  a.B = x.Z;
+  a.G = x.n_kv_groups;
+  a.hpg = x.H / x.n_kv_groups;
+  a.t = x.t;
+  a.n_cmp = x.n_cmp;
+  a.nslots = x.n_slots;
+  a.lprime = x.block_size_selection;
+  a.window = x.window_size;
+  decode_split(a);
+  return a;
+}
+
+int validate_decode(const nsa_decode_args& x) {
+  if (x.dtype != NSA_F32 && x.dtype != NSA_BF16) return fail(NSA_ERR_INVALID, "dtype %d not supported", x.dtype);
+  if (x.Z <= 0 || x.H <= 0 || x.n_kv_groups <= 0 || x.H % x.n_kv_groups)
+    return fail(NSA_ERR_INVALID, "bad shape Z=%d H=%d G=%d", x.Z, x.H, x.n_kv_groups);
+  if (x.t < 0 || x.t == INT32_MAX || x.n_cmp < 0 || x.window_size <= 0)
+    return fail(NSA_ERR_INVALID, "bad t=%d, n_cmp=%d or window_size=%d", x.t, x.n_cmp, x.window_size);
+  if (x.n_slots < 1 || x.n_slots > 64) return fail(NSA_ERR_INVALID, "n_slots=%d outside [1, 64]", x.n_slots);
+  if (x.block_size_selection <= 0 || x.block_size_selection % 16 || x.block_size_selection > (1 << 20))
+    return fail(NSA_ERR_INVALID, "block_size_selection=%d must be a positive multiple of 16", x.block_size_selection);
+  if (x.gate_act < 0 || x.gate_act > 2) return fail(NSA_ERR_INVALID, "gate_act=%d outside [0, 2]", x.gate_act);
+  if (!dims_supported(x.head_dim_qk, x.head_dim_v))
+    return fail(NSA_ERR_UNSUPPORTED, "no kernel for head dims dk=%d dv=%d", x.head_dim_qk, x.head_dim_v);
+  return NSA_OK;
+}
+
 }  // namespace
 
 int nsa::set_error(int code, const char* msg) { return fail(code, "%s", msg); }
 
 extern "C" {
 
-int nsa_abi_version(void) { return 5; }
+int nsa_abi_version(void) { return 6; }
 const char* nsa_last_error(void) { return g_err; }
 int nsa_head_dims_supported(int dtype, int dk, int dv) {
   return (dtype == NSA_F32 || dtype == NSA_BF16) && dims_supported(dk, dv);
@@ -513,6 +543,64 @@ int nsa_bwd_dq_deferrable(int branch, int dtype, int Z, int H, int G, int Tq, in
   Shape s{branch, dtype, Z, H, G, Tq, Tkv, dk, dv, nslots, lprime > 0 ? lprime : 64, window_size > 0 ? window_size : 1};
   if (G <= 0 || H % G || Z < 0 || Tq < 0) return 0;
   return s.stored_ds() ? 1 : 0;
+}
+
+size_t nsa_decode_workspace_size(const nsa_decode_args* x) {
+  if (!x || validate_decode(*x)) return 0;
+  return decode_part_bytes(decode_shape(*x), x->head_dim_v);
+}
+
+int nsa_decode_attn(const nsa_decode_args* x, void* ws, size_t ws_bytes, nsa_stream_t stream) {
+  if (!x) return fail(NSA_ERR_INVALID, "args is null");
+  int rc = validate_decode(*x);
+  if (rc) return rc;
+  const int esz = x->dtype == NSA_F32 ? 4 : 2;
+  if (!x->q || !x->out || !x->gates || !x->indices || !x->k[1] || !x->v[1] || !x->k[2] || !x->v[2] ||
+      (x->n_cmp > 0 && (!x->k[0] || !x->v[0])))
+    return fail(NSA_ERR_INVALID, "null tensor");
+  auto rows = [&](const void* p, int64_t sz, int64_t s1, int n1, int64_t s2, int n2) {
+    return ((uintptr_t)p) % 16 == 0 && (x->Z == 1 || (sz * esz) % 16 == 0) && (n1 == 1 || (s1 * esz) % 16 == 0) &&
+           (n2 == 1 || (s2 * esz) % 16 == 0);
+  };
+  if (!rows(x->q, x->stride_qz, x->stride_qh, x->H, 0, 1) || !rows(x->out, x->stride_oz, x->stride_oh, x->H, 0, 1))
+    return fail(NSA_ERR_LAYOUT, "q and out need 16-byte aligned rows");
+  for (int br = x->n_cmp > 0 ? 0 : 1; br < 3; ++br) {
+    const int nt = br == 0 ? x->n_cmp : x->t + 1;
+    if (!rows(x->k[br], x->stride_kz[br], x->stride_kg[br], x->n_kv_groups, x->stride_kt[br], nt) ||
+        !rows(x->v[br], x->stride_vz[br], x->stride_vg[br], x->n_kv_groups, x->stride_vt[br], nt))
+      return fail(NSA_ERR_LAYOUT, "cached keys and values need 16-byte aligned rows");
+  }
+  DecodeArgs a = decode_shape(*x);
+  const size_t need = decode_part_bytes(a, x->head_dim_v);
+  if (ws_bytes < need || !ws || ((uintptr_t)ws) % 16)
+    return fail(NSA_ERR_WORKSPACE, "workspace of %zu bytes (16-byte aligned) required, %zu given", need, ws_bytes);
+  a.q = x->q;
+  a.sq_b = x->stride_qz;
+  a.sq_h = x->stride_qh;
+  for (int br = 0; br < 3; ++br) {
+    a.k[br] = x->k[br];
+    a.v[br] = x->v[br];
+    a.sk_b[br] = x->stride_kz[br];
+    a.sk_g[br] = x->stride_kg[br];
+    a.sk_t[br] = x->stride_kt[br];
+    a.sv_b[br] = x->stride_vz[br];
+    a.sv_g[br] = x->stride_vg[br];
+    a.sv_t[br] = x->stride_vt[br];
+  }
+  a.idx = x->indices;
+  a.gates = x->gates;
+  a.sg_b = x->stride_gz;
+  a.sg_h = x->stride_gh;
+  a.sg_k = x->stride_gk;
+  a.out = x->out;
+  a.so_b = x->stride_oz;
+  a.so_h = x->stride_oh;
+  a.act = x->gate_act;
+  a.scale = x->sm_scale;
+  a.part = static_cast<float*>(ws);
+  if (!dispatch_decode(x->dtype, x->head_dim_qk, x->head_dim_v, a, (hipStream_t)stream))
+    return fail(NSA_ERR_UNSUPPORTED, "no decode kernel");
+  return check_hip("decode attention");
 }
 
 int nsa_bwd_dkdv_plan(int branch, int Z, int H, int G, int Tq, int Tkv, int nslots, int lprime, int window_size,

@@ -37,6 +37,29 @@ void launch_sel_csr(const int* clean, int* chunk_cnt, int B, int G, int Tq, int 
                     int* csr_t, int* csr_s, int* seg_off, int seg, hipStream_t st);
 int sel_csr_chunks(int Tq);
 
+// one decode step's attention (nsa_decode.hip); branch order of the gates
+enum DecodeBranch : int { kDecCmp = 0, kDecSel = 1, kDecWin = 2 };
+struct DecodeArgs {
+  const void* q;  // [B,H,DK]
+  int64_t sq_b, sq_h;
+  const void* k[3];  // per branch, strides (b, g, token)
+  const void* v[3];
+  int64_t sk_b[3], sk_g[3], sk_t[3], sv_b[3], sv_g[3], sv_t[3];
+  const int64_t* idx;  // [B*G][nslots]
+  const void* gates;   // [B,H,3]
+  int64_t sg_b, sg_h, sg_k;
+  void* out;  // [B,H,DV]
+  int64_t so_b, so_h;
+  float* part;  // workspace: [B*G][head tiles][nparts] partials
+  int nwg[3];   // workgroups (partials) of each branch
+  int nparts;
+  int B, G, hpg, t, n_cmp, nslots, lprime, window, act;
+  float scale;
+};
+void decode_split(DecodeArgs& a);  // nwg / nparts from the key counts
+size_t decode_part_bytes(const DecodeArgs& a, int dv);
+bool dispatch_decode(int dtype, int dk, int dv, const DecodeArgs& a, hipStream_t st);
+
 // record an error message for nsa_last_error(); returns `code`
 int set_error(int code, const char* msg);
 

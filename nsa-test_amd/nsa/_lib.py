@@ -12,7 +12,7 @@ from ctypes import c_float, c_int, c_int64, c_size_t, c_void_p
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().with_name("libnsa_hip.so")
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 NSA_F32 = 0
 NSA_BF16 = 1
@@ -80,7 +80,23 @@ SIGNATURES.update({
     "nsa_wgrad_workspace_size": (_Z, [_I] * 3),
     "nsa_wgrad": (_I, [_P, _L, _P, _L, _I, _I, _I, _P, _L, _I, _P, _Z, _P]),
     "nsa_bwd_dkdv_plan": (_I, [_I] * 9 + [_P, _P]),
+    "nsa_decode_workspace_size": (_Z, [_P]),
+    "nsa_decode_attn": (_I, [_P, _P, _Z, _P]),
 })
+
+
+class DecodeArgs(ctypes.Structure):
+    """nsa_decode_args of include/nsa_hip.h."""
+
+    _fields_ = [("q", _P), ("k", _P * 3), ("v", _P * 3), ("indices", _P), ("gates", _P), ("out", _P),
+                ("stride_qz", _L), ("stride_qh", _L), ("stride_oz", _L), ("stride_oh", _L),
+                ("stride_kz", _L * 3), ("stride_kg", _L * 3), ("stride_kt", _L * 3),
+                ("stride_vz", _L * 3), ("stride_vg", _L * 3), ("stride_vt", _L * 3),
+                ("stride_gz", _L), ("stride_gh", _L), ("stride_gk", _L),
+                ("Z", _I), ("H", _I), ("n_kv_groups", _I), ("t", _I), ("n_cmp", _I), ("n_slots", _I),
+                ("block_size_selection", _I), ("window_size", _I), ("head_dim_qk", _I), ("head_dim_v", _I),
+                ("gate_act", _I), ("dtype", _I), ("sm_scale", _F)]
+
 
 _lock = threading.Lock()
 _lib = None

@@ -302,3 +302,41 @@ def attn_bwd(branch: int, q, k, v, o, do, L, M, scale: float, *, window: int = 0
         else:
             dv = r if q.dtype == cdt else r.to(q.dtype)
     return dq, dk, dv
+
+
+def decode_direct(q, kv, n_slots: int, lprime: int) -> bool:
+    """Whether decode_attn takes these tensors as they are: one dtype (fp32 / bf16), a
+    compiled head-width pair, unit-stride 16-byte aligned rows, at least one slot."""
+    dt = q.dtype
+    dk, dv = kv[0].shape[-1], kv[1].shape[-1]
+    return (dt in (torch.float32, torch.bfloat16) and (dk, dv) in HEAD_DIM_PAIRS and 1 <= n_slots <= 64
+            and lprime % 16 == 0 and all(t.dtype == dt and _rows_ok(t) for t in (q, *kv)))
+
+
+def decode_attn(q, kv, n_cmp: int, indices, gates, gate_act: int, t: int, scale: float, lprime: int, window: int):
+    """One decode step's attention and gated mix (nsa_decode_attn): q [Z,H,1,dk] at absolute
+    position t; kv = (K_cmp, V_cmp, K_sel, V_sel, K_win, V_win), views [Z,G,tokens,*] of the
+    caches, of which the first n_cmp compressed and t + 1 other tokens are read; indices
+    [Z,G,1,n] int64 contiguous, distinct in a row; gates [Z,H,1,3] (before the activation) in
+    q's dtype.  Returns the mixed output [Z,H,1,dv] of [Z,1,H,dv] storage."""
+    _check_device(q, *kv, indices, gates)
+    Z, H, _, dk = q.shape
+    G, dv = kv[0].shape[1], kv[1].shape[-1]
+    out = torch.empty(Z, 1, H, dv, device=q.device, dtype=q.dtype)
+    a = _lib.DecodeArgs()
+    a.q, a.stride_qz, a.stride_qh = q.data_ptr(), q.stride(0), q.stride(1)
+    for i in range(3):
+        k, v = kv[2 * i], kv[2 * i + 1]
+        a.k[i], a.v[i] = k.data_ptr(), v.data_ptr()
+        a.stride_kz[i], a.stride_kg[i], a.stride_kt[i] = k.stride()[:3]
+        a.stride_vz[i], a.stride_vg[i], a.stride_vt[i] = v.stride()[:3]
+    a.indices, a.gates, a.out = indices.data_ptr(), gates.data_ptr(), out.data_ptr()
+    a.stride_gz, a.stride_gh, _, a.stride_gk = gates.stride()
+    a.stride_oz, a.stride_oh = out.stride(0), out.stride(2)
+    a.Z, a.H, a.n_kv_groups, a.t, a.n_cmp, a.n_slots = Z, H, G, t, n_cmp, indices.shape[-1]
+    a.block_size_selection, a.window_size, a.head_dim_qk, a.head_dim_v = lprime, window, dk, dv
+    a.gate_act, a.dtype, a.sm_scale = gate_act, _dtype_code(q.dtype), scale
+    p = ctypes.byref(a)
+    ws = torch.empty(max(int(_lib.load().nsa_decode_workspace_size(p)), 1), device=q.device, dtype=torch.uint8)
+    _lib.call("nsa_decode_attn", p, _ptr(ws), ws.numel(), _stream(q.device))
+    return out.transpose(1, 2)

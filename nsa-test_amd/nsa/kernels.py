@@ -673,8 +673,8 @@ def score_and_select(q: torch.Tensor, k_compressed: torch.Tensor, block_ends: to
     G, N = k_compressed.shape[1], k_compressed.shape[-1]
     cdt = _ops.compute_dtype(q.dtype)
     qc = q.to(cdt)
-    # the kernel reads each compressed key as one row: [B,G,N,dk] storage
-    kc = k_compressed.to(cdt).transpose(-1, -2).contiguous().transpose(-1, -2)
+    # the kernel reads each compressed key as one row (unit-stride features)
+    kc = _ops._rows(_kt(k_compressed.to(cdt))).transpose(-1, -2)
     be = block_ends.to(torch.int32).contiguous()
     s = config.l_prime // config.d
     nsel = (N + s - 1) // s
@@ -724,7 +724,8 @@ class NSAKVCache:
         self.k_win, self.v_win = buf(dk), buf(dv)
         n_max = max((max_len - c.l) // c.d + 1, 0)
         np_max = _n_pad(max(n_max, 1))
-        self.K_cmp = torch.zeros(batch, G, dk, np_max, device=device, dtype=dtype)
+        # [B,G,dk,Np] over [B,G,Np,dk] storage: a compressed key is one row for the kernels
+        self.K_cmp = torch.zeros(batch, G, np_max, dk, device=device, dtype=dtype).transpose(-1, -2)
         self.V_cmp = torch.zeros(batch, G, np_max, dv, device=device, dtype=dtype)
         self.block_ends = torch.full((np_max,), 999999, device=device, dtype=torch.int32)
         self.n_act = 0
@@ -863,15 +864,20 @@ class NSAAttention(torch.nn.Module):
         sel = score_and_select(q, kc, be, self.scale, c, return_scores=output_attentions, q_offset=t)
         indices = sel[0] if output_attentions else sel
         n = t + 1
-        o_c, _, _ = _ops.attn_fwd(COMPRESSION, q, _kt(kc), vc, self.scale, block_ends=be, q_offset=t)
-        o_s, _, _ = _ops.attn_fwd(SELECTION, q, cache.k_sel[:, :, :n], cache.v_sel[:, :, :n], self.scale,
-                                  indices=indices, lprime=c.l_prime, fallback=True, q_offset=t)
-        o_w, _, _ = _ops.attn_fwd(SLIDING, q, cache.k_win[:, :, :n], cache.v_win[:, :, :n], self.scale, window=c.w,
-                                  q_offset=t)
         gate_logits = self.gate_mlp(x).view(B, 1, H, 3).permute(0, 2, 1, 3)
-        cdt = _ops.compute_dtype(q.dtype)
-        os_ = [o.to(cdt).contiguous() for o in (o_c, o_s, o_w)]
-        o = _mix_fwd(os_, gate_logits.to(cdt), GATE_ACT[c.gate_mode]).to(q.dtype)
+        kv = (_kt(kc), vc, cache.k_sel, cache.v_sel, cache.k_win, cache.v_win)
+        if _ops.decode_direct(q, kv, c.n, c.l_prime) and gate_logits.dtype == q.dtype:
+            o = _ops.decode_attn(q, kv, cache.n_act, indices, gate_logits, GATE_ACT[c.gate_mode], t, self.scale,
+                                 c.l_prime, c.w)
+        else:  # padded head widths, mixed dtypes or layouts the decode kernel does not read
+            o_c, _, _ = _ops.attn_fwd(COMPRESSION, q, _kt(kc), vc, self.scale, block_ends=be, q_offset=t)
+            o_s, _, _ = _ops.attn_fwd(SELECTION, q, cache.k_sel[:, :, :n], cache.v_sel[:, :, :n], self.scale,
+                                      indices=indices, lprime=c.l_prime, fallback=True, q_offset=t)
+            o_w, _, _ = _ops.attn_fwd(SLIDING, q, cache.k_win[:, :, :n], cache.v_win[:, :, :n], self.scale,
+                                      window=c.w, q_offset=t)
+            cdt = _ops.compute_dtype(q.dtype)
+            os_ = [o.to(cdt).contiguous() for o in (o_c, o_s, o_w)]
+            o = _mix_fwd(os_, gate_logits.to(cdt), GATE_ACT[c.gate_mode]).to(q.dtype)
         out = self.dropout(self.o_proj(o.transpose(1, 2).reshape(B, 1, H * dv)))  # as forward does
         info = None
         if output_attentions:

@@ -58,3 +58,51 @@ def test_score_few_rows(dev, B, G, hpg, T, N, dk, l, lp, dtype):
                              n=9, positions=np.arange(q0, q0 + T, dtype=np.int32), want_scores=True)
     for a, b in zip(got, want):
         np.testing.assert_array_equal(a.cpu().numpy(), b)
+
+
+# the decode step's split over 256-key workgroups and 64-key waves: positions at their edges and
+# at block edges, no compressed token / one / 256 / 257, 1 / 4 / 16 / 17 / 40 heads a group (head
+# tiles), every compiled width, windows of one key and past the sequence, empty slots, caches of
+# either layout
+@pytest.mark.parametrize("B,G,hpg,t,n_cmp,dk,dv,lp,n,w,act", [
+    (1, 1, 16, 0, 0, 64, 64, 64, 1, 512, 1), (2, 2, 4, 255, 15, 32, 32, 16, 5, 1, 2),
+    (1, 2, 1, 256, 1, 128, 128, 48, 16, 256, 0), (1, 2, 17, 4159, 257, 64, 64, 64, 16, 257, 1),
+    (3, 1, 40, 4160, 256, 192, 128, 64, 4, 9000, 2), (1, 1, 16, 319, 18, 128, 128, 32, 64, 65, 1)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_decode_attention_edges(dev, B, G, hpg, t, n_cmp, dk, dv, lp, n, w, act, dtype):
+    H, T = G * hpg, t + 7  # the cache is longer than the sequence
+    g = torch.Generator().manual_seed(t + dk)
+
+    def rnd(*s):
+        return torch.randn(*s, generator=g).to(dtype)
+
+    q, gates = rnd(B, H, 1, dk), rnd(B, 1, H, 3).permute(0, 2, 1, 3)
+    nc = max(n_cmp, 1) + 3
+    kv = [rnd(B, G, nc, dk), rnd(B, nc, G, dv).transpose(1, 2), rnd(B, G, T, dk), rnd(B, G, T, dv),
+          rnd(B, T, G, dk).transpose(1, 2), rnd(B, G, T, dv)]
+    nb = t // lp + 1
+    idx = torch.stack([torch.randperm(max(nb + 2, n), generator=g)[:n] for _ in range(B * G)]).view(B, G, 1, n)
+    idx[torch.rand(B, G, 1, n, generator=g) < 0.2] = -1
+    idx[0, 0] = -1  # a row without any block takes its own
+    # what lies past the sequence never reaches a result
+    for x, e in ((kv[0], n_cmp), (kv[1], n_cmp), *((x, t + 1) for x in kv[2:])):
+        x[:, :, e:] = float("nan")
+    dkv = [x.to(dev) for x in kv]
+    assert _ops.decode_direct(q.to(dev), dkv, n, lp)
+    out = _ops.decode_attn(q.to(dev), dkv, n_cmp, idx.to(dev), gates.to(dev), act, t, dk ** -0.5, lp, w)
+    pos = dict(positions=np.array([t], np.int32))
+    a = [x.double().numpy() for x in kv]
+    be = np.arange(n_cmp, dtype=np.int32) * 0
+    cut = [x[:, :, :t + 1] for x in a[2:]]
+    qd = q.double().numpy()
+    sel = idx.numpy().copy()
+    sel[(sel < 0).all(-1)] = t // lp
+    o = [oracle.attn_fwd(oracle.COMPRESSION, qd, a[0][:, :, :n_cmp], a[1][:, :, :n_cmp], dk ** -0.5, block_ends=be,
+                         **pos)[0] if n_cmp else np.zeros((B, H, 1, dv)),
+         oracle.attn_fwd(oracle.SELECTION, qd, cut[0], cut[1], dk ** -0.5, indices=sel, lprime=lp, **pos)[0],
+         oracle.attn_fwd(oracle.SLIDING, qd, cut[2], cut[3], dk ** -0.5, window=w, **pos)[0]]
+    z = gates.double()
+    z = (z, torch.sigmoid(z), torch.softmax(z, -1))[act].numpy()
+    want = sum(z[..., i:i + 1] * o[i] for i in range(3))
+    err = np.linalg.norm(out.double().cpu().numpy() - want) / np.linalg.norm(want)
+    assert err < (2e-2 if dtype == torch.bfloat16 else 1e-5), err
