@@ -449,6 +449,22 @@ size_t nsa_wgrad_workspace_size(int rows, int n1, int n2);
 int nsa_wgrad(const void* dY, int64_t ld_dy, const void* X, int64_t ld_x, int rows, int n1, int n2, void* dW,
               int64_t ld_dw, int dtype, void* workspace, size_t workspace_bytes, nsa_stream_t stream);
 
+/* ---- linear layers over a few rows (no reference counterpart: torch GEMMs there) ------
+ * For each job: y[r][n] = act(sum_k x[r][k] w[n][k] + bias[n]), r < rows (1 to 64), n < n;
+ * fp32 sums, rounded to dtype once.  x [rows, k] and w [n, k] have unit-stride, 16-byte
+ * aligned rows of whole 16-byte pieces; bias [n] may be null; relu: 0 or 1.  y[r][n] is stored
+ * at out + r * stride_row + (n / group) * stride_group + n % group; group is n or more (one
+ * run), or a multiple of 16 that divides n.  Up to 8 jobs run in one launch. */
+typedef struct nsa_linear_job {
+  const void* w;
+  const void* bias;
+  void* out;
+  int64_t ldw, stride_row, stride_group;
+  int n, group, relu;
+} nsa_linear_job;
+int nsa_linear_few(const void* x, int64_t ld_x, int rows, int k, const nsa_linear_job* jobs, int n_jobs, int dtype,
+                   nsa_stream_t stream);
+
 /* ---- one decode step (no reference counterpart) --------------------------------------
  * The attention of one timestep per batch entry at absolute position t (the caches hold
  * positions 0 .. t): out[z,h] = sum over the branches (0 compression, 1 selection, 2 sliding

@@ -82,7 +82,15 @@ SIGNATURES.update({
     "nsa_bwd_dkdv_plan": (_I, [_I] * 9 + [_P, _P]),
     "nsa_decode_workspace_size": (_Z, [_P]),
     "nsa_decode_attn": (_I, [_P, _P, _Z, _P]),
+    "nsa_linear_few": (_I, [_P, _L, _I, _I, _P, _I, _I, _P]),
 })
+
+
+class LinearJob(ctypes.Structure):
+    """nsa_linear_job of include/nsa_hip.h."""
+
+    _fields_ = [("w", _P), ("bias", _P), ("out", _P), ("ldw", _L), ("stride_row", _L), ("stride_group", _L), ("n", _I),
+                ("group", _I), ("relu", _I)]
 
 
 class DecodeArgs(ctypes.Structure):

@@ -309,7 +309,10 @@ def decode_direct(q, kv, n_slots: int, lprime: int) -> bool:
     compiled head-width pair, unit-stride 16-byte aligned rows, at least one slot."""
     dt = q.dtype
     dk, dv = kv[0].shape[-1], kv[1].shape[-1]
-    return (dt in (torch.float32, torch.bfloat16) and (dk, dv) in HEAD_DIM_PAIRS and 1 <= n_slots <= 64
+    Z, G = kv[0].shape[:2]
+    return (q.shape[0] == Z and q.shape[1] % G == 0 and q.shape[2:] == (1, dk)
+            and all(x.shape[:2] == (Z, G) and x.shape[-1] == (dv if i & 1 else dk) for i, x in enumerate(kv))
+            and dt in (torch.float32, torch.bfloat16) and (dk, dv) in HEAD_DIM_PAIRS and 1 <= n_slots <= 64
             and lprime % 16 == 0 and all(t.dtype == dt and _rows_ok(t) for t in (q, *kv)))
 
 
@@ -322,6 +325,10 @@ def decode_attn(q, kv, n_cmp: int, indices, gates, gate_act: int, t: int, scale:
     _check_device(q, *kv, indices, gates)
     Z, H, _, dk = q.shape
     G, dv = kv[0].shape[1], kv[1].shape[-1]
+    if (min(x.shape[2] for x in kv[:2]) < n_cmp or min(x.shape[2] for x in kv[2:]) <= t
+            or indices.dtype != torch.int64 or not indices.is_contiguous() or indices.shape[:3] != (Z, G, 1)
+            or gates.shape != (Z, H, 1, 3) or gates.dtype != q.dtype):
+        raise ValueError(f"decode_attn: caches shorter than t = {t} / {n_cmp} blocks, or indices / gates of another form")
     out = torch.empty(Z, 1, H, dv, device=q.device, dtype=q.dtype)
     a = _lib.DecodeArgs()
     a.q, a.stride_qz, a.stride_qh = q.data_ptr(), q.stride(0), q.stride(1)
@@ -340,3 +347,24 @@ def decode_attn(q, kv, n_cmp: int, indices, gates, gate_act: int, t: int, scale:
     ws = torch.empty(max(int(_lib.load().nsa_decode_workspace_size(p)), 1), device=q.device, dtype=torch.uint8)
     _lib.call("nsa_decode_attn", p, _ptr(ws), ws.numel(), _stream(q.device))
     return out.transpose(1, 2)
+
+
+# Rows up to which linear_few stands for torch's GEMMs: 64 (the kernel's most) for a token's
+# eight projections in one launch, 16 for a single layer.  Measured in bf16, launch against
+# F.linear: 17408 x 2560 weights (as one layer) 1 / 16 / 32 / 64 rows 17 / 25 / 43 / 70 us against 35 /
+# 35 / 19 / 19 us, where eight layers take eight such GEMMs and six cache copies; 2560 x 8192
+# 13 / 20 / 26 / 38 us against 19 us; 2304 x 512 6 us against 19 us (its host time).
+LINEAR_FEW_ROWS, LINEAR_ONE_ROWS = 64, 16
+
+
+def linear_few(x, jobs) -> None:
+    """Linear layers over the few rows of x [rows, k] in one launch (nsa_linear_few): jobs of
+    (weight [n, k], bias or None, out, stride_row, stride_group, group, relu), out a tensor at
+    whose data pointer feature n of row r lies stride_row r + stride_group (n // group) +
+    n % group elements further on."""
+    arr = (_lib.LinearJob * len(jobs))()
+    for j, (w, b, out, sr, sg, group, relu) in zip(arr, jobs):
+        j.w, j.bias, j.out = w.data_ptr(), None if b is None else b.data_ptr(), out.data_ptr()
+        j.ldw, j.stride_row, j.stride_group, j.n, j.group, j.relu = w.stride(0), sr, sg, w.shape[0], group, relu
+    _lib.call("nsa_linear_few", _ptr(x), x.stride(0), x.shape[0], x.shape[1], arr, len(jobs), _dtype_code(x.dtype),
+              _stream(x.device))

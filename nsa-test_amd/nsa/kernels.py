@@ -731,6 +731,31 @@ class NSAKVCache:
         self.n_act = 0
 
 
+def _plain_linears(x, *layers) -> bool:
+    """Whether nsa_linear_few may stand for these (torch.nn.Linear, in, out features) applied
+    to tensors like x: the modules themselves (no subclass, parametrisation, hook or patched
+    forward), outside autocast and torch's interception modes, with those widths, one dtype
+    and device, 16-byte aligned rows."""
+    gm = torch.nn.modules.module
+    dt, dev = x.dtype, x.device
+    if (type(x) is not torch.Tensor or not x.is_cuda or dt not in (torch.float32, torch.bfloat16)
+            or torch.is_autocast_enabled("cuda") or torch._C._len_torch_dispatch_stack()
+            or torch._C._len_torch_function_stack() or gm._global_forward_hooks or gm._global_forward_pre_hooks):
+        return False
+    for m, n_in, n_out in layers:
+        d = m.__dict__
+        if type(m) is not torch.nn.Linear or d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d:
+            return False
+        w, b = m.weight, m.bias
+        if (type(w) is not torch.nn.Parameter or w.dtype != dt or w.device != dev or w.shape != (n_out, n_in)
+                or not _ops._rows_ok(w)):
+            return False
+        if b is not None and (type(b) is not torch.nn.Parameter or b.dtype != dt or b.device != dev
+                              or b.shape != (n_out,) or not b.is_contiguous()):
+            return False
+    return True
+
+
 # ========================================================================= the module
 class NSAAttention(torch.nn.Module):
     """Native Sparse Attention layer (reference nsa/kernels.py:2043-2507): projections,
@@ -841,6 +866,48 @@ class NSAAttention(torch.nn.Module):
         cache.length = t0 + T
         self._add_blocks(cache)
 
+    def _decode_inputs(self, x: torch.Tensor, cache: NSAKVCache):
+        """The token x [B,1,D] joins the cache; returns its queries [B,H,1,dk] and gate logits
+        [B,H,1,3].  Plain layers over a few rows run in two launches (every projection of
+        the token at once, each written where it belongs; the gate's second layer); others
+        through the modules."""
+        c = self.config
+        B, _, D = x.shape
+        H, G, dk, dv, t = c.n_heads, c.n_kv_groups, c.head_dim_qk, c.head_dim_v, cache.length
+        kv = ((self.k_compress, cache.k_cmp_in, dk), (self.v_compress, cache.v_cmp_in, dv),
+              (self.k_select, cache.k_sel, dk), (self.v_select, cache.v_sel, dv),
+              (self.k_sliding, cache.k_win, dk), (self.v_sliding, cache.v_win, dv))
+        gm = self.gate_mlp
+        seq = (type(gm) is torch.nn.Sequential and len(gm) == 3 and type(gm[0]) is torch.nn.Linear
+               and type(gm[1]) is torch.nn.ReLU
+               and not any(m.__dict__[h] for m in (gm, gm[1]) for h in ("_forward_hooks", "_forward_pre_hooks")))
+        g0, g2, hw = (gm[0], gm[2], gm[0].out_features) if seq else (None, None, 0)
+        few = (seq and B <= _ops.LINEAR_FEW_ROWS and t < cache.max_len
+               and D * x.element_size() % 16 == 0 and hw * x.element_size() % 16 == 0
+               and type(self).prefill is NSAAttention.prefill and type(self)._project_kv is NSAAttention._project_kv
+               and _plain_linears(x, (self.q_proj, D, H * dk), (g0, D, hw), (g2, hw, 3 * H),
+                                  *((m, D, G * w) for m, _, w in kv))
+               and all(type(b) is torch.Tensor and b.dtype == x.dtype and b.device == x.device
+                       and b.shape == (B, G, cache.max_len, w) and b.stride(-1) == 1 and w % 16 == 0
+                       for _, b, w in kv))
+        if not few:
+            self.prefill(x, cache)
+            q = self.q_proj(x).view(B, 1, H, dk).transpose(1, 2).contiguous()
+            return q, gm(x).view(B, 1, H, 3).permute(0, 2, 1, 3)
+        x2 = _ops._rows(x.reshape(B, D))
+        q = x.new_empty(B, H, 1, dk)
+        hid = x.new_empty(B, hw)
+        z = x.new_empty(B, 1, H, 3)
+        jobs = [(self.q_proj.weight, self.q_proj.bias, q, H * dk, 0, H * dk, 0),
+                (g0.weight, g0.bias, hid, hw, 0, hw, 1)]
+        for m, b, _ in kv:
+            jobs.append((m.weight, m.bias, b[:, :, t], b.stride(0), b.stride(1), b.shape[-1], 0))
+        _ops.linear_few(x2, jobs)
+        _ops.linear_few(hid, [(g2.weight, g2.bias, z, 3 * H, 0, 3 * H, 0)])
+        cache.length = t + 1
+        self._add_blocks(cache)
+        return q, z.permute(0, 2, 1, 3)
+
     @torch.no_grad()
     def decode(self, hidden_states: torch.Tensor, cache: NSAKVCache, output_attentions: bool = False):
         """One decode step (not in the reference): hidden_states [B,1,D] is the token at
@@ -854,9 +921,8 @@ class NSAAttention(torch.nn.Module):
             raise ValueError("decode takes one token per step")
         H, dk, dv = c.n_heads, c.head_dim_qk, c.head_dim_v
         t = cache.length
-        self.prefill(hidden_states, cache)
         x = hidden_states
-        q = self.q_proj(x).view(B, 1, H, dk).transpose(1, 2).contiguous()           # [B,H,1,dk]
+        q, gate_logits = self._decode_inputs(x, cache)
         n_pad = _n_pad(max(cache.n_act, 1)) if cache.n_act > 0 else 1
         kc = cache.K_cmp[..., :n_pad]
         vc = cache.V_cmp[:, :, :n_pad]
@@ -864,7 +930,6 @@ class NSAAttention(torch.nn.Module):
         sel = score_and_select(q, kc, be, self.scale, c, return_scores=output_attentions, q_offset=t)
         indices = sel[0] if output_attentions else sel
         n = t + 1
-        gate_logits = self.gate_mlp(x).view(B, 1, H, 3).permute(0, 2, 1, 3)
         kv = (_kt(kc), vc, cache.k_sel, cache.v_sel, cache.k_win, cache.v_win)
         if _ops.decode_direct(q, kv, c.n, c.l_prime) and gate_logits.dtype == q.dtype:
             o = _ops.decode_attn(q, kv, cache.n_act, indices, gate_logits, GATE_ACT[c.gate_mode], t, self.scale,
@@ -878,7 +943,14 @@ class NSAAttention(torch.nn.Module):
             cdt = _ops.compute_dtype(q.dtype)
             os_ = [o.to(cdt).contiguous() for o in (o_c, o_s, o_w)]
             o = _mix_fwd(os_, gate_logits.to(cdt), GATE_ACT[c.gate_mode]).to(q.dtype)
-        out = self.dropout(self.o_proj(o.transpose(1, 2).reshape(B, 1, H * dv)))  # as forward does
+        of = o.transpose(1, 2).reshape(B, H * dv)
+        if (B <= _ops.LINEAR_ONE_ROWS and H * dv * of.element_size() % 16 == 0
+                and _plain_linears(of, (self.o_proj, H * dv, D))):
+            out = x.new_empty(B, 1, D)
+            _ops.linear_few(of, [(self.o_proj.weight, self.o_proj.bias, out, D, 0, D, 0)])
+        else:
+            out = self.o_proj(of.view(B, 1, H * dv))
+        out = self.dropout(out)  # as forward does
         info = None
         if output_attentions:
             gates = torch.softmax(gate_logits, dim=-1) if c.gate_mode == "softmax" else torch.sigmoid(gate_logits)

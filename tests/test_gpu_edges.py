@@ -8,7 +8,7 @@ import oracle
 import pytest
 import torch
 
-from nsa import NSAConfig, _ops
+from nsa import NSAAttention, NSAConfig, NSAKVCache, _ops
 from nsa.kernels import score_and_select
 from test_gpu_branches import _check, _make
 
@@ -106,3 +106,57 @@ def test_decode_attention_edges(dev, B, G, hpg, t, n_cmp, dk, dv, lp, n, w, act,
     want = sum(z[..., i:i + 1] * o[i] for i in range(3))
     err = np.linalg.norm(out.double().cpu().numpy() - want) / np.linalg.norm(want)
     assert err < (2e-2 if dtype == torch.bfloat16 else 1e-5), err
+
+
+# few-row linear layers: rows at the 16-row tiles, widths at the 16-feature tiles, inputs at the
+# 32- (16-) feature chunks, the eight waves' turns and a last chunk of one piece; several jobs,
+# grouped outputs, bias, relu.  fp32 sums: 1e-6 norm-relative; bf16 rounding of the result 2^-9
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("K", [8, 40, 256, 2568])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_linear_few(dev, rows, K, dtype):
+    g = torch.Generator().manual_seed(rows + K)
+    x = torch.randn(rows, K + 8, generator=g).to(dtype).to(dev)[:, :K]  # padded rows
+    jobs, want = [], []
+    for i, (n, group) in enumerate([(1, 1), (17, 17), (96, 32), (15, 40), (208, 208)]):
+        w = (torch.randn(n, K, generator=g) / K ** 0.5).to(dtype).to(dev)
+        b = torch.randn(n, generator=g).to(dtype).to(dev) if i % 2 else None
+        ng, gs = -(-n // group), group + 3
+        o = torch.full((rows, ng, gs), 7.0, dtype=dtype, device=dev)
+        y = x.double() @ w.double().t() + (b.double() if b is not None else 0)
+        y = y.relu() if i % 3 == 1 else y
+        r = o.double()
+        for j in range(ng):
+            r[:, j, :min(group, n - j * group)] = y[:, j * group:(j + 1) * group]
+        jobs.append((w, b, o, o.stride(0), o.stride(1), group, int(i % 3 == 1)))
+        want.append(r)
+    _ops.linear_few(x, jobs)
+    for (_, _, o, *_), r in zip(jobs, want):
+        assert ((o.double() - r).norm() / r.norm()).item() < (2 ** -9 if dtype == torch.bfloat16 else 1e-6)
+        assert torch.equal(o[..., -3:].double(), r[..., -3:])  # nothing past a group
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_decode_projections_direct_and_through_modules(dev, dtype):
+    """Biased layers, several sequences: the token's projections in one launch against the
+    modules' own (taken when a layer carries a hook), on outputs and every cache."""
+    cfg = NSAConfig(d_model=96, head_dim_qk=64, head_dim_v=64, n_heads=8, n_kv_groups=2, l_prime=32, n=4, w=40,
+                    use_bias=True)
+    torch.manual_seed(3)
+    m = NSAAttention(cfg).to(dev, dtype).eval()
+    x = torch.randn(3, 90, 96, device=dev).to(dtype)
+    calls, res = [], []
+    for hooked in (False, True):
+        h = m.k_select.register_forward_hook(lambda *_: calls.append(1)) if hooked else None
+        cache = NSAKVCache(cfg, 3, 90, dev, dtype)
+        m.prefill(x[:, :70], cache)
+        calls.clear()
+        out = torch.cat([m.decode(x[:, t:t + 1], cache)[0] for t in range(70, 90)], 1)
+        res.append((out, cache.k_cmp_in, cache.v_cmp_in, cache.k_sel, cache.v_sel, cache.k_win, cache.v_win))
+        assert len(calls) == (20 if hooked else 0) and cache.length == 90
+        if h:
+            h.remove()
+    for a, b in zip(*res):
+        assert ((a.double() - b.double()).norm() / b.double().norm()).item() < (1e-2 if dtype == torch.bfloat16 else 1e-5)
+    with pytest.raises(ValueError):
+        m.decode(x[:, :1], cache)  # the cache is full
