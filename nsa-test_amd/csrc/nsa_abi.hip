@@ -50,6 +50,7 @@ struct Shape {
   int esz() const { return dtype == NSA_F32 ? 4 : 2; }
   int nblk() const { return br == kSelection ? (Tkv + lprime - 1) / lprime : 0; }
   int nsubblk() const { return (lprime + 63) / 64; }
+  int key_tiles() const { return (Tkv + dkdv_keys(br) - 1) / dkdv_keys(br); }  // sliding / compression
   // dK/dV work items per (b, g): key tiles x query segments of sg entries
   int items_for(int sg) const {
     if (br == kSelection) return nsubblk() * (nblk() + (int)(((int64_t)Tq * nslots + sg - 1) / sg));
@@ -64,12 +65,22 @@ struct Shape {
   // segment length: the whole query span in direct mode; 256 entries when that leaves
   // 4096 work items or more; else the multiple of 32 in [128, 256] that needs the
   // fewest entry-steps per CU, ceil(items / 256 CUs) x segment (ties to the shorter),
-  // so that a small launch does not end on a partly filled round of work items
+  // so that a small launch does not end on a partly filled round of work items.  A launch that
+  // does not fill one round even at 128 entries goes down to 32, an item's fixed cost (K / V
+  // loads, pipeline fill, partial) counted as 16 entries: the compression of H64 G4 T2048 dk
+  // 192 had 64 items for 256 CUs (dK/dV 111 -> 40 us)
   int seg() const {
     if (direct()) return min(window + dkdv_keys(br) - 1, Tq + dkdv_keys(br) - 1);
     if ((int64_t)Z * G * items_for(kSegTMax) >= 4096) return kSegTMax;
     int best = kSegTMax / 2;
     int64_t best_cost = INT64_MAX;
+    if ((int64_t)Z * G * items_for(best) < 256) {
+      for (int sg = 32; sg <= kSegTMax / 2; sg += 32) {
+        const int64_t cost = ((int64_t)Z * G * items_for(sg) + 255) / 256 * (sg + 16);
+        if (cost < best_cost) best = sg, best_cost = cost;
+      }
+      return best;
+    }
     for (int sg = kSegTMax / 2; sg <= kSegTMax; sg += 32) {
       const int64_t cost = ((int64_t)Z * G * items_for(sg) + 255) / 256 * sg;
       if (cost < best_cost) best = sg, best_cost = cost;
@@ -108,7 +119,7 @@ struct Shape {
 
 struct Layout {
   size_t krf = 0, kcf = 0, vrf = 0, vcf = 0, rstat = 0, clean = 0, chunk = 0, csr_off = 0, csr_t = 0,
-         seg_off = 0, csr_s = 0, ds = 0, partial = 0, total = 0;
+         seg_off = 0, csr_s = 0, plan = 0, ds = 0, partial = 0, total = 0;
 };
 
 // Offsets into the caller's workspace (every buffer 256-byte aligned).
@@ -148,6 +159,7 @@ Layout make_layout(const Shape& s, bool bwd) {
     }
   }
   if (bwd && s.br != kSelection && s.stored_ds()) L.ds = take(s.ds_bytes());
+  if (bwd && s.br == kCompression) L.plan = take(((size_t)2 * s.key_tiles() + 2) * 4);
   if (bwd && !s.direct()) L.partial = take(BG * s.items_per_bg() * dkdv_keys(s.br) * (size_t)(s.dk + s.dv) * s.esz());
   L.total = off;
   return L;
@@ -417,6 +429,10 @@ int run_bwd(const Shape& s, const BwdIO& io, float scale, int window, const int3
     a.csr_off = at<int>(ws, L.csr_off);
     a.csr_t = at<int>(ws, L.csr_t);
     a.seg_off = at<int>(ws, L.seg_off);
+  }
+  if (s.br == kCompression) {
+    launch_cmp_plan(a, at<int>(ws, L.plan), st);
+    a.cmp_plan = at<int>(ws, L.plan);
   }
   if ((rc = check_hip("backward prep"))) return rc;
   auto dq = [&]() -> int {

@@ -101,6 +101,10 @@ struct AttnArgs {
   const int* csr_off;     // [B,G,nblk+1]
   const int* csr_t;       // [B,G,Tq*nslots] query timesteps per block, ascending
   const int* seg_off;     // [B,G,nblk+1] work-item prefix per block
+  // compression dK/dV work list, the same for every (batch, group) (cmp_plan_kernel): segment
+  // length, then [ntiles + 1] the item prefix per key tile, then [ntiles] each tile's first
+  // query row that sees one of its keys
+  const int* cmp_plan;
   const int* csr_s;       // [B,G,Tq*nslots] the slot of each CSR entry in its timestep's cleaned list
   // selection, stored-dS backward (bf16, hpg and l' multiples of 16 and 64): the dK/dV
   // kernel writes every (timestep, slot) pair's dS in the MFMA operand order of the dQ

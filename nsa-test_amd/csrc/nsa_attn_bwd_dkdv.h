@@ -22,6 +22,9 @@
 // each wave stores one whole 1 KB fragment of it, read back with two transpose loads as
 // the lane's eight keys of one head: its share of the dQ product's dS^T operand.
 //
+// Compression items come from a work list built from the block ends (cmp_plan_kernel): only
+// the rows that see a tile's keys, cut into equal segments over all tiles.
+//
 // Every item writes its fp32 dK/dV partial for its keys; a reduce kernel sums the
 // segments of each key tile in a fixed order and accumulates into the caller's dK/dV.
 // Direct mode (sliding window with at least kDkdvDirectItems key tiles over all batches
@@ -48,6 +51,17 @@ __host__ __device__ inline int dkdv_nseg(int br, int Tq, int window, int seg) {
     return (span + seg - 1) / seg;
   }
   return (Tq + seg - 1) / seg;
+}
+
+// the tile of a work item: the largest j < n with so[j] <= i, of the tiles' item prefix so
+__device__ __forceinline__ int item_tile(const int* so, int n, int i) {
+  int lo = 0, hi = n;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (so[mid] <= i) lo = mid;
+    else hi = mid;
+  }
+  return lo;
 }
 
 // the two-row transposed store of one staged 16-byte piece
@@ -161,36 +175,27 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(DK <= 64 &&
     f_lo = t_lo * hpg;
     f_hi = t_hi > t_lo ? t_hi * hpg : f_lo;
   } else if (BR == kCompression) {
-    const int nseg = dkdv_nseg(kCompression, a.Tq, 0, a.seg);
-    const int tile = item / nseg, seg = item % nseg;
+    const int ntiles = (a.Tkv + KEYS - 1) / KEYS;
+    const int sg = a.cmp_plan[0];
+    const int* so = a.cmp_plan + 1;
+    if (item >= so[ntiles]) return;  // beyond the work list (uniform)
+    const int tile = item_tile(so, ntiles, item);
     key0 = tile * KEYS;
     if (tid < KEYS) {
       const int key = key0 + tid;
       s_be[tid] = key < a.Tkv ? a.block_ends[key] : 0x7fffffff;
     }
     __syncthreads();
-    int be_min = 0x7fffffff;
-#pragma unroll
-    for (int c = 0; c < KEYS / 64; ++c) be_min = min(be_min, s_be[c * 64 + lane]);
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) be_min = min(be_min, __shfl_xor(be_min, o));
-    const int t_lo = max(seg * a.seg, max(be_min, 0));
-    const int t_hi = min(a.Tq, (seg + 1) * a.seg);
+    const int t_lo = so[ntiles + 1 + tile] + (item - so[tile]) * sg;
     f_lo = t_lo * hpg;
-    f_hi = t_hi > t_lo ? t_hi * hpg : f_lo;
+    f_hi = min(a.Tq, t_lo + sg) * hpg;
   } else {
     const int nsubblk = (a.lprime + 63) / 64;
     const int sidx = item / nsubblk;
     sub = item % nsubblk;
     const int* so = a.seg_off + (int64_t)bg * (a.nblk + 1);
     if (sidx >= so[a.nblk]) return;  // beyond this group's work list (uniform)
-    int lo = 0, hi = a.nblk;         // largest j with so[j] <= sidx
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (so[mid] <= sidx) lo = mid;
-      else hi = mid;
-    }
-    const int j = lo;
+    const int j = item_tile(so, a.nblk, sidx);
     const int k = sidx - so[j];
     const int* co = a.csr_off + (int64_t)bg * (a.nblk + 1);
     const int e_lo = co[j] + k * a.seg;

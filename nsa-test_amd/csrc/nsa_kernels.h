@@ -25,6 +25,8 @@ bool dispatch_attn_bwd_dkdv(int dtype, int dk, int dv, int br, const AttnArgs& a
 // lse2 / delta (/ row_dot) of every query row before a dK/dV kernel that runs first
 bool launch_row_stats(int dtype, int dv, const AttnArgs& a, hipStream_t st);
 void launch_partial_reduce(int dtype, int dk, int dv, int br, const AttnArgs& a, hipStream_t st);
+// the compression dK/dV work list (a.cmp_plan) of at most a.items_per_bg items
+void launch_cmp_plan(const AttnArgs& a, int* plan, hipStream_t st);
 // dK / dV [B, G, Tkv, dk | dv] (a.dk / a.dv, any strides) set to zero
 void launch_zero_dkdv(int dtype, int dk, int dv, const AttnArgs& a, hipStream_t st);
 

@@ -34,6 +34,69 @@ bool dispatch_attn_bwd_dkdv(int dtype, int dk, int dv, int br, const AttnArgs& a
                        : dispatch_attn_bwd_dkdv_bf16(dk, dv, br, a, st);
 }
 
+// The compression work list (one workgroup; AttnArgs::cmp_plan).  A key tile of 128 compressed
+// keys is seen from its earliest block end on, so the tiles' row spans shrink along the
+// sequence and end with the padding tiles' empty ones: cut at fixed rows for every tile, half
+// the items were empty, each still loading its keys and writing a partial of zeros, and the
+// busy ones filled their last round of CUs partly.  Here the segment length is the smallest
+// multiple of a row chunk with which the visible spans take at most max_items items.
+// dK/dV at B2 H32 G2 T5003 dk = dv = 128: 228 -> 115-136 us; H64 G4 T8192 dk = 192: 366 -> 322 us (with
+// 3 us more in the reduce and 4-7 us for this launch).
+__global__ __launch_bounds__(256) void cmp_plan_kernel(const int* block_ends, int Tkv, int Tq, int hpg, int seg_max,
+                                                       int max_items, int* plan) {
+  __shared__ int s_total, s_best;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int KEYS = dkdv_keys(kCompression);
+  const int ntiles = (Tkv + KEYS - 1) / KEYS;
+  int* so = plan + 1;
+  int* ts = so + ntiles + 1;
+  if (tid == 0) s_total = 0, s_best = 255;
+  __syncthreads();
+  int mine = 0;
+  for (int k = wave; k < ntiles; k += 4) {
+    int m = 0x7fffffff;
+    for (int i = lane; i < KEYS; i += 64)
+      if (k * KEYS + i < Tkv) m = min(m, block_ends[k * KEYS + i]);
+    m = wave_butterfly(m, [](int x, int y) { return min(x, y); });
+    m = min(max(m, 0), Tq);
+    if (lane == 0) ts[k] = m;
+    mine += Tq - m;
+  }
+  if (lane == 0) atomicAdd(&s_total, mine);
+  __syncthreads();  // ts and the total (at most ntiles x Tq rows) are written
+  // candidate i: (lo + i) row chunks; seg_max, among them, always fits
+  const int step = max(1, 32 / hpg);
+  const int lo = max(1, (s_total / max(max_items, 1) + step - 1) / step);
+  const int sg = min((lo + tid) * step, seg_max);
+  int n = 0;
+  for (int k = 0; k < ntiles && n <= max_items; ++k) n += (Tq - ts[k] + sg - 1) / sg;
+  if (n <= max_items) atomicMin(&s_best, tid);
+  __syncthreads();
+  const int best = min((lo + s_best) * step, seg_max);
+  if (tid == 0) plan[0] = best;
+  if (wave == 0) {  // item prefix of the tiles
+    int carry = 0;
+    for (int k0 = 0; k0 < ntiles; k0 += 64) {
+      const int k = k0 + lane;
+      int x = k < ntiles ? (Tq - ts[k] + best - 1) / best : 0;
+      const int own = x;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o);
+        if (lane >= o) x += y;
+      }
+      if (k < ntiles) so[k] = carry + x - own;
+      carry += __shfl(x, 63);
+    }
+    if (lane == 0) so[ntiles] = carry;
+  }
+}
+
+void launch_cmp_plan(const AttnArgs& a, int* plan, hipStream_t st) {
+  hipLaunchKernelGGL(cmp_plan_kernel, dim3(1), dim3(256), 0, st, a.block_ends, a.Tkv, a.Tq, a.hpg, a.seg,
+                     a.items_per_bg, plan);
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void partial_reduce_kernel(AttnArgs a, int DK, int DV, int br, int split) {
   using S = typename Store<T>::type;
@@ -42,12 +105,19 @@ __global__ __launch_bounds__(256) void partial_reduce_kernel(AttnArgs a, int DK,
   const int width = DK + DV;
   int key0, key_hi, first, count, step;
   const int keys = dkdv_keys(br);  // keys of one item's partial
-  if (br != kSelection) {
+  if (br == kSliding) {
     const int nseg = dkdv_nseg(br, a.Tq, a.window, a.seg);
     key0 = blockIdx.x * keys;
     key_hi = a.Tkv;
     first = blockIdx.x * nseg;
     count = nseg;
+    step = 1;
+  } else if (br == kCompression) {
+    const int* so = a.cmp_plan + 1;
+    key0 = blockIdx.x * keys;
+    key_hi = a.Tkv;
+    first = so[blockIdx.x];
+    count = so[blockIdx.x + 1] - first;
     step = 1;
   } else {
     const int nsubblk = (a.lprime + 63) / 64;

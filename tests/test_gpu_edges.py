@@ -160,3 +160,23 @@ def test_decode_projections_direct_and_through_modules(dev, dtype):
         assert ((a.double() - b.double()).norm() / b.double().norm()).item() < (1e-2 if dtype == torch.bfloat16 else 1e-5)
     with pytest.raises(ValueError):
         m.decode(x[:, :1], cache)  # the cache is full
+
+
+# the compression dK/dV work list: one to five key tiles of which the last ones are padding or
+# partly so, spans cut into segments down to 32 rows and into more than the list's cap of equal
+# cuts, 1 / 4 / 16 / 40 heads a group (row chunks of one timestep and of many), rows that see
+# nothing, no row that sees anything
+@pytest.mark.parametrize("B,G,hpg,T,l,d,dtype,dk,dv", [
+    (1, 1, 16, 300, 32, 16, torch.bfloat16, 64, 64), (2, 2, 16, 2100, 8, 8, torch.bfloat16, 128, 128),
+    (1, 2, 4, 1290, 4, 2, torch.bfloat16, 64, 64), (1, 1, 1, 700, 2, 1, torch.float32, 32, 32),
+    (1, 1, 40, 257, 32, 16, torch.bfloat16, 192, 128), (3, 1, 3, 20, 32, 16, torch.float32, 64, 64),
+    (1, 1, 8, 1060, 32, 4, torch.float32, 64, 64)])
+def test_compression_work_list(dev, B, G, hpg, T, l, d, dtype, dk, dv):
+    n_act = max((T - l) // d + 1, 0)
+    n_pad = 1
+    while n_pad < n_act:
+        n_pad *= 2
+    be = torch.full((n_pad,), 999999, dtype=torch.int32)
+    be[:n_act] = torch.arange(n_act, dtype=torch.int32) * d + l - 1
+    q, kp, v, do = _make(T, B, G * hpg, G, T, n_pad, dk, dv, dtype, dev)
+    _check(_ops.COMPRESSION, q, kp, v, do, 1 / math.sqrt(dk), dtype, block_ends=be.to(dev))
