@@ -437,6 +437,35 @@ int nsa_compress_pool_bwd(const void* Y, const void* C, const void* dR, const vo
                           void* dV, int Z, int n_kv_groups, int n_ctx, int width, int head_dim_v, int l, int d,
                           int n_act, int token_major, int dtype, nsa_stream_t stream);
 
+/* ---- compress_tokens around its two token-wise GEMMs ----------------------------------
+ * The module's whole compression (nsa/kernels.py:2119-2208) but for Y = k W1[:, :dk]^T
+ * (forward) and dR = dK W2, dk = dY W1[:, :dk] (backward), which the caller's GEMMs form.
+ * Forward: C [l,W] = E W1[:, dk:]^T + b1, R (pooled, as nsa_compress_pool_fwd), K [Z,G,n_pad,dk]
+ * = R W2^T + b2 and V_cmp [Z,G,n_pad,dv], the blocks from n_act on zero; W = 2 dk, R
+ * [Z,G,n_pad,W] (rows from n_act on not written).  Backward, from X = k, dK, dV_cmp and dR (the
+ * layouts of K, V_cmp, R): dY and dV (the layouts of Y, V), dW1, db1, dW2, db2, dE (each may be
+ * null); sums over rows in fp32 in a fixed order.  All tensors compact, 16-byte aligned,
+ * one dtype; token_major as above; b1 / b2 may be null.  dk a multiple of 64, l at most 64;
+ * l and dv whole 16-byte pieces, (W + dv) at most 256 of them. */
+typedef struct nsa_compress_args {
+  const void* Y;
+  void* C;
+  const void* V;
+  void* R;
+  void* K;
+  void* V_cmp;
+  const void *E, *W1, *b1, *W2, *b2;
+  int Z, n_kv_groups, n_ctx, head_dim_qk, head_dim_v, l, d, n_act, n_pad, token_major, dtype;
+} nsa_compress_args;
+typedef struct nsa_compress_grads {
+  const void *X, *dK, *dV_cmp, *dR;
+  void *dY, *dV, *dW1, *db1, *dW2, *db2, *dE;
+} nsa_compress_grads;
+int nsa_compress_fwd(const nsa_compress_args* args, nsa_stream_t stream);
+size_t nsa_compress_bwd_workspace_size(const nsa_compress_args* args);
+int nsa_compress_bwd(const nsa_compress_args* args, const nsa_compress_grads* grads, void* workspace,
+                     size_t workspace_bytes, nsa_stream_t stream);
+
 /* ---- weight gradient of the compression MLP's token-wise layers ----------------------
  * No counterpart in the reference (autograd computes it there).  dW [n1, n2] (leading
  * dimension ld_dw) = dY^T X over `rows` token rows: dY [rows, n1], X [rows, n2], bf16,

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "../../include/nsa_hip.h"
 #include "nsa_attn.h"
 
 // Head-dimension pairs (DK, DV) with compiled kernels.  Other widths are served by
@@ -61,6 +62,17 @@ struct DecodeArgs {
 void decode_split(DecodeArgs& a);  // nwg / nparts from the key counts
 size_t decode_part_bytes(const DecodeArgs& a, int dv);
 bool dispatch_decode(int dtype, int dk, int dv, const DecodeArgs& a, hipStream_t st);
+
+// one linear layer over `batches` groups of `rows` rows (x / out batch strides in elements;
+// row strides ldx and job.stride_row); returns NSA_OK or an error code
+int launch_linear_rows(const void* x, int64_t ldx, int rows, int k, int batches, int64_t x_batch, int64_t out_batch,
+                       const nsa_linear_job& job, int dtype, hipStream_t st);
+// dW (and, when not null, db = the column sums of dY) over `rows` rows, logical row r being
+// physical row r / rows_per * row_pitch + r % rows_per of both operands; n1, n2 multiples of
+// 64; part: wgrad_bytes of fp32 workspace
+size_t wgrad_bytes(int rows, int n1, int n2);
+void launch_wgrad(int dtype, const void* dy, int64_t ld_dy, const void* x, int64_t ld_x, int rows, int rows_per,
+                  int row_pitch, int n1, int n2, void* dw, int64_t ld_dw, void* db, float* part, hipStream_t st);
 
 // record an error message for nsa_last_error(); returns `code`
 int set_error(int code, const char* msg);

@@ -22,7 +22,8 @@ constexpr int kLinJobs = 8, kLinWaves = 8, kLinU = 10, kLinMaxRows = 64;
 struct LinearArgs {
   const void* x;
   int64_t ldx;
-  int rows, k, njobs;
+  int rows, k, njobs;               // rows of one batch (grid z); 16 RT of them per workgroup (grid y)
+  int64_t x_batch, out_batch;
   int tile0[kLinJobs + 1];  // first 16-feature tile of each job
   nsa_linear_job job[kLinJobs];
 };
@@ -41,10 +42,11 @@ __global__ __launch_bounds__(64 * kLinWaves) void linear_few_kernel(LinearArgs a
   const nsa_linear_job& jb = a.job[j];
   const int n0 = ((int)blockIdx.x - a.tile0[j]) * 16;
   const S* w = reinterpret_cast<const S*>(jb.w) + (int64_t)min(n0 + c16, jb.n - 1) * jb.ldw;
+  const int row0 = blockIdx.y * 16 * RT;
   const S* xr[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
-    xr[rt] = reinterpret_cast<const S*>(a.x) + (int64_t)min(rt * 16 + c16, a.rows - 1) * a.ldx;
+    xr[rt] = reinterpret_cast<const S*>(a.x) + blockIdx.z * a.x_batch + (int64_t)min(row0 + rt * 16 + c16, a.rows - 1) * a.ldx;
   f32x4 acc[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) acc[rt] = zero4();
@@ -76,14 +78,14 @@ __global__ __launch_bounds__(64 * kLinWaves) void linear_few_kernel(LinearArgs a
   for (int rt = 0; rt < RT; ++rt) s_acc[wave][rt][lane] = acc[rt];
   __syncthreads();
   if (wave >= RT) return;
-  const int row = wave * 16 + c16;
+  const int row = row0 + wave * 16 + c16;
   if (row >= a.rows) return;
   f32x4 v = s_acc[0][wave][lane];
 #pragma unroll
   for (int i = 1; i < kLinWaves; ++i) v += s_acc[i][wave][lane];
   // lane (g4, c16): features n0 + 4 g4 + i of row c16; a group holds whole 16-feature tiles
   const S* bias = reinterpret_cast<const S*>(jb.bias);
-  S* o = reinterpret_cast<S*>(jb.out) + row * jb.stride_row + (n0 / jb.group) * jb.stride_group + n0 % jb.group + 4 * g4;
+  S* o = reinterpret_cast<S*>(jb.out) + blockIdx.z * a.out_batch + row * jb.stride_row + (n0 / jb.group) * jb.stride_group + n0 % jb.group + 4 * g4;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int n = n0 + 4 * g4 + i;
@@ -95,11 +97,29 @@ __global__ __launch_bounds__(64 * kLinWaves) void linear_few_kernel(LinearArgs a
 }
 
 template <typename T>
-static void launch_linear(const LinearArgs& a, hipStream_t st) {
-  const dim3 grid(a.tile0[a.njobs]), block(64 * kLinWaves);
+static void launch_linear(const LinearArgs& a, int batches, hipStream_t st) {
+  const dim3 grid(a.tile0[a.njobs], (a.rows + 63) / 64, batches), block(64 * kLinWaves);
   if (a.rows <= 16) hipLaunchKernelGGL((linear_few_kernel<T, 1>), grid, block, 0, st, a);
   else if (a.rows <= 32) hipLaunchKernelGGL((linear_few_kernel<T, 2>), grid, block, 0, st, a);
   else hipLaunchKernelGGL((linear_few_kernel<T, 4>), grid, block, 0, st, a);
+}
+
+int launch_linear_rows(const void* x, int64_t ldx, int rows, int k, int batches, int64_t x_batch, int64_t out_batch,
+                       const nsa_linear_job& job, int dtype, hipStream_t st) {
+  LinearArgs a{};
+  a.x = x;
+  a.ldx = ldx;
+  a.rows = rows;
+  a.k = k;
+  a.njobs = 1;
+  a.x_batch = x_batch;
+  a.out_batch = out_batch;
+  a.job[0] = job;
+  a.tile0[1] = (job.n + 15) / 16;
+  if (dtype == NSA_F32) launch_linear<float>(a, batches, st);
+  else launch_linear<bf16>(a, batches, st);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? NSA_OK : set_error(NSA_ERR_HIP, hipGetErrorString(e));
 }
 
 }  // namespace nsa
@@ -128,8 +148,8 @@ extern "C" int nsa_linear_few(const void* x, int64_t ld_x, int rows, int k, cons
     a.job[j] = b;
     a.tile0[j + 1] = a.tile0[j] + (b.n + 15) / 16;
   }
-  if (dtype == NSA_F32) launch_linear<float>(a, (hipStream_t)stream);
-  else launch_linear<bf16>(a, (hipStream_t)stream);
+  if (dtype == NSA_F32) launch_linear<float>(a, 1, (hipStream_t)stream);
+  else launch_linear<bf16>(a, 1, (hipStream_t)stream);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? NSA_OK : set_error(NSA_ERR_HIP, hipGetErrorString(e));
 }

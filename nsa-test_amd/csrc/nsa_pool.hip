@@ -31,7 +31,7 @@ __global__ __launch_bounds__(256) void pool_fwd_kernel(const typename Store<T>::
                                                        const typename Store<T>::type* __restrict__ V,
                                                        typename Store<T>::type* __restrict__ R,
                                                        typename Store<T>::type* __restrict__ Vc, int T_, int W, int dv,
-                                                       int l, int d, int n_act, int G, int tm) {
+                                                       int l, int d, int n_act, int np, int G, int tm) {
   // grid: (n_act, B*G); threads stride over the W + dv channels
   const int i = blockIdx.x;
   const int64_t bg = blockIdx.y;
@@ -44,11 +44,11 @@ __global__ __launch_bounds__(256) void pool_fwd_kernel(const typename Store<T>::
         const float y = Elem<T>::to_f32(Y[pool_row(bg, t0 + u, T_, G, tm) * W + c]) + Elem<T>::to_f32(C[(int64_t)u * W + c]);
         acc += y > 0.f ? y : 0.f;
       }
-      R[(bg * n_act + i) * W + c] = Elem<T>::from_f32(acc * inv);
+      R[(bg * np + i) * W + c] = Elem<T>::from_f32(acc * inv);
     } else {
       const int e = c - W;
       for (int u = 0; u < l; ++u) acc += Elem<T>::to_f32(V[pool_row(bg, t0 + u, T_, G, tm) * dv + e]);
-      Vc[(bg * n_act + i) * dv + e] = Elem<T>::from_f32(acc * inv);
+      Vc[(bg * np + i) * dv + e] = Elem<T>::from_f32(acc * inv);
     }
   }
 }
@@ -62,7 +62,7 @@ __global__ __launch_bounds__(256) void pool_bwd_tok_kernel(const typename Store<
                                                            const typename Store<T>::type* __restrict__ dVc,
                                                            typename Store<T>::type* __restrict__ dY,
                                                            typename Store<T>::type* __restrict__ dV, int T_, int W,
-                                                           int dv, int l, int d, int n_act, int G, int tm) {
+                                                           int dv, int l, int d, int n_act, int np, int G, int tm) {
   const int t = blockIdx.x;
   const int64_t bg = blockIdx.y;
   const float inv = 1.0f / (float)l;
@@ -77,12 +77,12 @@ __global__ __launch_bounds__(256) void pool_bwd_tok_kernel(const typename Store<
       for (int i = i_lo; i <= i_hi; ++i) {
         const int u = t - d * i;
         if (y + Elem<T>::to_f32(C[(int64_t)u * W + c]) > 0.f)
-          acc += Elem<T>::to_f32(dR[(bg * n_act + i) * W + c]);
+          acc += Elem<T>::to_f32(dR[(bg * np + i) * W + c]);
       }
       dY[row * W + c] = Elem<T>::from_f32(acc * inv);
     } else {
       const int e = c - W;
-      for (int i = i_lo; i <= i_hi; ++i) acc += Elem<T>::to_f32(dVc[(bg * n_act + i) * dv + e]);
+      for (int i = i_lo; i <= i_hi; ++i) acc += Elem<T>::to_f32(dVc[(bg * np + i) * dv + e]);
       dV[row * dv + e] = Elem<T>::from_f32(acc * inv);
     }
   }
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(256) void pool_bwd_c_kernel(const typename Store<T>
                                                          const typename Store<T>::type* __restrict__ C,
                                                          const typename Store<T>::type* __restrict__ dR,
                                                          float* __restrict__ dC, int BG, int T_, int W, int l, int d,
-                                                         int n_act, int G, int tm) {
+                                                         int n_act, int np, int G, int tm) {
   // 64 channels x 4 interleaved block groups per workgroup; the 4 group sums are
   // combined in a fixed order
   __shared__ float part[4][64];
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256) void pool_bwd_c_kernel(const typename Store<T>
 #pragma unroll 4
       for (int i = ig; i < n_act; i += 4) {
         const float y = Elem<T>::to_f32(Y[pool_row(bg, (int64_t)i * d + u, T_, G, tm) * W + c]);
-        const float g = Elem<T>::to_f32(dR[(bg * n_act + i) * W + c]);
+        const float g = Elem<T>::to_f32(dR[(bg * np + i) * W + c]);
         acc += (y + cu > 0.f) ? g : 0.f;
       }
     }
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(256) void pool_bwd_tok_vec_kernel(const typename St
                                                                const typename Store<T>::type* __restrict__ dVc,
                                                                typename Store<T>::type* __restrict__ dY,
                                                                typename Store<T>::type* __restrict__ dV, int T_, int W,
-                                                               int dv, int l, int d, int n_act, int ppt, int G, int tm) {
+                                                               int dv, int l, int d, int n_act, int np, int ppt, int G, int tm) {
   constexpr int EPF = 16 / sizeof(typename Store<T>::type);
   const int tpw = 256 / ppt;
   const int t = blockIdx.x * tpw + threadIdx.x / ppt;
@@ -176,7 +176,7 @@ __global__ __launch_bounds__(256) void pool_bwd_tok_vec_kernel(const typename St
     for (int i = i_lo; i <= i_hi; ++i) {
       const int u = t - d * i;
       unpack16<T>(*reinterpret_cast<const uint4*>(C + (int64_t)u * W + c), cu);
-      unpack16<T>(*reinterpret_cast<const uint4*>(dR + (bg * n_act + i) * W + c), x);
+      unpack16<T>(*reinterpret_cast<const uint4*>(dR + (bg * np + i) * W + c), x);
 #pragma unroll
       for (int k = 0; k < EPF; ++k)
         if (y[k] + cu[k] > 0.f) acc[k] += x[k];
@@ -187,7 +187,7 @@ __global__ __launch_bounds__(256) void pool_bwd_tok_vec_kernel(const typename St
   } else {
     const int e = c - W;
     for (int i = i_lo; i <= i_hi; ++i) {
-      unpack16<T>(*reinterpret_cast<const uint4*>(dVc + (bg * n_act + i) * dv + e), x);
+      unpack16<T>(*reinterpret_cast<const uint4*>(dVc + (bg * np + i) * dv + e), x);
 #pragma unroll
       for (int k = 0; k < EPF; ++k) acc[k] += x[k];
     }
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(1024) void pool_bwd_c_vec_kernel(const typename Sto
                                                               const typename Store<T>::type* __restrict__ C,
                                                               const typename Store<T>::type* __restrict__ dR,
                                                               float* __restrict__ dC, int BG, int T_, int W, int l,
-                                                              int d, int n_act, int G, int tm) {
+                                                              int d, int n_act, int np, int G, int tm) {
   constexpr int EPF = 16 / sizeof(typename Store<T>::type);
   constexpr int NPC = 64 / EPF;             // piece columns per workgroup
   constexpr int NG = 1024 / NPC;            // row groups
@@ -224,7 +224,7 @@ __global__ __launch_bounds__(1024) void pool_bwd_c_vec_kernel(const typename Sto
       const int64_t bg = q / n_act;
       const int i = (int)(q % n_act);
       unpack16<T>(*reinterpret_cast<const uint4*>(Y + pool_row(bg, (int64_t)i * d + u, T_, G, tm) * W + c), y);
-      unpack16<T>(*reinterpret_cast<const uint4*>(dR + q * W + c), g);
+      unpack16<T>(*reinterpret_cast<const uint4*>(dR + (bg * np + i) * W + c), g);
 #pragma unroll
       for (int k = 0; k < EPF; ++k)
         if (y[k] + cu[k] > 0.f) acc[k] += g[k];
@@ -248,14 +248,21 @@ __global__ __launch_bounds__(256) void pool_fwd_vec_kernel(const typename Store<
                                                            const typename Store<T>::type* __restrict__ C,
                                                            const typename Store<T>::type* __restrict__ V,
                                                            typename Store<T>::type* __restrict__ R,
-                                                           typename Store<T>::type* __restrict__ Vc, int T_, int W,
-                                                           int dv, int l, int d, int n_act, int ppt, int G, int tm) {
+                                                           typename Store<T>::type* __restrict__ Vc,
+                                                           typename Store<T>::type* __restrict__ Kc, int dk, int T_,
+                                                           int W, int dv, int l, int d, int n_act, int np, int ppt, int G, int tm) {
   constexpr int EPF = 16 / sizeof(typename Store<T>::type);
   const int bpw = 256 / ppt;
   const int i = blockIdx.x * bpw + threadIdx.x / ppt;
   const int pc = threadIdx.x % ppt;
-  if (threadIdx.x >= bpw * ppt || i >= n_act) return;
+  if (threadIdx.x >= bpw * ppt || i >= np) return;
   const int64_t bg = blockIdx.y;
+  if (i >= n_act) {  // padding blocks: zero compressed keys and values (R is not read there)
+    const int c = pc * EPF;
+    if (c < dk) *reinterpret_cast<uint4*>(Kc + (bg * np + i) * dk + c) = make_uint4(0, 0, 0, 0);
+    if (c >= W) *reinterpret_cast<uint4*>(Vc + (bg * np + i) * dv + c - W) = make_uint4(0, 0, 0, 0);
+    return;
+  }
   const float inv = 1.0f / (float)l;
   const int64_t t0 = (int64_t)i * d;
   float acc[EPF], x[EPF];
@@ -276,7 +283,7 @@ __global__ __launch_bounds__(256) void pool_fwd_vec_kernel(const typename Store<
     }
 #pragma unroll
     for (int k = 0; k < EPF; ++k) acc[k] *= inv;
-    *reinterpret_cast<uint4*>(R + (bg * n_act + i) * W + c) = pack16<T>(acc);
+    *reinterpret_cast<uint4*>(R + (bg * np + i) * W + c) = pack16<T>(acc);
   } else {
     const int e = c - W;
 #pragma unroll 8
@@ -287,8 +294,88 @@ __global__ __launch_bounds__(256) void pool_fwd_vec_kernel(const typename Store<
     }
 #pragma unroll
     for (int k = 0; k < EPF; ++k) acc[k] *= inv;
-    *reinterpret_cast<uint4*>(Vc + (bg * n_act + i) * dv + e) = pack16<T>(acc);
+    *reinterpret_cast<uint4*>(Vc + (bg * np + i) * dv + e) = pack16<T>(acc);
   }
+}
+
+// R / V_cmp of blocks 0 .. n_act - 1 of every (b, g), np block rows apart.  With np > n_act
+// (vectorised form only) the padding rows of Vc and of Kc [B,G,np,dk] are zeroed.
+template <typename T>
+static void pool_fwd(const void* Y, const void* C, const void* V, void* R, void* Vc, void* Kc, int dk, int Z, int G,
+                     int n_ctx, int W, int dv, int l, int d, int n_act, int np, int tm, hipStream_t st) {
+  using S = typename Store<T>::type;
+  const int epf = 16 / (int)sizeof(S), ppt = (W + dv) / epf;
+  const bool al = ((uintptr_t)Y | (uintptr_t)C | (uintptr_t)V | (uintptr_t)R | (uintptr_t)Vc) % 16 == 0;
+  if (al && W % epf == 0 && dv % epf == 0 && ppt <= 256) {
+    const int bpw = 256 / ppt;
+    hipLaunchKernelGGL(pool_fwd_vec_kernel<T>, dim3((np + bpw - 1) / bpw, Z * G), dim3(256), 0, st, (const S*)Y,
+                       (const S*)C, (const S*)V, (S*)R, (S*)Vc, (S*)Kc, dk, n_ctx, W, dv, l, d, n_act, np, ppt, G, tm);
+  } else {
+    hipLaunchKernelGGL(pool_fwd_kernel<T>, dim3(n_act, Z * G), dim3(256), 0, st, (const S*)Y, (const S*)C,
+                       (const S*)V, (S*)R, (S*)Vc, n_ctx, W, dv, l, d, n_act, np, G, tm);
+  }
+}
+
+template <typename T>
+static void pool_bwd(const void* Y, const void* C, const void* dR, const void* dVc, void* dY, float* dC, void* dV,
+                     int Z, int G, int n_ctx, int W, int dv, int l, int d, int n_act, int np, int tm, hipStream_t st) {
+  using S = typename Store<T>::type;
+  const int epf = 16 / (int)sizeof(S), ppt = (W + dv) / epf;
+  const bool al = ((uintptr_t)Y | (uintptr_t)C | (uintptr_t)dR | (uintptr_t)dVc | (uintptr_t)dY | (uintptr_t)dV) % 16 == 0;
+  const dim3 gc((W + 63) / 64, l);
+  if (al && W % epf == 0 && dv % epf == 0 && ppt <= 256) {
+    const int tpw = 256 / ppt;
+    hipLaunchKernelGGL(pool_bwd_tok_vec_kernel<T>, dim3((n_ctx + tpw - 1) / tpw, Z * G), dim3(256), 0, st,
+                       (const S*)Y, (const S*)C, (const S*)dR, (const S*)dVc, (S*)dY, (S*)dV, n_ctx, W, dv, l, d,
+                       n_act, np, ppt, G, tm);
+    hipLaunchKernelGGL(pool_bwd_c_vec_kernel<T>, gc, dim3(1024), 0, st, (const S*)Y, (const S*)C, (const S*)dR, dC,
+                       Z * G, n_ctx, W, l, d, n_act, np, G, tm);
+  } else {
+    hipLaunchKernelGGL(pool_bwd_tok_kernel<T>, dim3(n_ctx, Z * G), dim3(256), 0, st, (const S*)Y, (const S*)C,
+                       (const S*)dR, (const S*)dVc, (S*)dY, (S*)dV, n_ctx, W, dv, l, d, n_act, np, G, tm);
+    hipLaunchKernelGGL(pool_bwd_c_kernel<T>, gc, dim3(256), 0, st, (const S*)Y, (const S*)C, (const S*)dR, dC, Z * G,
+                       n_ctx, W, l, d, n_act, np, G, tm);
+  }
+}
+
+struct CompressBwd {
+  const void *E, *W1;
+  void *dW1, *db1, *dE;
+  int dk, W, l;
+};
+
+// Gradients of the position half of the first layer, C = E W1p^T + b1 (W1p = W1[:, dk:]), from
+// dC [l][W] fp32: dW1p[j][e] = sum_u dC[u][j] E[u][e], db1[j] = sum_u dC[u][j] (a thread each),
+// dE[u][e] = sum_j dC[u][j] W1p[j][e] (a wave each); fp32 sums in a fixed order, rounded once.
+template <typename T>
+__global__ __launch_bounds__(256) void compress_pos_grad_kernel(const float* __restrict__ dC, CompressBwd a) {
+  using S = typename Store<T>::type;
+  const int W = a.W, l = a.l, nw = W * l, ld1 = a.dk + l;
+  int q = blockIdx.x * 256 + threadIdx.x;
+  const int nthr = (nw + W + 255) / 256 * 256;
+  if (q < nthr) {
+    const int j = q < nw ? q / l : q - nw;
+    if (j >= W) return;
+    const S* E = reinterpret_cast<const S*>(a.E);
+    float s = 0.f;
+    if (q < nw) {
+      const int e = q % l;
+      for (int u = 0; u < l; ++u) s = fmaf(dC[u * W + j], Elem<T>::to_f32(E[u * l + e]), s);
+      if (a.dW1) reinterpret_cast<S*>(a.dW1)[(int64_t)j * ld1 + a.dk + e] = Elem<T>::from_f32(s);
+    } else {
+      for (int u = 0; u < l; ++u) s += dC[u * W + j];
+      if (a.db1) reinterpret_cast<S*>(a.db1)[j] = Elem<T>::from_f32(s);
+    }
+    return;
+  }
+  q = (q - nthr) >> 6;
+  if (q >= l * l || !a.dE) return;  // whole wave
+  const int u = q / l, e = q % l, lane = threadIdx.x & 63;
+  const S* W1 = reinterpret_cast<const S*>(a.W1);
+  float s = 0.f;
+  for (int j = lane; j < W; j += 64) s = fmaf(dC[u * W + j], Elem<T>::to_f32(W1[(int64_t)j * ld1 + a.dk + e]), s);
+  s = wave_butterfly(s, [](float x, float y) { return x + y; });
+  if (lane == 0) reinterpret_cast<S*>(a.dE)[u * l + e] = Elem<T>::from_f32(s);
 }
 
 }  // namespace nsa
@@ -300,39 +387,15 @@ using namespace nsa;
 extern "C" int nsa_compress_pool_fwd(const void* Y, const void* C, const void* V, void* R, void* Vc, int Z, int G,
                                      int n_ctx, int width, int head_dim_v, int l, int d, int n_act, int token_major,
                                      int dtype, nsa_stream_t stream) {
-  const int tm = token_major ? 1 : 0;
   if (dtype != NSA_F32 && dtype != NSA_BF16) return set_error(NSA_ERR_INVALID, "dtype not supported");
   if (Z <= 0 || G <= 0 || l <= 0 || d <= 0 || n_act < 0 || width <= 0 || head_dim_v <= 0)
     return set_error(NSA_ERR_INVALID, "bad shape");
   if (n_act > 0 && (int64_t)(n_act - 1) * d + l > n_ctx) return set_error(NSA_ERR_INVALID, "blocks exceed n_ctx");
   if (n_act == 0) return NSA_OK;
   TimingScope ts(kIdPoolFwd, (hipStream_t)stream);
-  dim3 grid(n_act, Z * G);
-  hipStream_t st = (hipStream_t)stream;
-  {
-    const int epf = dtype == NSA_F32 ? 4 : 8;
-    const int ppt = (width + head_dim_v) / epf;
-    const bool al = ((uintptr_t)Y | (uintptr_t)C | (uintptr_t)V | (uintptr_t)R | (uintptr_t)Vc) % 16 == 0;
-    if (al && width % epf == 0 && head_dim_v % epf == 0 && ppt <= 256) {
-      const int bpw = 256 / ppt;
-      dim3 gv((n_act + bpw - 1) / bpw, Z * G);
-      if (dtype == NSA_F32)
-        hipLaunchKernelGGL(pool_fwd_vec_kernel<float>, gv, dim3(256), 0, st, (const float*)Y, (const float*)C,
-                           (const float*)V, (float*)R, (float*)Vc, n_ctx, width, head_dim_v, l, d, n_act, ppt, G, tm);
-      else
-        hipLaunchKernelGGL(pool_fwd_vec_kernel<bf16>, gv, dim3(256), 0, st, (const uint16_t*)Y, (const uint16_t*)C,
-                           (const uint16_t*)V, (uint16_t*)R, (uint16_t*)Vc, n_ctx, width, head_dim_v, l, d, n_act,
-                           ppt, G, tm);
-      hipError_t e = hipGetLastError();
-      return e == hipSuccess ? NSA_OK : set_error(NSA_ERR_HIP, hipGetErrorString(e));
-    }
-  }
-  if (dtype == NSA_F32)
-    hipLaunchKernelGGL(pool_fwd_kernel<float>, grid, dim3(256), 0, st, (const float*)Y, (const float*)C,
-                       (const float*)V, (float*)R, (float*)Vc, n_ctx, width, head_dim_v, l, d, n_act, G, tm);
-  else
-    hipLaunchKernelGGL(pool_fwd_kernel<bf16>, grid, dim3(256), 0, st, (const uint16_t*)Y, (const uint16_t*)C,
-                       (const uint16_t*)V, (uint16_t*)R, (uint16_t*)Vc, n_ctx, width, head_dim_v, l, d, n_act, G, tm);
+  auto fn = dtype == NSA_F32 ? pool_fwd<float> : pool_fwd<bf16>;
+  fn(Y, C, V, R, Vc, nullptr, 0, Z, G, n_ctx, width, head_dim_v, l, d, n_act, n_act, token_major ? 1 : 0,
+     (hipStream_t)stream);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? NSA_OK : set_error(NSA_ERR_HIP, hipGetErrorString(e));
 }
@@ -348,46 +411,86 @@ extern "C" int nsa_compress_pool_bwd(const void* Y, const void* C, const void* d
     return set_error(NSA_ERR_INVALID, "bad shape");
   if (n_act > 0 && (int64_t)(n_act - 1) * d + l > n_ctx) return set_error(NSA_ERR_INVALID, "blocks exceed n_ctx");
   if (n_ctx == 0) return NSA_OK;
-  hipStream_t st = (hipStream_t)stream;
   TimingScope ts(kIdPoolBwd, (hipStream_t)stream);
-  dim3 gt(n_ctx, Z * G), gc((width + 63) / 64, l);
+  auto fn = dtype == NSA_F32 ? pool_bwd<float> : pool_bwd<bf16>;
+  fn(Y, C, dR, dVc, dY, dC, dV, Z, G, n_ctx, width, head_dim_v, l, d, n_act, n_act, token_major ? 1 : 0,
+     (hipStream_t)stream);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? NSA_OK : set_error(NSA_ERR_HIP, hipGetErrorString(e));
+}
+
+// ---- compress_tokens around the two token-wise GEMMs (Y = k W1k^T, dR = dK W2) ----
+static int check_compress(const nsa_compress_args* x) {
+  if (!x) return set_error(NSA_ERR_INVALID, "args is null");
+  if (x->dtype != NSA_F32 && x->dtype != NSA_BF16) return set_error(NSA_ERR_INVALID, "dtype not supported");
+  const int epf = x->dtype == NSA_F32 ? 4 : 8, W = 2 * x->head_dim_qk;
+  if (x->Z <= 0 || x->n_kv_groups <= 0 || x->n_act <= 0 || x->n_pad < x->n_act || x->l <= 0 || x->d <= 0 ||
+      (int64_t)(x->n_act - 1) * x->d + x->l > x->n_ctx)
+    return set_error(NSA_ERR_INVALID, "bad shape");
+  if (x->l > 64 || x->l % epf || x->head_dim_qk <= 0 || x->head_dim_qk % 64 || x->head_dim_v <= 0 ||
+      x->head_dim_v % epf || (W + x->head_dim_v) / epf > 256)
+    return set_error(NSA_ERR_UNSUPPORTED, "compress_tokens: widths without a kernel");
+  const void* in[] = {x->Y, x->C, x->V, x->R, x->K, x->V_cmp, x->E, x->W1, x->W2};
+  for (const void* p : in)
+    if (!p || (uintptr_t)p % 16) return set_error(NSA_ERR_LAYOUT, "compress_tokens: tensors must be 16-byte aligned");
+  return NSA_OK;
+}
+
+extern "C" int nsa_compress_fwd(const nsa_compress_args* x, nsa_stream_t stream) {
+  int rc = check_compress(x);
+  if (rc) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  const int dk = x->head_dim_qk, W = 2 * dk, esz = x->dtype == NSA_F32 ? 4 : 2, BG = x->Z * x->n_kv_groups;
+  // C = E W1p^T + b1, then the pooling, then K_cmp = R W2^T + b2 over each group's n_act rows
+  nsa_linear_job c{reinterpret_cast<const char*>(x->W1) + (size_t)dk * esz, x->b1, x->C, dk + x->l, W, 0, W, W, 0};
+  if ((rc = launch_linear_rows(x->E, x->l, x->l, x->l, 1, 0, 0, c, x->dtype, st))) return rc;
   {
-    const int epf = dtype == NSA_F32 ? 4 : 8;
-    const int ppt = (width + head_dim_v) / epf;
-    const bool al = ((uintptr_t)Y | (uintptr_t)C | (uintptr_t)dR | (uintptr_t)dVc | (uintptr_t)dY | (uintptr_t)dV) % 16 == 0;
-    if (al && width % epf == 0 && head_dim_v % epf == 0 && ppt <= 256) {
-      const int tpw = 256 / ppt;
-      dim3 gv((n_ctx + tpw - 1) / tpw, Z * G);
-      if (dtype == NSA_F32) {
-        hipLaunchKernelGGL(pool_bwd_tok_vec_kernel<float>, gv, dim3(256), 0, st, (const float*)Y, (const float*)C,
-                           (const float*)dR, (const float*)dVc, (float*)dY, (float*)dV, n_ctx, width, head_dim_v, l,
-                           d, n_act, ppt, G, tm);
-        hipLaunchKernelGGL(pool_bwd_c_vec_kernel<float>, gc, dim3(1024), 0, st, (const float*)Y, (const float*)C,
-                           (const float*)dR, dC, Z * G, n_ctx, width, l, d, n_act, G, tm);
-      } else {
-        hipLaunchKernelGGL(pool_bwd_tok_vec_kernel<bf16>, gv, dim3(256), 0, st, (const uint16_t*)Y,
-                           (const uint16_t*)C, (const uint16_t*)dR, (const uint16_t*)dVc, (uint16_t*)dY,
-                           (uint16_t*)dV, n_ctx, width, head_dim_v, l, d, n_act, ppt, G, tm);
-        hipLaunchKernelGGL(pool_bwd_c_vec_kernel<bf16>, gc, dim3(1024), 0, st, (const uint16_t*)Y,
-                           (const uint16_t*)C, (const uint16_t*)dR, dC, Z * G, n_ctx, width, l, d, n_act, G, tm);
-      }
-      hipError_t e = hipGetLastError();
-      return e == hipSuccess ? NSA_OK : set_error(NSA_ERR_HIP, hipGetErrorString(e));
-    }
+    TimingScope ts(kIdPoolFwd, st);
+    auto fn = x->dtype == NSA_F32 ? pool_fwd<float> : pool_fwd<bf16>;
+    fn(x->Y, x->C, x->V, x->R, x->V_cmp, x->K, dk, x->Z, x->n_kv_groups, x->n_ctx, W, x->head_dim_v, x->l, x->d,
+       x->n_act, x->n_pad, x->token_major ? 1 : 0, st);
   }
-  if (dtype == NSA_F32) {
-    hipLaunchKernelGGL(pool_bwd_tok_kernel<float>, gt, dim3(256), 0, st, (const float*)Y, (const float*)C,
-                       (const float*)dR, (const float*)dVc, (float*)dY, (float*)dV, n_ctx, width, head_dim_v, l, d,
-                       n_act, G, tm);
-    hipLaunchKernelGGL(pool_bwd_c_kernel<float>, gc, dim3(256), 0, st, (const float*)Y, (const float*)C,
-                       (const float*)dR, dC, Z * G, n_ctx, width, l, d, n_act, G, tm);
-  } else {
-    hipLaunchKernelGGL(pool_bwd_tok_kernel<bf16>, gt, dim3(256), 0, st, (const uint16_t*)Y, (const uint16_t*)C,
-                       (const uint16_t*)dR, (const uint16_t*)dVc, (uint16_t*)dY, (uint16_t*)dV, n_ctx, width,
-                       head_dim_v, l, d, n_act, G, tm);
-    hipLaunchKernelGGL(pool_bwd_c_kernel<bf16>, gc, dim3(256), 0, st, (const uint16_t*)Y, (const uint16_t*)C,
-                       (const uint16_t*)dR, dC, Z * G, n_ctx, width, l, d, n_act, G, tm);
+  nsa_linear_job k{x->W2, x->b2, x->K, W, dk, 0, dk, dk, 0};
+  return launch_linear_rows(x->R, W, x->n_act, W, BG, (int64_t)x->n_pad * W, (int64_t)x->n_pad * dk, k, x->dtype, st);
+}
+
+extern "C" size_t nsa_compress_bwd_workspace_size(const nsa_compress_args* x) {
+  if (check_compress(x)) return 0;
+  const int dk = x->head_dim_qk, W = 2 * dk, BG = x->Z * x->n_kv_groups;
+  const size_t a = wgrad_bytes(BG * x->n_act, dk, W), b = wgrad_bytes(BG * x->n_ctx, W, dk);
+  return (size_t)x->l * W * 4 + (a > b ? a : b);
+}
+
+extern "C" int nsa_compress_bwd(const nsa_compress_args* x, const nsa_compress_grads* g, void* ws, size_t ws_bytes,
+                                nsa_stream_t stream) {
+  int rc = check_compress(x);
+  if (rc) return rc;
+  if (!g || !g->X || !g->dK || !g->dV_cmp || !g->dR || !g->dY || !g->dV)
+    return set_error(NSA_ERR_INVALID, "compress_tokens: null gradient");
+  if (((uintptr_t)g->X | (uintptr_t)g->dK | (uintptr_t)g->dV_cmp | (uintptr_t)g->dR | (uintptr_t)g->dY |
+       (uintptr_t)g->dV) % 16)
+    return set_error(NSA_ERR_LAYOUT, "compress_tokens: gradients must be 16-byte aligned");
+  if (!ws || (uintptr_t)ws % 16 || ws_bytes < nsa_compress_bwd_workspace_size(x))
+    return set_error(NSA_ERR_WORKSPACE, "compress_tokens: workspace too small or not 16-byte aligned");
+  hipStream_t st = (hipStream_t)stream;
+  const int dk = x->head_dim_qk, W = 2 * dk, BG = x->Z * x->n_kv_groups, l = x->l;
+  float* dC = reinterpret_cast<float*>(ws);
+  float* part = dC + (size_t)l * W;
+  if (g->dW2 || g->db2)
+    launch_wgrad(x->dtype, g->dK, dk, x->R, W, BG * x->n_act, x->n_act, x->n_pad, dk, W, g->dW2, W, g->db2, part, st);
+  {
+    TimingScope ts(kIdPoolBwd, st);
+    auto fn = x->dtype == NSA_F32 ? pool_bwd<float> : pool_bwd<bf16>;
+    fn(x->Y, x->C, g->dR, g->dV_cmp, g->dY, dC, g->dV, x->Z, x->n_kv_groups, x->n_ctx, W, x->head_dim_v, l, x->d,
+       x->n_act, x->n_pad, x->token_major ? 1 : 0, st);
   }
+  CompressBwd a{x->E, x->W1, g->dW1, g->db1, g->dE, dk, W, l};
+  const unsigned blocks = (l * W + W + 255) / 256 + (l * l * 64 + 255) / 256;
+  if (x->dtype == NSA_F32) hipLaunchKernelGGL(compress_pos_grad_kernel<float>, dim3(blocks), dim3(256), 0, st, dC, a);
+  else hipLaunchKernelGGL(compress_pos_grad_kernel<bf16>, dim3(blocks), dim3(256), 0, st, dC, a);
+  if (g->dW1)
+    launch_wgrad(x->dtype, g->dY, W, g->X, dk, BG * x->n_ctx, BG * x->n_ctx, BG * x->n_ctx, W, dk, g->dW1, dk + l,
+                 nullptr, part, st);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? NSA_OK : set_error(NSA_ERR_HIP, hipGetErrorString(e));
 }

@@ -83,7 +83,25 @@ SIGNATURES.update({
     "nsa_decode_workspace_size": (_Z, [_P]),
     "nsa_decode_attn": (_I, [_P, _P, _Z, _P]),
     "nsa_linear_few": (_I, [_P, _L, _I, _I, _P, _I, _I, _P]),
+    "nsa_compress_fwd": (_I, [_P, _P]),
+    "nsa_compress_bwd_workspace_size": (_Z, [_P]),
+    "nsa_compress_bwd": (_I, [_P, _P, _P, _Z, _P]),
 })
+
+
+class CompressArgs(ctypes.Structure):
+    """nsa_compress_args of include/nsa_hip.h."""
+
+    _fields_ = [(n, _P) for n in ("Y", "C", "V", "R", "K", "V_cmp", "E", "W1", "b1", "W2", "b2")] + [
+        (n, _I) for n in ("Z", "n_kv_groups", "n_ctx", "head_dim_qk", "head_dim_v", "l", "d", "n_act", "n_pad",
+                          "token_major", "dtype")]
+
+
+class CompressGrads(ctypes.Structure):
+    """nsa_compress_grads of include/nsa_hip.h."""
+
+    _fields_ = [(n, _P) for n in ("X", "dK", "dV_cmp", "dR", "dY", "dV", "dW1", "db1", "dW2", "db2", "dE")]
+
 
 
 class LinearJob(ctypes.Structure):
@@ -167,6 +185,15 @@ def size(name: str, *args) -> int:
     r = _SIZE_CACHE.get(key)
     if r is None:
         r = _SIZE_CACHE[key] = int(getattr(load(), name)(*args))
+    return r
+
+
+def size_of(name: str, args, key) -> int:
+    """A workspace-size query over an argument struct whose sizes `key` determines."""
+    k = (name, key)
+    r = _SIZE_CACHE.get(k)
+    if r is None:
+        r = _SIZE_CACHE[k] = int(getattr(load(), name)(ctypes.byref(args)))
     return r
 
 

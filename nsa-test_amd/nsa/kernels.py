@@ -34,6 +34,7 @@ Deliberate differences from the reference, all toward its own oracle
 """
 from __future__ import annotations
 
+import ctypes
 import functools
 import math
 from dataclasses import dataclass
@@ -548,6 +549,81 @@ class _CompressPool(torch.autograd.Function):
         return dY.to(ydt), dC.to(cdt_in), dV.to(vdt), None, None, None, None
 
 
+def _compact(t):
+    """t contiguous and 16-byte aligned (a copy only when it is not)."""
+    return t if t.is_contiguous() and t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
+
+
+class _CompressTokens(torch.autograd.Function):
+    """compress_tokens as one function: two token-wise GEMMs (torch) around one HIP call each
+    way (nsa_compress_fwd / nsa_compress_bwd: position bias, pooling, output layer and block
+    padding; the pooling's and all weights' gradients).  keys / values [B,G,T,*], or [B,T,G,*]
+    with tm.  Returns (K_cmp as [B,G,Np,dk], V_cmp [B,G,Np,dv])."""
+
+    @staticmethod
+    def usable(keys, values, W1, b1, W2, b2, E, l) -> bool:
+        """Whether the HIP calls take these: fp32 / bf16 on the GPU outside autocast, dk a multiple
+        of 64, whole 16-byte pieces, the reference's weight shapes."""
+        dt, dk, dv = keys.dtype, keys.shape[-1], values.shape[-1]
+        if dt not in (torch.float32, torch.bfloat16) or not keys.is_cuda or torch.is_autocast_enabled("cuda"):
+            return False
+        epf = 16 // keys.element_size()
+        ts = [values, W1, W2, E] + [b for b in (b1, b2) if b is not None]
+        return (all(t.dtype == dt and t.device == keys.device for t in ts) and dk % 64 == 0 and dv % epf == 0
+                and l <= 64 and l % epf == 0 and (2 * dk + dv) // epf <= 256 and W1.shape == (2 * dk, dk + l)
+                and W2.shape == (dk, 2 * dk) and E.shape == (l, l))
+
+    @staticmethod
+    def forward(ctx, keys, values, W1, b1, W2, b2, E, l, d, n_act, n_pad, tm):
+        keys, values, W1, W2, E = (_compact(t) for t in (keys, values, W1, W2, E))
+        b1, b2 = (None if b is None else b.contiguous() for b in (b1, b2))
+        B, T, G, dk = keys.shape if tm else (keys.shape[0], keys.shape[2], keys.shape[1], keys.shape[3])
+        dv, W = values.shape[-1], 2 * dk
+        dev, dt = keys.device, keys.dtype
+        Y = torch.mm(keys.view(-1, dk), W1[:, :dk].t())
+        C = torch.empty(l, W, device=dev, dtype=dt)
+        R = torch.empty(B, G, n_pad, W, device=dev, dtype=dt)
+        K = torch.empty(B, G, n_pad, dk, device=dev, dtype=dt)
+        V = torch.empty(B, G, n_pad, dv, device=dev, dtype=dt)
+        ctx.dims = (B, G, T, dk, dv, l, d, n_act, n_pad, int(tm), _ops._dtype_code(dt))
+        ctx.has_b = (b1 is not None, b2 is not None)
+        a = _CompressTokens._args(ctx.dims, Y, C, values, R, K, V, E, W1, b1, W2, b2)
+        _lib.call("nsa_compress_fwd", ctypes.byref(a), _ops._stream(dev))
+        ctx.save_for_backward(keys, Y, C, R, W1, W2, E)
+        return K, V
+
+    @staticmethod
+    def _args(dims, *tensors):
+        p = [None if t is None else t.data_ptr() for t in tensors]
+        B, G, T, dk, dv, l, d, n_act, n_pad, tm, dt = dims
+        return _lib.CompressArgs(*p, B, G, T, dk, dv, l, d, n_act, n_pad, tm, dt)
+
+    @staticmethod
+    def backward(ctx, dK, dV):
+        keys, Y, C, R, W1, W2, E = ctx.saved_tensors
+        B, G, T, dk, dv, l, d, n_act, n_pad, tm, _ = ctx.dims
+        need = ctx.needs_input_grad
+        dK, dV = _compact(dK), _compact(dV)
+        dR = torch.mm(dK.view(-1, dk), W2)
+        dY = torch.empty_like(Y)
+        dval = torch.empty(*((B, T, G) if tm else (B, G, T)), dv, device=Y.device, dtype=Y.dtype)
+        dW1 = torch.empty_like(W1) if need[2] else None
+        dW2 = torch.empty_like(W2) if need[4] else None
+        dE = torch.empty_like(E) if need[6] else None
+        db1 = W1.new_empty(2 * dk) if ctx.has_b[0] and need[3] else None
+        db2 = W2.new_empty(dk) if ctx.has_b[1] and need[5] else None
+        # (values, K, V_cmp and the biases are forward operands: any aligned address stands in)
+        a = _CompressTokens._args(ctx.dims, Y, C, keys, R, dK, dV, E, W1, None, W2, None)
+        g = _lib.CompressGrads(*[None if t is None else t.data_ptr()
+                                 for t in (keys, dK, dV, dR, dY, dval, dW1, db1, dW2, db2, dE)])
+        ws = torch.empty(_lib.size_of("nsa_compress_bwd_workspace_size", a, ctx.dims), device=Y.device,
+                         dtype=torch.uint8)
+        _lib.call("nsa_compress_bwd", ctypes.byref(a), ctypes.byref(g), _ops._ptr(ws), ws.numel(),
+                  _ops._stream(Y.device))
+        dkeys = torch.mm(dY, W1[:, :dk]).view(keys.shape) if need[0] else None
+        return dkeys, dval if need[1] else None, dW1, db1, dW2, db2, dE, None, None, None, None, None
+
+
 # ============================================================== selection (Eq. 9 / 10)
 GATE_ACT = {"none": 0, "sigmoid": 1, "softmax": 2}  # gate_act codes of nsa_gate_mix_*
 
@@ -808,12 +884,18 @@ class NSAAttention(torch.nn.Module):
             return (torch.zeros(B, G, dk, n_pad, device=dev, dtype=dt), torch.zeros(B, G, n_pad, dv, device=dev, dtype=dt),
                     block_ends, n_act)
         l1, l2 = self.compress_mlp[0], self.compress_mlp[2]
-        W1k, W1p = _SplitCols.apply(l1.weight, dk)
         # keys / values as the module's projections store them ([B,T,G,d], viewed
         # [B,G,T,d]) are used in that order: the GEMM and the pooling then read them
         # without a transposing copy, and their gradients come back in the same layout
         tm = G > 1 and keys.transpose(1, 2).is_contiguous() and values.transpose(1, 2).is_contiguous()
         kin = keys.transpose(1, 2) if tm else keys
+        ws = [None if p is None else p.to(dt)
+              for p in (l1.weight, l1.bias, l2.weight, l2.bias, self.pos_embed.weight)]
+        if _CompressTokens.usable(keys, values, *ws, c.l):
+            Kc, Vc = _CompressTokens.apply(kin, values.transpose(1, 2) if tm else values, *ws, c.l, c.d, n_act, n_pad,
+                                           tm)
+            return Kc.transpose(-1, -2), Vc, block_ends, n_act
+        W1k, W1p = _SplitCols.apply(l1.weight, dk)
         Y = _LinearSplitK.apply(kin, W1k.to(dt), None)                           # [B,G,T,2dk] ([B,T,G,2dk])
         C = F.linear(self.pos_embed.weight.to(dt), W1p.to(dt),
                      l1.bias.to(dt) if l1.bias is not None else None)             # [l,2dk]

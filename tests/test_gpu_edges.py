@@ -180,3 +180,56 @@ def test_compression_work_list(dev, B, G, hpg, T, l, d, dtype, dk, dv):
     be[:n_act] = torch.arange(n_act, dtype=torch.int32) * d + l - 1
     q, kp, v, do = _make(T, B, G * hpg, G, T, n_pad, dk, dv, dtype, dev)
     _check(_ops.COMPRESSION, q, kp, v, do, 1 / math.sqrt(dk), dtype, block_ends=be.to(dev))
+
+
+# compress_tokens as one call each way: one block / a power of two of them / padding, tokens past
+# the last block, one and several batches and groups in either storage order, every width of the
+# weight-gradient tiles, row counts about its 64- (32-) row steps, overlapping and disjoint blocks.
+# Against the same formula in float64: fp32 1e-5 (rounding of the sums).  bf16: 1e-2 for outputs;
+# gradients 6e-2, because a pre-activation within its bf16 rounding (2^-9 of |y| ~ 1) of zero has
+# its unit's gradient switched: about 2^-9 of the units, sqrt(2^-9) = 4.4e-2 of the norm
+@pytest.mark.parametrize("B,G,T,dk,dv,l,d,major", [
+    (1, 1, 8, 64, 8, 8, 8, False), (1, 2, 32, 64, 64, 32, 16, True), (2, 3, 177, 128, 40, 32, 16, True),
+    (2, 2, 95, 192, 128, 32, 32, False), (1, 4, 1056, 192, 128, 32, 16, True), (3, 1, 130, 64, 128, 64, 16, False)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_compress_tokens_edges(dev, B, G, T, dk, dv, l, d, major, dtype):
+    cfg = NSAConfig(d_model=64, head_dim_qk=dk, head_dim_v=dv, n_heads=G, n_kv_groups=G, l=l, d=d, l_prime=64 if 64 % d == 0
+                    else d)
+    torch.manual_seed(T)
+    m = NSAAttention(cfg).to(dev, dtype)
+
+    def rnd(w):
+        x = torch.randn(B, T, G, w, device=dev).to(dtype)
+        return (x.transpose(1, 2) if major else x.transpose(1, 2).contiguous()).detach().requires_grad_()
+
+    k, v = rnd(dk), rnd(dv)
+    kc, vc, be, n = m.compress_tokens(k, v)
+    npad = kc.shape[-1]
+    assert n == (T - l) // d + 1 and npad >= n and (npad & (npad - 1)) == 0
+    assert not kc[..., n:].any() and not vc[:, :, n:].any()
+    gk, gv = torch.randn_like(kc), torch.randn_like(vc)
+    gk[..., n:], gv[:, :, n:] = float("nan"), float("nan")  # the padding's gradients are dropped
+    names = ("compress_mlp.0.weight", "compress_mlp.0.bias", "compress_mlp.2.weight", "compress_mlp.2.bias",
+             "pos_embed.weight")
+    ps = [m.get_parameter(x) for x in names]
+    got = torch.autograd.grad([kc, vc], [k, v, *ps], [gk, gv])
+    W1, b1, W2, b2, E = P = [p.detach().double().requires_grad_() for p in ps]
+    kd, vd = (x.detach().double().requires_grad_() for x in (k, v))
+    y = (kd @ W1[:, :dk].t()).unfold(2, l, d).transpose(-1, -2) + (E @ W1[:, dk:].t() + b1)
+    rk, rv = torch.relu(y).mean(-2) @ W2.t() + b2, vd.unfold(2, l, d).mean(-1)
+    want = torch.autograd.grad([rk, rv], [kd, vd, *P], [gk[..., :n].transpose(-1, -2).double(), gv[:, :, :n].double()])
+
+    def err(a, b):
+        return ((a.double() - b).norm() / b.norm()).item()
+
+    bf = dtype == torch.bfloat16
+    assert max(err(kc[..., :n].transpose(-1, -2), rk), err(vc[:, :, :n], rv)) < (1e-2 if bf else 1e-5)
+    errs = {x: err(a, b) for x, a, b in zip(("k", "v") + names, got, want)}
+    assert max(errs.values()) < (6e-2 if bf else 1e-5), errs
+    # frozen layers: the other gradients are the same
+    for p in ps[2:]:
+        p.requires_grad_(False)
+    kc, vc, _, _ = m.compress_tokens(k, v)
+    part = torch.autograd.grad([kc, vc], [k, v, *ps[:2]], [gk, gv])
+    for a, b in zip(part, got):
+        assert torch.equal(a, b)
