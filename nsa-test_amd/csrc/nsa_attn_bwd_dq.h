@@ -68,7 +68,8 @@ void attn_bwd_dq_kernel(AttnArgs a) {
   const int grp = bg % a.G;
   const int hpg = a.hpg;
   const int ncols = a.Tq * hpg;
-  const int col_base = blockIdx.x * kDqCols;
+  // compression: the late timesteps, which see the most blocks, first
+  const int col_base = (BR == kCompression ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * kDqCols;
   const int t_first = col_base / hpg;
   const int t_last = min(a.Tq - 1, (col_base + kDqCols - 1) / hpg);
   const float scale2 = a.scale * kLog2e;
@@ -403,7 +404,9 @@ __global__ __launch_bounds__(64 * kDqWaves) void attn_bwd_dq_ds_kernel(AttnArgs 
   const int grp = bg % a.G;
   const int hpg = a.hpg;
   const int ncols = a.Tq * hpg;
-  const int col_base = blockIdx.x * kDqCols;
+  // with a compression pass: the late timesteps, which see the most blocks, first
+  const bool late_first = BR == kCompression || a.pair_ds;
+  const int col_base = (late_first ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * kDqCols;
   const int t_first = col_base / hpg;
   const int t_last = min(a.Tq - 1, (col_base + kDqCols - 1) / hpg);
 

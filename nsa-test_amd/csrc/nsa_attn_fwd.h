@@ -79,7 +79,8 @@ __global__ __launch_bounds__(64 * kFwdWaves) void attn_fwd_kernel(AttnArgs a) {
   const int grp = bg % a.G;
   const int hpg = a.hpg;
   const int ncols = a.Tq * hpg;
-  const int col_base = blockIdx.x * kFwdCols;
+  // compression: the late timesteps, which see the most blocks, first
+  const int col_base = (BR == kCompression ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * kFwdCols;
   // positions are absolute (query row r is at a.q0 + r); rows are addressed relatively
   const int t_first = col_base / hpg + a.q0;
   const int t_last = min(a.Tq - 1, (col_base + kFwdCols - 1) / hpg) + a.q0;

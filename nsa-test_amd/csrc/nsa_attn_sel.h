@@ -20,13 +20,15 @@
 namespace nsa {
 
 constexpr int kSelWaveCols = 16;
-// timesteps a wave's 16 columns can touch (column groups start at multiples of 16)
-__host__ __device__ inline int sel_max_t(int hpg) {
-  return hpg % 16 == 0 ? 1 : 16 % hpg == 0 ? 16 / hpg : 15 / hpg + 2;
+// timesteps a wave's columns can touch (column groups start at multiples of cols)
+__host__ __device__ inline int sel_max_t(int hpg, int cols) {
+  return hpg % cols == 0 ? 1 : cols % hpg == 0 ? cols / hpg : (cols - 1) / hpg + 2;
 }
 __host__ __device__ inline int sel_words(int nblk) { return (nblk + 31) / 32; }
 // LDS words of one wave's block bitmaps: the union's, then one per timestep
-__host__ __device__ inline int sel_wave_words(int hpg, int nblk) { return (sel_max_t(hpg) + 1) * sel_words(nblk); }
+__host__ __device__ inline int sel_wave_words(int hpg, int nblk, int cols = kSelWaveCols) {
+  return (sel_max_t(hpg, cols) + 1) * sel_words(nblk);
+}
 
 // Keys per tile.  A tile's K / V fragments and their successors' loads live in registers:
 // 64 keys in bf16; in fp32, at twice the bytes, a 64-key tile spilled (dQ 134 registers at
@@ -43,6 +45,25 @@ __device__ __forceinline__ int xcd_contiguous(int i, int n) {
   const int base = n >> 3, rem = n & 7;
   return (xcd < rem ? xcd * (base + 1) : rem * (base + 1) + (xcd - rem) * base) + k;
 }
+// Logical id of a workgroup of the selection kernels (ids: batch-group major, timesteps
+// ascending).  A timestep's cost grows with the blocks it can select, so with contiguous
+// ranges the XCDs that held the early timesteps finished first, and ascending order left
+// the longest workgroups for the last, partly filled round.  Late timesteps go first, and the
+// XCDs take runs of kXcdRun ids in turn, which keeps neighbouring timesteps on one L2; with
+// whole batch-groups to share out (a multiple of 8) each XCD keeps its own, so that its L2
+// holds one group's K / V.  Forward / dQ in us, before -> after: H64 G4 T2048 dk 192 160 /
+// 163 -> 137 / 140, T8192 634 / 657 -> 613 / 624; B2 H16 G4 T4096 dk 64 118 / 215 -> 106 / 128
+// (runs of 1, 2 and 4 alike; of 16 and 64 up to 10 % slower).
+constexpr int kXcdRun = 4;
+__device__ __forceinline__ int sel_workgroup(int i, int n, int nbg) {
+  if (nbg % 8 == 0) return (i & 7) * (n >> 3) + (n >> 3) - 1 - (i >> 3);
+  const int full = n / (8 * kXcdRun) * (8 * kXcdRun);
+  if (i < full) {
+    const int k = i >> 3;
+    return n - 1 - ((k / kXcdRun * 8 + (i & 7)) * kXcdRun + k % kXcdRun);
+  }
+  return n - 1 - (full + xcd_contiguous(i - full, n - full));
+}
 
 // Per-wave bookkeeping: the timesteps of the wave's columns.
 struct SelWave {
@@ -55,9 +76,9 @@ struct SelWave {
 // the timestep's list took a serial chain of up to nslots LDS reads, and more time than
 // the tile's products (bf16 forward, B3 H16 G4 T1537 dk = dv = 64: 80 -> 61 us).
 __device__ __forceinline__ void sel_wave_setup(const AttnArgs& a, int bg, int f0, uint32_t* bits, uint32_t* tb,
-                                               SelWave& w, int lane) {
+                                               SelWave& w, int lane, int cols = kSelWaveCols) {
   const int ncols = a.Tq * a.hpg;
-  const int flast = min(f0 + kSelWaveCols, ncols) - 1;
+  const int flast = min(f0 + cols, ncols) - 1;
   w.t_first = f0 / a.hpg;
   w.nt = flast / a.hpg - w.t_first + 1;
   const int nwords = sel_words(a.nblk);
@@ -114,7 +135,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform control below
   const int g4 = lane >> 4, c16 = lane & 15;
-  const int L = xcd_contiguous(blockIdx.x, gridDim.x);
+  const int L = sel_workgroup(blockIdx.x, gridDim.x, a.B * a.G);
   const int bg = L / ncoltiles;
   const int b = bg / a.G, grp = bg % a.G;
   const int hpg = a.hpg;
@@ -345,8 +366,254 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   }
 }
 
+// bf16 forward on 32 x 32 x 16 MFMAs: a wave = 32 columns (two timesteps at 16 heads per group,
+// eight at 4, half a timestep at 64), the union of their blocks walked 32 keys at a time, in
+// the same two phases (the common blocks through a double buffer in LDS).  The fragment-native
+// copies serve it as they are: a lane takes the 16-byte piece of its row and slot group from
+// each, 256 contiguous bytes per 16 lanes.  sel_fwd32 says where it runs.
+template <typename T, int DK, int DV>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void attn_sel_fwd32_kernel(AttnArgs a, int ncoltiles) {
+  using S = typename Store<T>::type;
+  constexpr int NK = DK / 16, NV = DV / 32;  // K fragments (16 features), V^T feature tiles
+  constexpr int TKF = 2 * (DK / 32) + DV / 16;  // 1 KB fragments of a 32-key tile: K rowfrags, V^T colfrags
+  // two tiles (phase 1), then per wave the block bitmaps, then the common blocks'
+  extern __shared__ __attribute__((aligned(16))) uint4 sel32_lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hf = lane >> 5, c32 = lane & 31;
+  const int L = sel_workgroup(blockIdx.x, gridDim.x, a.B * a.G);
+  const int bg = L / ncoltiles;
+  const int b = bg / a.G, grp = bg % a.G;
+  const int hpg = a.hpg;
+  const int ncols = a.Tq * hpg;
+  const int f0 = (L % ncoltiles) * 128 + wave * 32;
+  const bool active = f0 < ncols;  // idle waves still meet the phase-1 barriers
+  const float scale2 = a.scale * kLog2e;
+  const int nwords = sel_words(a.nblk);
+  const int wwords = sel_wave_words(hpg, a.nblk, 32);
+  SelWave w{0, 0};
+  uint32_t* maps = reinterpret_cast<uint32_t*>(sel32_lds + 2 * TKF * 64);
+  uint32_t* s_common = maps + 4 * wwords;
+  uint32_t* bits = maps + wave * wwords;
+  uint32_t* tb = bits + nwords;
+  if (active) {
+    sel_wave_setup(a, bg, f0, bits, tb, w, lane, 32);
+  } else {
+    for (int i = lane; i < nwords; i += 64) bits[i] = 0;
+  }
+  __syncthreads();  // every wave's bitmap is written
+  for (int i = threadIdx.x; i < nwords; i += 256)
+    s_common[i] = maps[i] & maps[wwords + i] & maps[2 * wwords + i] & maps[3 * wwords + i];
+  __syncthreads();
+
+  const int f = f0 + c32;
+  const bool colv = active && f < ncols;
+  const int colt = colv ? f / hpg : w.t_first;
+  const int colh = colv ? grp * hpg + f % hpg : grp * hpg;
+  const int tpos = colt + a.q0;  // absolute position
+  const int t_last = w.t_first + w.nt - 1 + a.q0;
+  const uint32_t* mybits = tb + (colt - w.t_first) * nwords;
+  const S* qp = reinterpret_cast<const S*>(a.q) + b * a.sq_b + (int64_t)colh * a.sq_h + (int64_t)colt * a.sq_t;
+  uint4 qf[NK];
+#pragma unroll
+  for (int m = 0; m < NK; ++m)
+    qf[m] = colv ? *reinterpret_cast<const uint4*>(qp + m * 16 + hf * 8) : make_uint4(0, 0, 0, 0);
+
+  // the lane's pieces of the rowfrag K (rows key0 + c32) and colfrag V^T copies
+  const S* krf = reinterpret_cast<const S*>(a.krf) + (int64_t)bg * a.Tp * DK;
+  const S* vcf = reinterpret_cast<const S*>(a.vcf) + (int64_t)bg * DV * a.Tp;
+  const int ko = (c32 >> 4) * (DK * 16) + (hf * 16 + (c32 & 15)) * 8, vo = (c32 >> 4) * 512 + (hf * 16 + (c32 & 15)) * 8;
+  uint4 kf[NK], vf[2][NV];
+  auto load_k = [&](int key0) __attribute__((always_inline)) {
+    const S* p = krf + (int64_t)key0 * DK + ko;
+#pragma unroll
+    for (int m = 0; m < NK; ++m) kf[m] = *reinterpret_cast<const uint4*>(p + m * 256);
+  };
+  auto load_v = [&](int key0) __attribute__((always_inline)) {
+    const S* p = vcf + (int64_t)key0 * DV + vo;
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int j = 0; j < NV; ++j) vf[m][j] = *reinterpret_cast<const uint4*>(p + j * 1024 + m * 256);
+  };
+  f32x16 oacc[NV];
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) oacc[j][i] = 0.f;
+  float m2 = -INFINITY, mtrue = -INFINITY, lsum = 0.f;  // exponent reference, true maximum, sum
+
+  // one tile: S^T from the K fragments, the online softmax (mid() between S^T and it, where
+  // the next K loads go out), O^T += V^T P^T
+  auto tile = [&](int key0, int blk, int blk_hi, auto kfrag, auto vfrag, auto mid) __attribute__((always_inline)) {
+    const int blk_lo = blk * a.lprime;
+    const uint32_t mw = mybits[blk >> 5];
+    // S^T [32 keys][32 columns]: register 4 j + i holds key 8 j + 4 hf + i of column c32
+    f32x16 st;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) st[i] = 0.f;
+#pragma unroll
+    for (int m = 0; m < NK; ++m)
+      st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kfrag(m)),
+                                                   __builtin_bit_cast(bf16x8, qf[m]), st, 0, 0, 0);
+    mid();
+    const bool colsel = colv && ((mw >> (blk & 31)) & 1);
+    const int kend = colsel ? max(blk_lo, a.causal ? min(blk_hi, tpos + 1) : blk_hi) : blk_lo;
+    const uint32_t span = (uint32_t)(kend - blk_lo);
+    const int kb = key0 + 4 * hf - blk_lo;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = (uint32_t)(kb + 8 * j + i) < span ? st[4 * j + i] : -INFINITY;
+        st[4 * j + i] = v;
+        mx = fmaxf(mx, v);
+      }
+    mx = lane_fold<32>(mx, [](float x, float y) { return fmaxf(x, y); }) * scale2;
+    mtrue = fmaxf(mtrue, mx);
+    if (__ballot(mx > m2 + kLazyRescale) != 0ull) {
+      const float mnew = fmaxf(m2, mtrue);
+      const float alpha = m2 == -INFINITY ? 0.f : fast_exp2(m2 - mnew);
+      lsum *= alpha;
+#pragma unroll
+      for (int j = 0; j < NV; ++j) oacc[j] *= alpha;
+      m2 = mnew;
+    }
+    const float nref = m2 == -INFINITY ? 0.f : -m2;
+    float rs = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      st[i] = fast_exp2(mul_add_rounded(st[i], scale2, nref));
+      rs += st[i];
+    }
+    lsum += lane_fold<32>(rs, [](float x, float y) { return x + y; });
+    // P^T as the second operand: slots 4 hf + i and 16 + 4 hf + i (+ 8 for m = 1), the keys one
+    // group of a C-permuted V^T chunk holds
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const uint4 pf = make_uint4(pack_bf16x2(st[4 * m], st[4 * m + 1]), pack_bf16x2(st[4 * m + 2], st[4 * m + 3]),
+                                  pack_bf16x2(st[4 * m + 8], st[4 * m + 9]), pack_bf16x2(st[4 * m + 10], st[4 * m + 11]));
+#pragma unroll
+      for (int j = 0; j < NV; ++j)
+        oacc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vfrag(m, j)),
+                                                          __builtin_bit_cast(bf16x8, pf), oacc[j], 0, 0, 0);
+    }
+  };
+  // cursor over the 32-key tiles of the blocks of a bitmap (uniform)
+  int c_wd, c_blk, c_key0, c_hi;
+  uint32_t c_word;
+  auto start = [&]() {
+    c_wd = c_blk = -1;
+    c_key0 = c_hi = 0;
+    c_word = 0;
+  };
+  auto advance = [&](int t_end, auto word) -> bool {
+    if (c_blk >= 0) {
+      c_key0 += 32;
+      if (c_key0 < c_hi && !(a.causal && c_key0 > t_end)) return true;
+    }
+    while (c_word == 0) {
+      if (++c_wd >= nwords) return false;
+      c_word = __builtin_amdgcn_readfirstlane(word(c_wd));
+    }
+    c_blk = c_wd * 32 + __builtin_ctz(c_word);
+    c_word &= c_word - 1;
+    const int lo = c_blk * a.lprime;
+    c_hi = min(lo + a.lprime, a.Tkv);
+    c_key0 = lo & ~31;
+    return true;
+  };
+
+  // ---- phase 1: the workgroup's common blocks through a double buffer in LDS --------------
+  {
+    const int t_max = (min((L % ncoltiles) * 128 + 128, ncols) - 1) / hpg + a.q0;
+    auto word = [&](int i) { return s_common[i]; };
+    auto copy = [&](int key0, int buf) __attribute__((always_inline)) {
+      for (int fr = wave; fr < TKF; fr += 4) {
+        const S* src = fr < 2 * (DK / 32) ? krf + (int64_t)key0 * DK + fr * 512
+                                          : vcf + (int64_t)key0 * DV + (fr - 2 * (DK / 32)) * 512;
+        copy16_to_lds_async(src + lane * 8, sel32_lds + (buf * TKF + fr) * 64);
+      }
+    };
+    start();
+    bool have = advance(t_max, word);
+    if (have) copy(c_key0, 0);
+    int buf = 0;
+    while (have) {
+      const int key0 = c_key0, blk = c_blk, hi = c_hi;
+      have = advance(t_max, word);
+      wait_vmcnt<0>();  // this wave's copies of the tile have landed
+      __syncthreads();  // every wave's have; the other buffer is no longer read
+      if (have) copy(c_key0, buf ^ 1);
+      if (active) {
+        const S* kt = reinterpret_cast<const S*>(sel32_lds + buf * TKF * 64) + ko;
+        const S* vt = reinterpret_cast<const S*>(sel32_lds + (buf * TKF + 2 * (DK / 32)) * 64) + vo;
+        tile(key0, blk, hi, [&](int m) { return *reinterpret_cast<const uint4*>(kt + m * 256); },
+             [&](int m, int j) { return *reinterpret_cast<const uint4*>(vt + j * 1024 + m * 256); }, [] {});
+      }
+      buf ^= 1;
+    }
+  }
+  if (!active) return;
+
+  // ---- phase 2: the rest of the wave's union, straight from L2 ----------------------------
+  auto word = [&](int i) { return bits[i] & ~s_common[i]; };
+  start();
+  bool have = advance(t_last, word);
+  if (have) {
+    load_k(c_key0);
+    load_v(c_key0);
+  }
+  while (have) {
+    const int key0 = c_key0, blk = c_blk, hi = c_hi;
+    const bool next = advance(t_last, word);
+    tile(key0, blk, hi, [&](int m) { return kf[m]; }, [&](int m, int j) { return vf[m][j]; },
+         [&] { if (next) load_k(c_key0); });
+    if (next) load_v(c_key0);
+    have = next;
+  }
+  if (colv) {
+    const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+    if (lsum > 0.f) lsum *= fast_exp2(m2 - mtrue);  // the sum relative to the true maximum
+    S* op = reinterpret_cast<S*>(a.o) + b * a.so_b + (int64_t)colh * a.so_h + (int64_t)colt * a.so_t;
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        store4<T>(op + j * 32 + 8 * q + 4 * hf, f32x4{oacc[j][4 * q], oacc[j][4 * q + 1], oacc[j][4 * q + 2], oacc[j][4 * q + 3]} * inv);
+    if (hf == 0) {
+      if (a.L)
+        a.L[b * a.sl_b + (int64_t)colh * a.sl_h + (int64_t)colt * a.sl_t] = lsum > 0.f ? logf(lsum) : -INFINITY;
+      if (a.M) a.M[b * a.sm_b + (int64_t)colh * a.sm_h + (int64_t)colt * a.sm_t] = mtrue * kLn2;
+    }
+  }
+}
+
+// Whether the bf16 forward takes 32 columns a wave.  With a multiple of 32 heads the wave is
+// one timestep and reads its blocks once instead of twice (B2 H64 G2 T2000 dk 128: 214 -> 155 us).
+// Otherwise it pays where the timesteps of a wave select mostly the same blocks (few
+// blocks for the slots) and the launch still gives every SIMD two waves: H64 G4 T2048 dk 192
+// 137 -> 129 us, B2 H16 G4 T4096 dk 64 106 -> 98, B3 H16 G4 T1537 58 -> 51; with 8 blocks a slot the
+// union grows (H32 G2 T8192 dk 64 146 -> 153, T32768 dk 128 1150 -> 1218), with fewer waves the
+// latency shows (H8 G2 T4000 dk 64 47 -> 65).
+inline bool sel_fwd32(const AttnArgs& a) {
+  if (a.hpg % 32 == 0) return true;
+  return (int64_t)a.B * a.G * a.Tq * a.hpg >= 2048 * 32 && a.nblk <= 4 * a.nslots;
+}
+
 template <typename T, int DK, int DV>
 void launch_attn_sel_fwd(const AttnArgs& a, hipStream_t s) {
+  if constexpr (sizeof(typename Store<T>::type) == 2) {
+    if (sel_fwd32(a)) {
+      const int nct = (a.Tq * a.hpg + 127) / 128;
+      const size_t lds = (size_t)2048 * (2 * (DK / 32) + DV / 16) + 16 * (size_t)sel_wave_words(a.hpg, a.nblk, 32) +
+                         4 * (size_t)sel_words(a.nblk);
+      allow_dynamic_lds(reinterpret_cast<const void*>(&attn_sel_fwd32_kernel<T, DK, DV>), lds);
+      hipLaunchKernelGGL((attn_sel_fwd32_kernel<T, DK, DV>), dim3(nct * a.B * a.G), dim3(256), lds, s, a, nct);
+      return;
+    }
+  }
   using SH = SelFwdShared<T, DK, DV>;
   const int ncoltiles = (a.Tq * a.hpg + 63) / 64;
   // at most 40 KB of tile + 36 KB of bitmaps (hpg = 1, kSelMaxBlocks): two workgroups per CU
@@ -378,7 +645,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DK <= 64 ? 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform control below
   const int g4 = lane >> 4, c16 = lane & 15;
-  const int L = xcd_contiguous(blockIdx.x, gridDim.x);
+  const int L = sel_workgroup(blockIdx.x, gridDim.x, a.B * a.G);
   const int bg = L / ncoltiles;
   const int b = bg / a.G, grp = bg % a.G;
   const int hpg = a.hpg;
@@ -630,7 +897,7 @@ __global__ __launch_bounds__(256) void attn_sel_dq_ds_kernel(AttnArgs a, int nwa
   const int lane = threadIdx.x & 63;
   const int g4 = lane >> 4, c16 = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int W = xcd_contiguous(blockIdx.x, gridDim.x) * 4 + wave;
+  const int W = sel_workgroup(blockIdx.x, gridDim.x, a.B * a.G) * 4 + wave;
   if (W >= nwaves) return;
   const int nhg = a.hpg >> 4, nsub = a.lprime >> 6;
   const int per_bg = a.Tq * nhg;

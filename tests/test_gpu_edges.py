@@ -233,3 +233,18 @@ def test_compress_tokens_edges(dev, B, G, T, dk, dv, l, d, major, dtype):
     part = torch.autograd.grad([kc, vc], [k, v, *ps[:2]], [gk, gv])
     for a, b in zip(part, got):
         assert torch.equal(a, b)
+
+
+# the 32-column selection forward: one timestep a wave (32 and 64 heads a group; a partly filled
+# last workgroup, a single row), several that share most blocks (from 65536 rows and at most
+# four blocks a slot on: the rule's edges from both sides), timesteps that straddle waves, blocks
+# of half a tile and of one and a half; workgroup orders for whole and partial rounds of XCDs
+@pytest.mark.parametrize("B,G,hpg,T,lp,n,dtype,dk,dv", [
+    (1, 2, 32, 77, 64, 4, torch.bfloat16, 128, 128), (1, 1, 64, 1, 16, 1, torch.bfloat16, 64, 64),
+    (1, 1, 64, 130, 48, 7, torch.bfloat16, 192, 128), (4, 4, 4, 1024, 32, 8, torch.bfloat16, 32, 32),
+    (4, 4, 4, 1025, 32, 8, torch.bfloat16, 32, 32), (4, 4, 4, 1023, 16, 16, torch.bfloat16, 32, 32),
+    (8, 4, 3, 700, 64, 5, torch.bfloat16, 64, 64)])
+def test_selection_forward_32_columns(dev, B, G, hpg, T, lp, n, dtype, dk, dv):
+    q, kp, v, do = _make(hpg + T, B, G * hpg, G, T, T, dk, dv, dtype, dev)
+    idx = _lists(T, B, G, T, n, (T + lp - 1) // lp).to(dev)
+    _check(_ops.SELECTION, q, kp, v, do, 1 / math.sqrt(dk), dtype, indices=idx, lprime=lp)
