@@ -525,6 +525,36 @@ typedef struct nsa_decode_args {
 size_t nsa_decode_workspace_size(const nsa_decode_args* args);
 int nsa_decode_attn(const nsa_decode_args* args, void* workspace, size_t workspace_bytes, nsa_stream_t stream);
 
+/* A whole decode step of the module over plain linear layers, in one call: the token rows x
+ * [Z, d_model] (1 to 64) through the layers w / bias (null: none) 0 q, 1 .. 6 the keys and
+ * values of the three branches, 7 and 8 the gate's, 9 the output projection, weights [out, in]
+ * with unit-stride, 16-byte aligned rows.  phases bit 0: the projections, keys and values stored
+ * as token t of cache[0 .. 5] (compression inputs, selection, window; k then v; strides z, g,
+ * token), and the gate; bit 1: Eq. 8 -> top-n over the n_blocks compressed keys
+ * (k_cmp / v_cmp, unit feature stride, strides z, g, block; block_ends [n_blocks]; n_cmp of
+ * them completed), the attention and mix of nsa_decode_attn, and out [Z, d_model] (row stride
+ * ld_out) through layer 9.  Both phases of a step get the same workspace
+ * (nsa_decode_step_workspace_size bytes, 16-byte aligned), which carries q and the gate. */
+typedef struct nsa_decode_step_args {
+  const void* x;
+  const void* w[10];
+  const void* bias[10];
+  void* cache[6];
+  const void* k_cmp;
+  const void* v_cmp;
+  const int32_t* block_ends;
+  void* out;
+  int64_t ld_x, ld_out;
+  int64_t ldw[10];
+  int64_t stride_cz[6], stride_cg[6], stride_ct[6];
+  int64_t stride_kz, stride_kg, stride_kn, stride_vz, stride_vg, stride_vn;
+  int Z, H, n_kv_groups, d_model, head_dim_qk, head_dim_v, gate_hidden, t, n_cmp, n_blocks;
+  int l, d, l_prime, n, include_fixed, n_fixed, window_size, gate_act, dtype, phases;
+  float sm_scale;
+} nsa_decode_step_args;
+size_t nsa_decode_step_workspace_size(const nsa_decode_step_args* args);
+int nsa_decode_step(const nsa_decode_step_args* args, void* workspace, size_t workspace_bytes, nsa_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -619,6 +619,133 @@ int nsa_decode_attn(const nsa_decode_args* x, void* ws, size_t ws_bytes, nsa_str
   return check_hip("decode attention");
 }
 
+// Offsets of a decode step's workspace: q, gate hidden, gate logits, mixed output, indices,
+// scoring and attention scratch.
+struct StepLayout {
+  size_t q, hid, z, o, idx, score, attn, total, score_bytes, attn_bytes;
+};
+static StepLayout step_layout(const nsa_decode_step_args& x, const nsa_decode_args& at) {
+  StepLayout L{};
+  const size_t es = x.dtype == NSA_F32 ? 4 : 2, Z = x.Z;
+  size_t off = 0;
+  auto take = [&](size_t b) {
+    const size_t o = off;
+    off += align256(b);
+    return o;
+  };
+  L.q = take(Z * x.H * x.head_dim_qk * es);
+  L.hid = take(Z * x.gate_hidden * es);
+  L.z = take(Z * x.H * 3 * es);
+  L.o = take(Z * x.H * x.head_dim_v * es);
+  L.idx = take(Z * x.n_kv_groups * x.n * 8);
+  L.score_bytes = nsa_score_topn_workspace_size(x.Z, x.H, x.n_kv_groups, 1, x.head_dim_qk, x.n_blocks, x.n);
+  L.attn_bytes = nsa_decode_workspace_size(&at);
+  L.score = take(L.score_bytes);
+  L.attn = take(L.attn_bytes);
+  L.total = off;
+  return L;
+}
+
+static nsa_decode_args step_attn(const nsa_decode_step_args& x) {
+  nsa_decode_args a{};
+  a.k[0] = x.k_cmp;
+  a.v[0] = x.v_cmp;
+  a.stride_kz[0] = x.stride_kz;
+  a.stride_kg[0] = x.stride_kg;
+  a.stride_kt[0] = x.stride_kn;
+  a.stride_vz[0] = x.stride_vz;
+  a.stride_vg[0] = x.stride_vg;
+  a.stride_vt[0] = x.stride_vn;
+  for (int br = 1; br < 3; ++br) {
+    a.k[br] = x.cache[2 * br];
+    a.v[br] = x.cache[2 * br + 1];
+    a.stride_kz[br] = x.stride_cz[2 * br];
+    a.stride_kg[br] = x.stride_cg[2 * br];
+    a.stride_kt[br] = x.stride_ct[2 * br];
+    a.stride_vz[br] = x.stride_cz[2 * br + 1];
+    a.stride_vg[br] = x.stride_cg[2 * br + 1];
+    a.stride_vt[br] = x.stride_ct[2 * br + 1];
+  }
+  a.stride_qz = (int64_t)x.H * x.head_dim_qk;
+  a.stride_qh = x.head_dim_qk;
+  a.stride_oz = (int64_t)x.H * x.head_dim_v;
+  a.stride_oh = x.head_dim_v;
+  a.stride_gz = 3 * (int64_t)x.H;
+  a.stride_gh = 3;
+  a.stride_gk = 1;
+  a.Z = x.Z;
+  a.H = x.H;
+  a.n_kv_groups = x.n_kv_groups;
+  a.t = x.t;
+  a.n_cmp = x.n_cmp;
+  a.n_slots = x.n;
+  a.block_size_selection = x.l_prime;
+  a.window_size = x.window_size;
+  a.head_dim_qk = x.head_dim_qk;
+  a.head_dim_v = x.head_dim_v;
+  a.gate_act = x.gate_act;
+  a.dtype = x.dtype;
+  a.sm_scale = x.sm_scale;
+  return a;
+}
+
+size_t nsa_decode_step_workspace_size(const nsa_decode_step_args* x) {
+  if (!x || x->Z <= 0 || x->H <= 0 || x->n_kv_groups <= 0 || x->H % x->n_kv_groups || x->n <= 0 || x->gate_hidden <= 0 ||
+      x->head_dim_qk <= 0 || x->head_dim_v <= 0 || x->n_blocks < 0)
+    return 0;
+  const nsa_decode_args a = step_attn(*x);
+  return step_layout(*x, a).total;
+}
+
+int nsa_decode_step(const nsa_decode_step_args* x, void* ws, size_t ws_bytes, nsa_stream_t stream) {
+  if (!x) return fail(NSA_ERR_INVALID, "args is null");
+  nsa_decode_args a = step_attn(*x);
+  int rc = validate_decode(a);
+  if (rc) return rc;
+  if (x->gate_hidden <= 0 || x->d_model <= 0 || x->n_blocks < x->n_cmp || !(x->phases & 3) || (x->phases & ~3))
+    return fail(NSA_ERR_INVALID, "bad gate_hidden=%d, d_model=%d, n_blocks=%d or phases=%d", x->gate_hidden, x->d_model,
+                x->n_blocks, x->phases);
+  const StepLayout L = step_layout(*x, a);
+  if (!ws || (uintptr_t)ws % 16 || ws_bytes < L.total)
+    return fail(NSA_ERR_WORKSPACE, "workspace of %zu bytes (16-byte aligned) required, %zu given", L.total, ws_bytes);
+  const int H = x->H, G = x->n_kv_groups, dk = x->head_dim_qk, dv = x->head_dim_v, hw = x->gate_hidden;
+  auto job = [&](int i, void* out, int n, int64_t row, int64_t grp, int group, int relu) {
+    return nsa_linear_job{x->w[i], x->bias[i], out, x->ldw[i], row, grp, n, group, relu};
+  };
+  void *q = at<char>(ws, L.q), *hid = at<char>(ws, L.hid), *z = at<char>(ws, L.z), *o = at<char>(ws, L.o);
+  if (x->phases & 1) {
+    const int es = x->dtype == NSA_F32 ? 4 : 2;
+    nsa_linear_job jobs[8];
+    jobs[0] = job(0, q, H * dk, (int64_t)H * dk, 0, H * dk, 0);
+    jobs[1] = job(7, hid, hw, hw, 0, hw, 1);
+    for (int i = 0; i < 6; ++i) {
+      const int w = i & 1 ? dv : dk;
+      if (!x->cache[i]) return fail(NSA_ERR_INVALID, "null cache");
+      jobs[2 + i] = job(1 + i, static_cast<char*>(x->cache[i]) + (int64_t)x->t * x->stride_ct[i] * es, G * w,
+                        x->stride_cz[i], x->stride_cg[i], w, 0);
+    }
+    if ((rc = nsa_linear_few(x->x, x->ld_x, x->Z, x->d_model, jobs, 8, x->dtype, stream))) return rc;
+    const nsa_linear_job gate = job(8, z, 3 * H, 3 * H, 0, 3 * H, 0);
+    if ((rc = nsa_linear_few(hid, hw, x->Z, hw, &gate, 1, x->dtype, stream))) return rc;
+  }
+  if (x->phases & 2) {
+    int64_t* idx = at<int64_t>(ws, L.idx);
+    rc = nsa_score_topn_ex(q, x->k_cmp, x->block_ends, idx, nullptr, nullptr, (int64_t)H * dk, dk, dk, 1, x->stride_kz,
+                           x->stride_kg, 1, x->stride_kn, (int64_t)G * x->n, x->n, x->n, 1, x->Z, H, G, 1, dk,
+                           x->n_blocks, x->l, x->d, x->l_prime, x->n, x->include_fixed, x->n_fixed, x->dtype,
+                           x->sm_scale, x->t, at<char>(ws, L.score), L.score_bytes, stream);
+    if (rc) return rc;
+    a.q = q;
+    a.indices = idx;
+    a.gates = z;
+    a.out = o;
+    if ((rc = nsa_decode_attn(&a, at<char>(ws, L.attn), L.attn_bytes, stream))) return rc;
+    const nsa_linear_job out = job(9, x->out, x->d_model, x->ld_out, 0, x->d_model, 0);
+    if ((rc = nsa_linear_few(o, (int64_t)H * dv, x->Z, H * dv, &out, 1, x->dtype, stream))) return rc;
+  }
+  return NSA_OK;
+}
+
 int nsa_bwd_dkdv_plan(int branch, int Z, int H, int G, int Tq, int Tkv, int nslots, int lprime, int window_size,
                       int* items_per_bg, int* segment) {
   Shape s{branch, NSA_BF16, Z, H, G, Tq, Tkv, 64, 64, nslots, lprime > 0 ? lprime : 64, window_size > 0 ? window_size : 1};

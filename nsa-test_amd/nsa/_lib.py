@@ -83,6 +83,8 @@ SIGNATURES.update({
     "nsa_decode_workspace_size": (_Z, [_P]),
     "nsa_decode_attn": (_I, [_P, _P, _Z, _P]),
     "nsa_linear_few": (_I, [_P, _L, _I, _I, _P, _I, _I, _P]),
+    "nsa_decode_step_workspace_size": (_Z, [_P]),
+    "nsa_decode_step": (_I, [_P, _P, _Z, _P]),
     "nsa_compress_fwd": (_I, [_P, _P]),
     "nsa_compress_bwd_workspace_size": (_Z, [_P]),
     "nsa_compress_bwd": (_I, [_P, _P, _P, _Z, _P]),
@@ -102,6 +104,18 @@ class CompressGrads(ctypes.Structure):
 
     _fields_ = [(n, _P) for n in ("X", "dK", "dV_cmp", "dR", "dY", "dV", "dW1", "db1", "dW2", "db2", "dE")]
 
+
+
+class DecodeStepArgs(ctypes.Structure):
+    """nsa_decode_step_args of include/nsa_hip.h."""
+
+    _fields_ = [("x", _P), ("w", _P * 10), ("bias", _P * 10), ("cache", _P * 6), ("k_cmp", _P), ("v_cmp", _P),
+                ("block_ends", _P), ("out", _P), ("ld_x", _L), ("ld_out", _L), ("ldw", _L * 10),
+                ("stride_cz", _L * 6), ("stride_cg", _L * 6), ("stride_ct", _L * 6),
+                *((n, _L) for n in ("stride_kz", "stride_kg", "stride_kn", "stride_vz", "stride_vg", "stride_vn")),
+                *((n, _I) for n in ("Z", "H", "n_kv_groups", "d_model", "head_dim_qk", "head_dim_v", "gate_hidden", "t",
+                                    "n_cmp", "n_blocks", "l", "d", "l_prime", "n", "include_fixed", "n_fixed",
+                                    "window_size", "gate_act", "dtype", "phases")), ("sm_scale", _F)]
 
 
 class LinearJob(ctypes.Structure):

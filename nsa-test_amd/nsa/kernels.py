@@ -822,9 +822,9 @@ def _plain_linears(x, *layers) -> bool:
         d = m.__dict__
         if type(m) is not torch.nn.Linear or d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d:
             return False
-        w, b = m.weight, m.bias
+        w, b = d["_parameters"].get("weight"), d["_parameters"].get("bias")
         if (type(w) is not torch.nn.Parameter or w.dtype != dt or w.device != dev or w.shape != (n_out, n_in)
-                or not _ops._rows_ok(w)):
+                or not w.is_contiguous() or w.data_ptr() % 16 or n_in * w.element_size() % 16):
             return False
         if b is not None and (type(b) is not torch.nn.Parameter or b.dtype != dt or b.device != dev
                               or b.shape != (n_out,) or not b.is_contiguous()):
@@ -948,6 +948,90 @@ class NSAAttention(torch.nn.Module):
         cache.length = t0 + T
         self._add_blocks(cache)
 
+    def _decode_few(self, x: torch.Tensor, cache: NSAKVCache):
+        """(the projections of the caches in order, the caches, the gate's layers) where the few-row
+        kernels may run the token's layers on x [B,1,D], else None: plain layers (see
+        _plain_linears) over at most 64 rows, caches of x's dtype with unit-stride features, and
+        room for the token."""
+        c, md = self.config, self._modules
+        B, _, D = x.shape
+        H, G, dk, dv = c.n_heads, c.n_kv_groups, c.head_dim_qk, c.head_dim_v
+        gm = md["gate_mlp"]
+        if (B > _ops.LINEAR_FEW_ROWS or cache.length >= cache.max_len or type(gm) is not torch.nn.Sequential
+                or len(gm._modules) != 3 or type(self).prefill is not NSAAttention.prefill
+                or type(self)._project_kv is not NSAAttention._project_kv or dk % 16 or dv % 16):
+            return None
+        g0, act, g2 = gm._modules.values()
+        if (type(g0) is not torch.nn.Linear or type(act) is not torch.nn.ReLU
+                or any(m.__dict__[h] for m in (gm, act) for h in ("_forward_hooks", "_forward_pre_hooks"))):
+            return None
+        hw = g0.out_features
+        projs = (md["k_compress"], md["v_compress"], md["k_select"], md["v_select"], md["k_sliding"], md["v_sliding"])
+        bufs = (cache.k_cmp_in, cache.v_cmp_in, cache.k_sel, cache.v_sel, cache.k_win, cache.v_win)
+        if not _plain_linears(x, (md["q_proj"], D, H * dk), (g0, D, hw), (g2, hw, 3 * H),
+                              *((m, D, G * (dv if i & 1 else dk)) for i, m in enumerate(projs))):
+            return None
+        for i, b in enumerate(bufs):
+            if (type(b) is not torch.Tensor or b.dtype != x.dtype or b.device != x.device
+                    or b.shape != (B, G, cache.max_len, dv if i & 1 else dk) or b.stride(-1) != 1):
+                return None
+        return projs, bufs, (g0, g2)
+
+    def _decode_step(self, x: torch.Tensor, cache: NSAKVCache):
+        """The whole decode step in one library call (nsa_decode_step; two when the token completes
+        a compression block): the output [B,1,D] before dropout, or None where it does not
+        apply (see _decode_few; also plain output projection, compiled head widths, every
+        cache row 16-byte aligned).  A step is bound by the host: projections, scoring,
+        attention and output as calls of their own took 155 us of it, this takes about 75."""
+        c = self.config
+        B, _, D = x.shape
+        H, G, dk, dv, t = c.n_heads, c.n_kv_groups, c.head_dim_qk, c.head_dim_v, cache.length
+        few = self._decode_few(x, cache)
+        kc, vc, be = cache.K_cmp, cache.V_cmp, cache.block_ends
+        o_proj = self._modules["o_proj"]
+        if (few is None or (dk, dv) not in _ops.HEAD_DIM_PAIRS or not 1 <= c.n <= 64 or c.l_prime % 16
+                or not _plain_linears(x, (o_proj, H * dv, D)) or kc.dtype != x.dtype or vc.dtype != x.dtype or kc.device != x.device or vc.device != x.device
+                or be.device != x.device
+                or kc.shape[:3] != (B, G, dk) or vc.shape != (B, G, kc.shape[3], dv) or be.shape != kc.shape[3:]
+                or be.dtype != torch.int32 or not be.is_contiguous()
+                or not all(_ops._rows_ok(b) for b in (_kt(kc), vc, *few[1]))):
+            return None
+        projs, bufs, (g0, g2) = few
+        x2 = _ops._rows(x.reshape(B, D))
+        out = x.new_empty(B, 1, D)
+        n_act = (t + 1 - c.l) // c.d + 1 if t + 1 >= c.l else 0  # blocks once the token is in
+        np_ = _n_pad(max(n_act, 1))
+        a = _lib.DecodeStepArgs()
+        a.x, a.ld_x, a.out, a.ld_out = x2.data_ptr(), x2.stride(0), out.data_ptr(), D
+        ps = [m._parameters for m in (self._modules["q_proj"], *projs, g0, g2, o_proj)]
+        a.w[:] = [p["weight"].data_ptr() for p in ps]
+        a.bias[:] = [None if p["bias"] is None else p["bias"].data_ptr() for p in ps]
+        a.ldw[:] = [D, D, D, D, D, D, D, D, g0.out_features, H * dv]
+        a.cache[:] = [b.data_ptr() for b in bufs]
+        st = [b.stride() for b in bufs]
+        a.stride_cz[:], a.stride_cg[:], a.stride_ct[:] = [s[0] for s in st], [s[1] for s in st], [s[2] for s in st]
+        a.k_cmp, a.v_cmp, a.block_ends = kc.data_ptr(), vc.data_ptr(), be.data_ptr()
+        a.stride_kz, a.stride_kg, _, a.stride_kn = kc.stride()
+        a.stride_vz, a.stride_vg, a.stride_vn = vc.stride()[:3]
+        (a.Z, a.H, a.n_kv_groups, a.d_model, a.head_dim_qk, a.head_dim_v, a.gate_hidden, a.t, a.n_cmp, a.n_blocks, a.l,
+         a.d, a.l_prime, a.n, a.include_fixed, a.n_fixed, a.window_size, a.gate_act, a.dtype, a.sm_scale) = (
+            B, H, G, D, dk, dv, g0.out_features, t, n_act, np_, c.l, c.d, c.l_prime, c.n,
+            int(bool(c.include_fixed_in_selection)), int(c.n_fixed), c.w, GATE_ACT[c.gate_mode],
+            _ops._dtype_code(x.dtype), self.scale)
+        p = ctypes.byref(a)
+        ws = torch.empty(_lib.load().nsa_decode_step_workspace_size(p), device=x.device, dtype=torch.uint8)
+        wp, nb, stream = _ops._ptr(ws), ws.numel(), _ops._stream(x.device)
+        new_block = n_act > cache.n_act
+        if new_block:
+            a.phases = 1
+            _lib.call("nsa_decode_step", p, wp, nb, stream)
+            cache.length = t + 1
+            self._add_blocks(cache)
+        a.phases = 2 if new_block else 3
+        _lib.call("nsa_decode_step", p, wp, nb, stream)
+        cache.length = t + 1
+        return out
+
     def _decode_inputs(self, x: torch.Tensor, cache: NSAKVCache):
         """The token x [B,1,D] joins the cache; returns its queries [B,H,1,dk] and gate logits
         [B,H,1,3].  Plain layers over a few rows run in two launches (every projection of
@@ -955,34 +1039,21 @@ class NSAAttention(torch.nn.Module):
         through the modules."""
         c = self.config
         B, _, D = x.shape
-        H, G, dk, dv, t = c.n_heads, c.n_kv_groups, c.head_dim_qk, c.head_dim_v, cache.length
-        kv = ((self.k_compress, cache.k_cmp_in, dk), (self.v_compress, cache.v_cmp_in, dv),
-              (self.k_select, cache.k_sel, dk), (self.v_select, cache.v_sel, dv),
-              (self.k_sliding, cache.k_win, dk), (self.v_sliding, cache.v_win, dv))
-        gm = self.gate_mlp
-        seq = (type(gm) is torch.nn.Sequential and len(gm) == 3 and type(gm[0]) is torch.nn.Linear
-               and type(gm[1]) is torch.nn.ReLU
-               and not any(m.__dict__[h] for m in (gm, gm[1]) for h in ("_forward_hooks", "_forward_pre_hooks")))
-        g0, g2, hw = (gm[0], gm[2], gm[0].out_features) if seq else (None, None, 0)
-        few = (seq and B <= _ops.LINEAR_FEW_ROWS and t < cache.max_len
-               and D * x.element_size() % 16 == 0 and hw * x.element_size() % 16 == 0
-               and type(self).prefill is NSAAttention.prefill and type(self)._project_kv is NSAAttention._project_kv
-               and _plain_linears(x, (self.q_proj, D, H * dk), (g0, D, hw), (g2, hw, 3 * H),
-                                  *((m, D, G * w) for m, _, w in kv))
-               and all(type(b) is torch.Tensor and b.dtype == x.dtype and b.device == x.device
-                       and b.shape == (B, G, cache.max_len, w) and b.stride(-1) == 1 and w % 16 == 0
-                       for _, b, w in kv))
-        if not few:
+        H, dk, t = c.n_heads, c.head_dim_qk, cache.length
+        few = self._decode_few(x, cache)
+        if few is None:
             self.prefill(x, cache)
             q = self.q_proj(x).view(B, 1, H, dk).transpose(1, 2).contiguous()
-            return q, gm(x).view(B, 1, H, 3).permute(0, 2, 1, 3)
+            return q, self.gate_mlp(x).view(B, 1, H, 3).permute(0, 2, 1, 3)
+        projs, bufs, (g0, g2) = few
+        hw = g0.out_features
         x2 = _ops._rows(x.reshape(B, D))
         q = x.new_empty(B, H, 1, dk)
         hid = x.new_empty(B, hw)
         z = x.new_empty(B, 1, H, 3)
         jobs = [(self.q_proj.weight, self.q_proj.bias, q, H * dk, 0, H * dk, 0),
                 (g0.weight, g0.bias, hid, hw, 0, hw, 1)]
-        for m, b, _ in kv:
+        for m, b in zip(projs, bufs):
             jobs.append((m.weight, m.bias, b[:, :, t], b.stride(0), b.stride(1), b.shape[-1], 0))
         _ops.linear_few(x2, jobs)
         _ops.linear_few(hid, [(g2.weight, g2.bias, z, 3 * H, 0, 3 * H, 0)])
@@ -1004,6 +1075,10 @@ class NSAAttention(torch.nn.Module):
         H, dk, dv = c.n_heads, c.head_dim_qk, c.head_dim_v
         t = cache.length
         x = hidden_states
+        if not output_attentions:
+            out = self._decode_step(x, cache)
+            if out is not None:
+                return self.dropout(out), None  # as forward does
         q, gate_logits = self._decode_inputs(x, cache)
         n_pad = _n_pad(max(cache.n_act, 1)) if cache.n_act > 0 else 1
         kc = cache.K_cmp[..., :n_pad]

@@ -248,3 +248,35 @@ def test_selection_forward_32_columns(dev, B, G, hpg, T, lp, n, dtype, dk, dv):
     q, kp, v, do = _make(hpg + T, B, G * hpg, G, T, T, dk, dv, dtype, dev)
     idx = _lists(T, B, G, T, n, (T + lp - 1) // lp).to(dev)
     _check(_ops.SELECTION, q, kp, v, do, 1 / math.sqrt(dk), dtype, indices=idx, lprime=lp)
+
+
+# the whole decode step in one call against its parts (taken when the attention details are
+# asked for): the same kernels, so the same bits, with blocks completing on the way, before the
+# first block, with every gate mode, with and without fixed blocks, after a prompt and from empty
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,T0,n,gate,fixed,bias", [(1, 0, 4, "sigmoid", True, False), (3, 61, 5, "softmax", False, True),
+                                                    (17, 300, 8, "sigmoid", True, True)])
+def test_decode_step_matches_its_parts(dev, dtype, B, T0, n, gate, fixed, bias):
+    cfg = NSAConfig(d_model=64, head_dim_qk=64, head_dim_v=64, n_heads=8, n_kv_groups=2, l_prime=32, n=n, w=48,
+                    gate_mode=gate, include_fixed_in_selection=fixed, use_bias=bias)
+    torch.manual_seed(B)
+    m = NSAAttention(cfg).to(dev, dtype).eval()
+    T = T0 + 40
+    x = torch.randn(B, T, 64, device=dev).to(dtype)
+    res = []
+    for parts in (False, True):
+        cache = NSAKVCache(cfg, B, T, dev, dtype)
+        if T0:
+            m.prefill(x[:, :T0], cache)
+        if not parts:
+            assert m._decode_step(x[:, T0:T0 + 1], cache) is not None and cache.length == T0 + 1
+            cache.length, cache.n_act = T0, max((T0 - 32) // 16 + 1, 0)
+        outs = [m.decode(x[:, t:t + 1], cache, output_attentions=parts)[0] for t in range(T0, T)]
+        assert cache.length == T and cache.n_act == (T - 32) // 16 + 1
+        res.append((torch.cat(outs, 1), cache.k_cmp_in, cache.v_cmp_in, cache.k_sel, cache.v_sel, cache.k_win,
+                    cache.v_win, cache.K_cmp, cache.V_cmp, cache.block_ends))
+    for i, (a, b) in enumerate(zip(*res)):
+        if i or B <= 16:  # above 16 rows the parts' output projection is torch's
+            assert torch.equal(a, b), i
+        else:
+            assert ((a.double() - b.double()).norm() / b.double().norm()).item() < (2 ** -8 if dtype == torch.bfloat16 else 1e-6)
