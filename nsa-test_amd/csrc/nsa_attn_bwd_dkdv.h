@@ -25,6 +25,13 @@
 // Compression items come from a work list built from the block ends (cmp_plan_kernel): only
 // the rows that see a tile's keys, cut into equal segments over all tiles.
 //
+// Bound by LDS reads (each wave reads the chunk's rows twice, busy 50 % of the cycles) and by
+// their latency at two waves per SIMD: the S and dP products of all row subtiles are therefore
+// one straight run of independent accumulator chains, and the mask stands under one branch on
+// scalar values (with the subtiles one after the other and a branch per masked element:
+// selection, T 8192 H64 G4 dk 192, 1190 -> 1026 us; sliding window 629 -> 565; compression,
+// T 5003 H32 G2 dk 128, 124 -> 113).
+//
 // Every item writes its fp32 dK/dV partial for its keys; a reduce kernel sums the
 // segments of each key tile in a fixed order and accumulates into the caller's dK/dV.
 // Direct mode (sliding window with at least kDkdvDirectItems key tiles over all batches
@@ -150,7 +157,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(DK <= 64 &&
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g4 = lane >> 4;
   const int c16 = lane & 15;
   const int bg = blockIdx.y;
@@ -237,11 +244,26 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(DK <= 64 &&
       wave_be_min = min(wave_be_min, __shfl_xor(wave_be_min, o));
       wave_be_max = max(wave_be_max, __shfl_xor(wave_be_max, o));
     }
+    wave_be_min = __builtin_amdgcn_readfirstlane(wave_be_min);
+    wave_be_max = __builtin_amdgcn_readfirstlane(wave_be_max);
   }
 
   // Wait for the K/V fragments here: otherwise the loop's first use of them becomes a
   // wait inside the loop body, which also stalls on the prefetch of the next chunk.
   __builtin_amdgcn_s_waitcnt(0);
+
+  // the timesteps that see the lane's key: [vis_lo, vis_lo + vis_span), with 0 <= vis_lo, so
+  // the mark -1 of a row past the item's end is never among them
+  int vis_lo;
+  uint32_t vis_span = 0x80000000u;
+  if (BR == kSliding) {
+    vis_lo = mykey;
+    vis_span = mykey < a.Tkv ? max(a.window, 0) : 0;
+  } else if (BR == kCompression) {
+    vis_lo = max(mybe, 0);
+  } else {
+    vis_lo = mykey < blk_hi ? (a.causal ? mykey : 0) : 0x7fffffff;
+  }
 
   f32x4 dka[DK / 16], dva[DV / 16];
 #pragma unroll
@@ -435,8 +457,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(DK <= 64 &&
 
     // rows are in ascending t, so the chunk spans [t_min, t_max]
     const bool full = fc + RC <= f_hi;
-    const int t_min = row_t(min(fc, f_hi - 1));
-    const int t_max = row_t(min(fc + RC, f_hi) - 1);
+    const int t_min = __builtin_amdgcn_readfirstlane(row_t(min(fc, f_hi - 1)));
+    const int t_max = __builtin_amdgcn_readfirstlane(row_t(min(fc + RC, f_hi) - 1));
     bool active, all_visible;
     if (BR == kSliding) {
       active = kw0 <= t_max && kw0 + 15 > t_min - a.window;
@@ -449,52 +471,62 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(DK <= 64 &&
       all_visible = full && (!a.causal || kw0 + 15 <= t_min) && kw0 + 15 < blk_hi;
     }
 
-    // Waves whose keys no row of the chunk can see still run the (fully masked) products:
-    // a branch around them makes the compiler shuttle the dK/dV accumulators between
-    // register files on every chunk, which costs more than the skipped work.
-    (void)active;
-    {
-      f32x4 pt[RC / 16], dst[RC / 16];
+    // Sliding window: a wave whose keys no row of the chunk sees (one chunk in six at window
+    // 512) leaves the machine to the others (T 8192 H64 G4 dk 192: 589 -> 565 us).  The other
+    // branches meet such chunks at the diagonal only and run their fully masked products: the
+    // branch costs them registers (compression spills at dk 192, 336 -> 661 us; selection
+    // 1026 -> 1064 us).
+    if (BR != kSliding || active) {
+      f32x4 pt[RC / 16], dst[RC / 16];  // S, then P; dP, then dS
 #pragma unroll
       for (int rs = 0; rs < RC / 16; ++rs) {
-        f32x4 sacc = zero4(), pacc = zero4();
-        const S* qrow = &Qs[buf][(rs * 16 + c16) * QP];
-        const S* orow = &Os[buf][(rs * 16 + c16) * OP];
+        pt[rs] = zero4();
+        dst[rs] = zero4();
+      }
 #pragma unroll
-        for (int kc = 0; kc < NKC; ++kc) sacc = Mma<T>::run(sacc, frag_std<T>(qrow + kc * KC, g4), kf[kc]);
+      for (int kc = 0; kc < NKC; ++kc)
 #pragma unroll
-        for (int kc = 0; kc < NVC; ++kc) pacc = Mma<T>::run(pacc, frag_std<T>(orow + kc * KC, g4), vf[kc]);
-        // the lane's four rows rs*16 + 4*g4 + i: their statistics as one 16-byte read each,
-        // the mask applied to the exponent argument (no divergent branch)
-        const int r4 = rs * 16 + 4 * g4;
-        const float4 l2v = *reinterpret_cast<const float4*>(&s_l2[buf][r4]);
-        const float4 dlv = *reinterpret_cast<const float4*>(&s_dl[buf][r4]);
-        const float4 gv = *reinterpret_cast<const float4*>(&s_g[buf][r4]);
-        const int4 tv = *reinterpret_cast<const int4*>(&s_t[buf][r4]);
-        const float l2a[4] = {l2v.x, l2v.y, l2v.z, l2v.w}, dla[4] = {dlv.x, dlv.y, dlv.z, dlv.w};
+        for (int rs = 0; rs < RC / 16; ++rs)
+          pt[rs] = Mma<T>::run(pt[rs], frag_std<T>(&Qs[buf][(rs * 16 + c16) * QP + kc * KC], g4), kf[kc]);
+#pragma unroll
+      for (int kc = 0; kc < NVC; ++kc)
+#pragma unroll
+        for (int rs = 0; rs < RC / 16; ++rs)
+          dst[rs] = Mma<T>::run(dst[rs], frag_std<T>(&Os[buf][(rs * 16 + c16) * OP + kc * KC], g4), vf[kc]);
+      // the lane's four rows rs*16 + 4*g4 + i: their statistics as one 16-byte read each
+#pragma unroll
+      for (int rs = 0; rs < RC / 16; ++rs) {
+        const float4 l2v = *reinterpret_cast<const float4*>(&s_l2[buf][rs * 16 + 4 * g4]);
+        const float l2a[4] = {l2v.x, l2v.y, l2v.z, l2v.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pt[rs][i] = pt[rs][i] * scale2 - l2a[i];
+      }
+      // the mask, on the exponent arguments, under one branch on scalar values: chunks whose
+      // rows all see the wave's keys skip it
+      if (!all_visible) {
+#pragma unroll
+        for (int rs = 0; rs < RC / 16; ++rs) {
+          const int4 tv = *reinterpret_cast<const int4*>(&s_t[buf][rs * 16 + 4 * g4]);
+          const int ta[4] = {tv.x, tv.y, tv.z, tv.w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const bool vis = (uint32_t)(ta[i] - vis_lo) < vis_span;
+            pt[rs][i] = vis ? pt[rs][i] : -INFINITY;
+          }
+        }
+      }
+#pragma unroll
+      for (int rs = 0; rs < RC / 16; ++rs) {
+        const float4 dlv = *reinterpret_cast<const float4*>(&s_dl[buf][rs * 16 + 4 * g4]);
+        const float4 gv = *reinterpret_cast<const float4*>(&s_g[buf][rs * 16 + 4 * g4]);
+        const float dla[4] = {dlv.x, dlv.y, dlv.z, dlv.w};
         const float ga[4] = {gv.x, gv.y, gv.z, gv.w};
-        const int ta[4] = {tv.x, tv.y, tv.z, tv.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          // masked elements: the argument clamped to -inf by a min with a selected
-          // constant, the conditions combined with bitwise operators (a select of the
-          // argument itself, or short-circuit ands, become divergent branches in the
-          // loop); chunks whose rows all see the wave's keys skip the mask (uniform)
-          // (compression keeps the select: measured faster there)
-          float arg = sacc[i] * scale2 - l2a[i];
-          if (BR == kCompression) {
-            arg = (all_visible || (ta[i] >= 0 && mybe <= ta[i])) ? arg : -INFINITY;
-          } else if (!all_visible) {
-            const int t = ta[i];
-            bool vis;
-            if (BR == kSliding) vis = (t >= 0) & (mykey <= t) & (mykey > t - a.window) & (mykey < a.Tkv);
-            else vis = (t >= 0) & ((a.causal == 0) | (mykey <= t)) & (mykey < blk_hi);
-            arg = fminf(arg, vis ? INFINITY : -INFINITY);
-          }
           // lse2 is +inf for rows that saw no key: p = 0 there
-          const float p = fast_exp2(arg) * ga[i];  // gated: g dO
+          const float p = fast_exp2(pt[rs][i]) * ga[i];  // gated: g dO
           pt[rs][i] = p;
-          dst[rs][i] = p * (pacc[i] - dla[i]);
+          dst[rs][i] = p * (dst[rs][i] - dla[i]);
         }
         if constexpr (kStoreDs) {  // the lane's four heads of its key, into the chunk's tile
           if (a.ds)
@@ -527,6 +559,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(DK <= 64 &&
           dka[j] = Mma<T>::run(dka[j], frag_cperm<T>(&QTs[buf][(j * 16 + c16) * RP + kc2 * CK], g4), sf);
         }
       }
+    } else if constexpr (kStoreDs) {  // no row of the chunk sees the wave's keys: its dS is zero
+      if (a.ds)
+#pragma unroll
+        for (int rs = 0; rs < RC / 16; ++rs)
+          *reinterpret_cast<uint2*>(&s_dst[c & 1][rs][(wave * 16 + c16) * 16 + 4 * g4]) = make_uint2(0, 0);
     }
   };
   if constexpr (kDepth == 2) {
