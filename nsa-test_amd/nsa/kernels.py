@@ -750,7 +750,8 @@ def score_and_select(q: torch.Tensor, k_compressed: torch.Tensor, block_ends: to
     cdt = _ops.compute_dtype(q.dtype)
     qc = q.to(cdt)
     # the kernel reads each compressed key as one row (unit-stride features)
-    kc = _ops._rows(_kt(k_compressed.to(cdt))).transpose(-1, -2)
+    kt = _kt(k_compressed.to(cdt))
+    kc = (kt if kt.is_contiguous() else _ops._rows(kt)).transpose(-1, -2)
     be = block_ends.to(torch.int32).contiguous()
     s = config.l_prime // config.d
     nsel = (N + s - 1) // s
