@@ -23,8 +23,8 @@ constexpr int kRowChunk = 32;
 // Compression dQ from the stored dS keeps the block end of every 32-key chunk's first key
 // in LDS; the host stores dS for compression only up to this many chunks (65536 blocks).
 constexpr int kDqCbeMax = 2048;
-// Query entries (timesteps; selection: CSR entries) per dK/dV work item: 128 or 256,
-// chosen per launch (dkdv_seg_len), at most kSegTMax.
+// Query entries (timesteps; selection: CSR entries) per dK/dV work item: 32 to 256,
+// chosen per launch, at most kSegTMax.
 constexpr int kSegTMax = 256;
 // dK/dV key tiles (all batches and groups) from which the sliding-window backward gives
 // each tile all its query rows in one work item (one item per CU or more)

@@ -6,8 +6,8 @@
 // group K/V (kt [T][dk], kn [dk][T], vt [dv][T], vn [T][dv]) into MFMA operand
 // registers -- no LDS staging and no workgroup barrier -- so a wave never waits for
 // blocks another wave's timesteps chose, and blocks shared by neighbouring timesteps
-// (the fixed initial / local blocks, correlated top-n) are served by L2.  Workgroups
-// are mapped XCD-contiguously so that neighbouring timesteps share an L2.
+// (the fixed initial / local blocks, correlated top-n) are served by L2.  Workgroups run
+// the late timesteps first and are dealt to the XCDs in short runs (sel_workgroup).
 //
 // Key j is visible to column (t, h) iff j lies in a block the row selected (the
 // cleaned, de-duplicated list), j < N_CTX_KV and (causal) j <= t

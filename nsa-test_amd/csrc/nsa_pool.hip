@@ -8,8 +8,9 @@
 // C = E W1p^T + b1 (l x 2dk).  W2 and the mean commute, so
 //            K_cmp[i] = W2 R[i] + b2,   R[i] = mean_u relu(Y[d*i+u] + C[u]),
 // a GEMM over the n_cmp pooled rows.  The GEMMs and their input gradients stay in torch
-// (hipBLASLt), the weight gradients are nsa_wgrad (nsa_wgrad.hip); this file holds the
-// HBM-bound middle: R and V_cmp (forward) and dY, dC, dV (backward).
+// (hipBLASLt), the weight gradients are those of nsa_wgrad.hip; this file holds the
+// HBM-bound middle, R and V_cmp (forward) and dY, dC, dV (backward), and the calls that run
+// everything but the GEMMs of one direction (nsa_compress_fwd, nsa_compress_bwd).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
