@@ -28,9 +28,10 @@
 // Bound by LDS reads (each wave reads the chunk's rows twice, busy 50 % of the cycles) and by
 // their latency at two waves per SIMD: the S and dP products of all row subtiles are therefore
 // one straight run of independent accumulator chains, and the mask stands under one branch on
-// scalar values (with the subtiles one after the other and a branch per masked element:
-// selection, T 8192 H64 G4 dk 192, 1190 -> 1026 us; sliding window 629 -> 565; compression,
-// T 5003 H32 G2 dk 128, 124 -> 113).
+// scalar values (with the subtiles one after the other and a branch per masked element, T 8192
+// H64 G4 dk 192: sliding window 630 -> 547 us; compression, T 5003 H32 G2 dk 128, 124 -> 113-120;
+// selection 1061 -> 1023 alone, 1.2 ms either way within a long run: it takes 6.2 GB through
+// the memory side).
 //
 // Every item writes its fp32 dK/dV partial for its keys; a reduce kernel sums the
 // segments of each key tile in a fixed order and accumulates into the caller's dK/dV.
