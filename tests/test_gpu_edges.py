@@ -182,6 +182,21 @@ def test_compression_work_list(dev, B, G, hpg, T, l, d, dtype, dk, dv):
     _check(_ops.COMPRESSION, q, kp, v, do, 1 / math.sqrt(dk), dtype, block_ends=be.to(dev))
 
 
+# sliding-window dK/dV: a wave whose 16 keys no row of a chunk sees skips it.  Windows below, at
+# and past a wave's keys and a row chunk, shorter and longer than the sequence; chunks of less
+# than a timestep to 32 of them; with and without stored dS; one item per key tile (256 tiles).
+# (Window 2 is the smallest: at 1 the probability is 1 and the exact dQ and dK are zero, so a
+# relative error has no meaning.)
+@pytest.mark.parametrize("B,G,hpg,T,w,dtype,dk,dv", [
+    (1, 1, 16, 700, 2, torch.bfloat16, 64, 64), (1, 2, 16, 403, 17, torch.bfloat16, 192, 128),
+    (2, 1, 16, 257, 600, torch.bfloat16, 128, 128), (1, 1, 1, 1500, 128, torch.bfloat16, 64, 64),
+    (1, 2, 40, 150, 33, torch.bfloat16, 128, 128), (2, 128, 1, 100, 16, torch.bfloat16, 32, 32),
+    (1, 1, 4, 391, 48, torch.float32, 64, 64), (1, 1, 3, 200, 2, torch.float32, 32, 32)])
+def test_sliding_chunks_out_of_sight(dev, B, G, hpg, T, w, dtype, dk, dv):
+    q, k, v, do = _make(T + w, B, G * hpg, G, T, T, dk, dv, dtype, dev)
+    _check(_ops.SLIDING, q, k, v, do, 1 / math.sqrt(dk), dtype, window=w)
+
+
 # compress_tokens as one call each way: one block / a power of two of them / padding, tokens past
 # the last block, one and several batches and groups in either storage order, every width of the
 # weight-gradient tiles, row counts about its 64- (32-) row steps, overlapping and disjoint blocks.
