@@ -16,6 +16,7 @@
 #include "nsa_attn.h"
 #include "nsa_device.h"
 #include "nsa_attn_rowstats.h"
+#include "nsa_order.h"
 
 namespace nsa {
 
@@ -37,33 +38,6 @@ __host__ __device__ inline int sel_wave_words(int hpg, int nblk, int cols = kSel
 // -> 561 us, now two waves per SIMD instead of one; forward 437 -> 424 us at four).
 template <typename T>
 constexpr int kSelTile = sizeof(typename Store<T>::type) == 2 ? 64 : 32;
-
-// Workgroup id -> logical id such that each XCD (ids dispatched round-robin over 8)
-// receives a contiguous range of logical ids.
-__device__ __forceinline__ int xcd_contiguous(int i, int n) {
-  const int xcd = i & 7, k = i >> 3;
-  const int base = n >> 3, rem = n & 7;
-  return (xcd < rem ? xcd * (base + 1) : rem * (base + 1) + (xcd - rem) * base) + k;
-}
-// Logical id of a workgroup of the selection kernels (ids: batch-group major, timesteps
-// ascending).  A timestep's cost grows with the blocks it can select, so with contiguous
-// ranges the XCDs that held the early timesteps finished first, and ascending order left
-// the longest workgroups for the last, partly filled round.  Late timesteps go first, and the
-// XCDs take runs of kXcdRun ids in turn, which keeps neighbouring timesteps on one L2; with
-// whole batch-groups to share out (a multiple of 8) each XCD keeps its own, so that its L2
-// holds one group's K / V.  Forward / dQ in us, before -> after: H64 G4 T2048 dk 192 160 /
-// 163 -> 137 / 140, T8192 634 / 657 -> 613 / 624; B2 H16 G4 T4096 dk 64 118 / 215 -> 106 / 128
-// (runs of 1, 2 and 4 alike; of 16 and 64 up to 10 % slower).
-constexpr int kXcdRun = 4;
-__device__ __forceinline__ int sel_workgroup(int i, int n, int nbg) {
-  if (nbg % 8 == 0) return (i & 7) * (n >> 3) + (n >> 3) - 1 - (i >> 3);
-  const int full = n / (8 * kXcdRun) * (8 * kXcdRun);
-  if (i < full) {
-    const int k = i >> 3;
-    return n - 1 - ((k / kXcdRun * 8 + (i & 7)) * kXcdRun + k % kXcdRun);
-  }
-  return n - 1 - (full + xcd_contiguous(i - full, n - full));
-}
 
 // Per-wave bookkeeping: the timesteps of the wave's columns.
 struct SelWave {

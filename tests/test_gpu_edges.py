@@ -253,7 +253,8 @@ def test_compress_tokens_edges(dev, B, G, T, dk, dv, l, d, major, dtype):
 # the 32-column selection forward: one timestep a wave (32 and 64 heads a group; a partly filled
 # last workgroup, five rows: a lone key has an exact dQ of zero, so no relative error), several that share most blocks (from 65536 rows and at most
 # four blocks a slot on: the rule's edges from both sides), timesteps that straddle waves, blocks
-# of half a tile and of one and a half; workgroup orders for whole and partial rounds of XCDs
+# of half a tile and of one and a half; the forward's workgroup orders for whole and partial rounds
+# of XCDs (the stored-dS dQ's: test_selection_dq_workgroup_order)
 @pytest.mark.parametrize("B,G,hpg,T,lp,n,dtype,dk,dv", [
     (1, 2, 32, 77, 64, 4, torch.bfloat16, 128, 128), (1, 1, 64, 5, 16, 1, torch.bfloat16, 64, 64),
     (1, 1, 64, 130, 48, 7, torch.bfloat16, 192, 128), (4, 4, 4, 1024, 32, 8, torch.bfloat16, 32, 32),
@@ -263,6 +264,26 @@ def test_selection_forward_32_columns(dev, B, G, hpg, T, lp, n, dtype, dk, dv):
     q, kp, v, do = _make(hpg + T, B, G * hpg, G, T, T, dk, dv, dtype, dev)
     idx = _lists(T, B, G, T, n, (T + lp - 1) // lp).to(dev)
     _check(_ops.SELECTION, q, kp, v, do, 1 / math.sqrt(dk), dtype, indices=idx, lprime=lp)
+
+
+# the dQ kernel of the stored dS (16 and 32 heads a group, blocks of 64 keys) has ceil(waves / 4)
+# workgroups: a multiple of neither 8 nor the batch-groups when T % 4 is 1, 2 or 3, with 8 and 16
+# batch-groups, which the XCDs share out whole, and 6, which they do not.  Added to a given dQ the
+# result is the overwritten one plus it: both rounded to bf16 once, 2^-8 of the sum
+@pytest.mark.parametrize("B,G,hpg,T", [(2, 4, 16, 301), (8, 1, 16, 202), (4, 4, 16, 129), (1, 8, 32, 67),
+                                       (4, 2, 16, 5), (3, 2, 16, 131), (2, 8, 16, 100)])
+def test_selection_dq_workgroup_order(dev, B, G, hpg, T):
+    lp, n, dk, dt = 64, 4, 64, torch.bfloat16
+    q, kp, v, do = _make(hpg + T, B, G * hpg, G, T, T, dk, dk, dt, dev)
+    idx = _lists(T, B, G, T, n, (T + lp - 1) // lp).to(dev)
+    out, (dq, _, _) = _check(_ops.SELECTION, q, kp, v, do, 1 / math.sqrt(dk), dt, indices=idx, lprime=lp)
+    k = kp.transpose(-1, -2)
+    _, L, M = _ops.attn_fwd(_ops.SELECTION, q, k, v, 1 / math.sqrt(dk), indices=idx, lprime=lp)
+    base = torch.randn_like(q)
+    acc, _, _ = _ops.attn_bwd(_ops.SELECTION, q, k, v, out, do, L, M, 1 / math.sqrt(dk), indices=idx, lprime=lp,
+                              dq=base.clone(), dq_accumulate=True)
+    want = base.double() + dq.double()
+    assert ((acc.double() - want).abs() <= 2 ** -8 * (want.abs() + dq.double().abs()) + 1e-6).all()
 
 
 # the whole decode step in one call against its parts (taken when the attention details are

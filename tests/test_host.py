@@ -1,7 +1,9 @@
 """CPU tests of the host side: configuration semantics, the torch selection helpers,
 the C ABI library (loads, exports every declared symbol) and the launch surface's
 argument handling.  No GPU computation happens here."""
+import ctypes
 import re
+import subprocess
 from pathlib import Path
 
 import numpy as np
@@ -282,3 +284,35 @@ def test_compression_stored_ds_block_limit():
     stored = _lib.size("nsa_bwd_workspace_size", *args(65536, _lib.NSA_BF16))
     recomputed = _lib.size("nsa_bwd_workspace_size", *args(65537, _lib.NSA_BF16))
     assert stored - recomputed >= ds - 2 * 1024 * 1024  # one more block changes the rest little
+
+
+# ------------------------------------------------------------------ workgroup orders
+def test_workgroup_orders_are_permutations(tmp_path):
+    """Every workgroup order hands out each of its n ids exactly once, for grids of any size and
+    any number of batch-groups (g++ on the header the kernels include)."""
+    (tmp_path / "order.cpp").write_text("""
+        #define __host__
+        #define __device__
+        #define __forceinline__ inline
+        #include <vector>
+        #include "nsa_order.h"
+        static int bad(int n, int nbg) {
+          std::vector<char> a(n), b(n);
+          for (int i = 0; i < n; ++i) {
+            const int x = nsa::sel_workgroup(i, n, nbg), y = nsa::xcd_contiguous(i, n);
+            if (x < 0 || x >= n || a[x]++ || y < 0 || y >= n || b[y]++) return 1;
+          }
+          return 0;
+        }
+        extern "C" int first_bad(int n_max, int nbg) {
+          for (int n = 1; n <= n_max; ++n)
+            if (bad(n, nbg)) return n;
+          return bad(100003, nbg) ? 100003 : 0;
+        }
+    """)
+    so = tmp_path / "order.so"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-I", str(ROOT / "nsa-test_amd" / "csrc"),
+                    str(tmp_path / "order.cpp"), "-o", str(so)], check=True)
+    fn = ctypes.CDLL(str(so)).first_bad
+    for nbg in (*range(1, 17), 24, 32, 64):
+        assert fn(4096, nbg) == 0, nbg
