@@ -236,7 +236,8 @@ __global__ void decode_mix_kernel(DecodeArgs a, int nheadtiles) {
       l += w * p[i * np + 16 + c];
       o += w * p[i * np + 32 + c * dv + f];
     }
-    out += gate[br] * (l > 0.f ? o / l : 0.f);  // no visible key: 0
+    // no visible key: 0 (the sum is exactly 0); a NaN sum is one of a visible key and stays
+    out += gate[br] * (l == 0.f ? 0.f : o / l);
     p += a.nwg[br] * np;
   }
   reinterpret_cast<S*>(a.out)[b * a.so_b + (int64_t)h * a.so_h + f] = Elem<T>::from_f32(out);

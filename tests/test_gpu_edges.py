@@ -108,6 +108,33 @@ def test_decode_attention_edges(dev, B, G, hpg, t, n_cmp, dk, dv, lp, n, w, act,
     assert err < (2e-2 if dtype == torch.bfloat16 else 1e-5), err
 
 
+# a NaN or an infinite score within the visible keys of each branch in turn reaches the output of
+# every head that sees it, and no other (with an infinite key: the heads whose query makes it
+# +inf, as exp(inf - inf); the others give that key the weight 0)
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("br", [0, 1, 2])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_decode_attention_keeps_nan(dev, br, bad, dtype):
+    B, G, hpg, t, n_cmp, d, lp, n, w = 2, 2, 4, 300, 17, 64, 16, 5, 100
+    g = torch.Generator().manual_seed(br)
+
+    def rnd(*s):
+        return torch.randn(*s, generator=g).to(dtype).to(dev)
+
+    q, gates = rnd(B, G * hpg, 1, d), rnd(B, G * hpg, 1, 3)
+    kv = [rnd(B, G, n_cmp if i < 2 else t + 1, d) for i in range(6)]
+    idx = torch.tensor([0, 3, 7, 12, 18]).expand(B, G, 1, n).contiguous().to(dev)
+    args = (n_cmp, idx, gates, 1, t, 0.1, lp, w)
+    clean = _ops.decode_attn(q, kv, *args)
+    kv[2 * br][1, 0, (5, 7 * lp + 3, t - 50)[br], 11] = bad
+    out = _ops.decode_attn(q, kv, *args)
+    hit = torch.zeros(B, G, hpg, dtype=torch.bool, device=dev)
+    hit[1, 0] = True if math.isnan(bad) else q[1, :hpg, 0, 11] > 0
+    hit = hit.view(B, G * hpg, 1)
+    assert hit.any() and torch.equal(out.isnan(), hit.unsqueeze(-1).expand_as(out))
+    assert torch.equal(out[:, hpg:], clean[:, hpg:]) and torch.equal(out[0], clean[0])
+
+
 # few-row linear layers: rows at the 16-row tiles, widths at the 16-feature tiles, inputs at the
 # 32- (16-) feature chunks, the eight waves' turns and a last chunk of one piece; several jobs,
 # grouped outputs, bias, relu.  fp32 sums: 1e-6 norm-relative; bf16 rounding of the result 2^-9
