@@ -570,6 +570,17 @@ __global__ __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu
     else
       win = __builtin_amdgcn_readfirstlane(
           wave_butterfly(bv == mx ? bi : 0x7fffffff, [](int x, int y) { return min(x, y); }));
+    if constexpr (FAST9) {
+      // no lane has an output left (only NaN sums remain, from a query or key with one): the
+      // lowest entry at -inf, taken before or past nsel, which no attention kernel selects twice
+      if (win == 0x7fffffff) {
+        int lo = 0x7fffffff;
+#pragma unroll
+        for (int s = NQ - 1; s >= 0; --s)
+          if (agg[s] == -INFINITY) lo = 64 * s + lane;
+        win = __builtin_amdgcn_readfirstlane(wave_butterfly(lo, [](int x, int y) { return min(x, y); }));
+      }
+    }
     if (lane == (win & 63)) {  // its owner marks it taken
       if constexpr (FAST9) {
 #pragma unroll

@@ -60,6 +60,25 @@ def test_score_few_rows(dev, B, G, hpg, T, N, dk, l, lp, dtype):
         np.testing.assert_array_equal(a.cpu().numpy(), b)
 
 
+# a query row with a NaN: its group's sums are NaN at every block, and what is left to take is the
+# first entry past the last block (here 100 of 100), never an index that no block can have; the
+# rows beside it are untouched.  A wave per timestep and a timestep's heads across waves
+@pytest.mark.parametrize("T", [4, 1500])
+@pytest.mark.parametrize("fixed", [False, True])
+def test_score_nan_row(dev, T, fixed):
+    cfg = NSAConfig(head_dim_qk=64, n_heads=4, n_kv_groups=1, n=9, include_fixed_in_selection=fixed)
+    N, q0 = 400, 16 * 379 + 31  # l' = 4 d: 100 blocks, the own one of row 0 is 95
+    g = torch.Generator().manual_seed(0)
+    q = torch.randn(1, 4, T, 64, generator=g).to(dev)
+    k = torch.randn(1, 1, 64, N, generator=g).to(dev)
+    be = torch.arange(N, dtype=torch.int32, device=dev) * 16 + 31
+    clean = score_and_select(q, k, be, 0.2, cfg, q_offset=q0)
+    q[:, 1, 0] = float("nan")
+    got = score_and_select(q, k, be, 0.2, cfg, q_offset=q0)
+    assert got[0, 0, 0].tolist() == ([0, 94, 95] + 6 * [100] if fixed else 9 * [100])
+    assert torch.equal(got[:, :, 1:], clean[:, :, 1:])
+
+
 # the decode step's split over 256-key workgroups and 64-key waves: positions at their edges and
 # at block edges, no compressed token / one / 256 / 257, 1 / 4 / 16 / 17 / 40 heads a group (head
 # tiles), every compiled width, windows of one key and past the sequence, empty slots, caches of
