@@ -501,9 +501,9 @@ int nsa_linear_few(const void* x, int64_t ld_x, int rows, int k, const nsa_linea
  * and the mix in fp32, rounded to dtype once.  The keys and values are read where they lie
  * (unit feature stride, 16-byte aligned rows, strides (z, g, token) in elements):
  *   branch 0  the n_cmp compressed tokens completed so far (all visible)
- *   branch 1  the distinct blocks indices[z,g,0..n_slots-1] (contiguous int64, negative =
- *             none; later blocks are masked) of block_size_selection keys, a multiple of 16;
- *             a row without any block takes block t / block_size_selection
+ *   branch 1  the blocks indices[z,g,0..n_slots-1] (contiguous int64, negative = none, a
+ *             repeat counts once; later blocks are masked) of block_size_selection keys, a
+ *             multiple of 16; a row without any block takes block t / block_size_selection
  *   branch 2  the last window_size positions
  * q [Z,H,dk] and out [Z,H,dv] have unit feature stride and 16-byte aligned rows; gates [Z,H,3]
  * in dtype; gate_act as in nsa_gate_mix_fwd.  workspace: nsa_decode_workspace_size bytes. */

@@ -66,7 +66,8 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(DecodeArgs a) {
       const int p = pos0 + 16 * u, slot = p / a.lprime;
       const int blk = slot < a.nslots ? __builtin_amdgcn_readlane(lv, slot) : -1;
       const int64_t k0 = (int64_t)blk * a.lprime + p % a.lprime;
-      const bool ok = blk >= 0 && k0 <= a.t;
+      // a block counts at the first slot that names it (the cleaned lists are sets as well)
+      const bool ok = blk >= 0 && k0 <= a.t && __builtin_ctzll(__ballot(lv == blk)) == slot;
       key0[u] = ok ? (int)k0 : 0;
       nv[u] = ok ? min(16, a.t + 1 - (int)k0) : 0;
     }

@@ -320,7 +320,7 @@ def decode_attn(q, kv, n_cmp: int, indices, gates, gate_act: int, t: int, scale:
     """One decode step's attention and gated mix (nsa_decode_attn): q [Z,H,1,dk] at absolute
     position t; kv = (K_cmp, V_cmp, K_sel, V_sel, K_win, V_win), views [Z,G,tokens,*] of the
     caches, of which the first n_cmp compressed and t + 1 other tokens are read; indices
-    [Z,G,1,n] int64 contiguous, distinct in a row; gates [Z,H,1,3] (before the activation) in
+    [Z,G,1,n] int64 contiguous; gates [Z,H,1,3] (before the activation) in
     q's dtype.  Returns the mixed output [Z,H,1,dv] of [Z,1,H,dv] storage."""
     _check_device(q, *kv, indices, gates)
     Z, H, _, dk = q.shape

@@ -154,6 +154,25 @@ def test_decode_attention_keeps_nan(dev, br, bad, dtype):
     assert torch.equal(out[:, hpg:], clean[:, hpg:]) and torch.equal(out[0], clean[0])
 
 
+# repeated blocks count once, as in the forward kernels (whose cleaned lists are the same set): the
+# same bits as with -1 in the repeats' place
+@pytest.mark.parametrize("n", [2, 16, 64])
+def test_decode_attention_repeated_blocks(dev, n):
+    t, lp, d, w = 1500, 32, 64, 40
+    g = torch.Generator().manual_seed(n)
+    q, gates = torch.randn(2, 8, 1, d, generator=g).to(dev), torch.randn(2, 8, 1, 3, generator=g).to(dev)
+    kv = [torch.randn(2, 2, 20 if i < 2 else t + 1, d, generator=g).to(dev) for i in range(6)]
+    idx = torch.randint(0, max(n // 2, 1), (2, 2, 1, n), generator=g)
+    idx[0, 0, 0] = 5
+    once = idx.clone()
+    for row in once.view(-1, n):
+        for j in range(n - 1, 0, -1):
+            if row[j] in row[:j]:
+                row[j] = -1
+    a, b = (_ops.decode_attn(q, kv, 17, x.to(dev), gates, 1, t, 0.1, lp, w) for x in (idx, once))
+    assert torch.equal(a, b)
+
+
 # few-row linear layers: rows at the 16-row tiles, widths at the 16-feature tiles, inputs at the
 # 32- (16-) feature chunks, the eight waves' turns and a last chunk of one piece; several jobs,
 # grouped outputs, bias, relu.  fp32 sums: 1e-6 norm-relative; bf16 rounding of the result 2^-9
