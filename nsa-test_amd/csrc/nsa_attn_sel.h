@@ -305,7 +305,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   while (have) {
     const int key0 = c_key0, blk = c_blk;
     const int blk_hi = c_hi;
-    // S^T[key, col] for the 64 keys of this tile
+    // S^T[key, col] for the TK keys of this tile
     f32x4 st[NKS];
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
@@ -565,15 +565,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
 }
 
 // Whether the bf16 forward takes 32 columns a wave.  With a multiple of 32 heads the wave is
-// one timestep and reads its blocks once instead of twice (B2 H64 G2 T2000 dk 128: 214 -> 155 us).
+// one timestep and reads its blocks once instead of twice, but walks twice the products alone:
+// it pays from two waves per SIMD on (2048), and from four where every timestep selects all
+// blocks, which the 16-column workgroups share through LDS, and has many to walk.  16 against 32
+// columns in us, hpg 32 (64) dk 128: 1024 waves 37 / 41 (23 / 26), T2048 70 / 58 (116 / 94), T3000
+// 100 / 80 (180 / 128); 16 blocks of 16 slots: B2 T1024 46 / 52 (86 / 63), B2 G2 T1024 88 / 74 (168 /
+// 119); 8 of them: B4 T512 37 / 32 (57 / 47); B2 G2 H64 T2000 214 / 155.
 // Otherwise it pays where the timesteps of a wave select mostly the same blocks (few
 // blocks for the slots) and the launch still gives every SIMD two waves: H64 G4 T2048 dk 192
 // 137 -> 129 us, B2 H16 G4 T4096 dk 64 106 -> 98, B3 H16 G4 T1537 58 -> 51; with 8 blocks a slot the
 // union grows (H32 G2 T8192 dk 64 146 -> 153, T32768 dk 128 1150 -> 1218), with fewer waves the
 // latency shows (H8 G2 T4000 dk 64 47 -> 65).
 inline bool sel_fwd32(const AttnArgs& a) {
-  if (a.hpg % 32 == 0) return true;
-  return (int64_t)a.B * a.G * a.Tq * a.hpg >= 2048 * 32 && a.nblk <= 4 * a.nslots;
+  const int64_t waves = (int64_t)a.B * a.G * a.Tq * a.hpg / 32;
+  if (a.hpg % 32 == 0) return waves >= 4096 || (waves >= 2048 && (a.nblk > a.nslots || a.Tkv <= 512));
+  return waves >= 2048 && a.nblk <= 4 * a.nslots;
 }
 
 template <typename T, int DK, int DV>

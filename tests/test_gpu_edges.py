@@ -315,8 +315,10 @@ def test_compress_tokens_edges(dev, B, G, T, dk, dv, l, d, major, dtype):
         assert torch.equal(a, b)
 
 
-# the 32-column selection forward: one timestep a wave (32 and 64 heads a group; a partly filled
-# last workgroup, five rows: a lone key has an exact dQ of zero, so no relative error), several that share most blocks (from 65536 rows and at most
+# the 32-column selection forward: one timestep a wave (32 to 96 heads a group, from 2048 waves on,
+# from 4096 where all of more than 512 keys' blocks fit the slots: the rule's edges from both
+# sides; a partly filled last workgroup; five rows: a lone key has an exact dQ of zero, so no relative error), several that
+# share most blocks (from 65536 rows and at most
 # four blocks a slot on: the rule's edges from both sides), timesteps that straddle waves, blocks
 # of half a tile and of one and a half; the forward's workgroup orders for whole and partial rounds
 # of XCDs (the stored-dS dQ's: test_selection_dq_workgroup_order)
@@ -324,7 +326,11 @@ def test_compress_tokens_edges(dev, B, G, T, dk, dv, l, d, major, dtype):
     (1, 2, 32, 77, 64, 4, torch.bfloat16, 128, 128), (1, 1, 64, 5, 16, 1, torch.bfloat16, 64, 64),
     (1, 1, 64, 130, 48, 7, torch.bfloat16, 192, 128), (4, 4, 4, 1024, 32, 8, torch.bfloat16, 32, 32),
     (4, 4, 4, 1025, 32, 8, torch.bfloat16, 32, 32), (4, 4, 4, 1023, 16, 16, torch.bfloat16, 32, 32),
-    (8, 4, 3, 700, 64, 5, torch.bfloat16, 64, 64)])
+    (8, 4, 3, 700, 64, 5, torch.bfloat16, 64, 64), (1, 1, 64, 1023, 16, 3, torch.bfloat16, 64, 64),
+    (1, 1, 64, 1025, 16, 3, torch.bfloat16, 64, 64), (1, 1, 64, 1030, 48, 5, torch.bfloat16, 192, 128),
+    (1, 2, 32, 1029, 32, 33, torch.bfloat16, 64, 64), (2, 2, 32, 1025, 32, 33, torch.bfloat16, 64, 64),
+    (1, 1, 96, 1400, 16, 1, torch.bfloat16, 32, 32), (4, 1, 32, 512, 64, 8, torch.bfloat16, 32, 32),
+    (4, 1, 32, 513, 64, 9, torch.bfloat16, 32, 32)])
 def test_selection_forward_32_columns(dev, B, G, hpg, T, lp, n, dtype, dk, dv):
     q, kp, v, do = _make(hpg + T, B, G * hpg, G, T, T, dk, dv, dtype, dev)
     idx = _lists(T, B, G, T, n, (T + lp - 1) // lp).to(dev)
