@@ -533,7 +533,8 @@ int nsa_decode_attn(const nsa_decode_args* args, void* workspace, size_t workspa
  * token), and the gate; bit 1: Eq. 8 -> top-n over the n_blocks compressed keys
  * (k_cmp / v_cmp, unit feature stride, strides z, g, block; block_ends [n_blocks]; n_cmp of
  * them completed), the attention and mix of nsa_decode_attn, and out [Z, d_model] (row stride
- * ld_out) through layer 9.  Both phases of a step get the same workspace
+ * ld_out) through layer 9, or with w[9] null the mixed heads themselves, out [Z, H dv] (16-byte
+ * aligned rows).  Both phases of a step get the same workspace
  * (nsa_decode_step_workspace_size bytes, 16-byte aligned), which carries q and the gate. */
 typedef struct nsa_decode_step_args {
   const void* x;

@@ -739,7 +739,12 @@ int nsa_decode_step(const nsa_decode_step_args* x, void* ws, size_t ws_bytes, ns
     a.indices = idx;
     a.gates = z;
     a.out = o;
+    if (!x->w[9]) {  // no output projection: the mixed heads are the result
+      a.out = x->out;
+      a.stride_oz = x->ld_out;
+    }
     if ((rc = nsa_decode_attn(&a, at<char>(ws, L.attn), L.attn_bytes, stream))) return rc;
+    if (!x->w[9]) return NSA_OK;
     const nsa_linear_job out = job(9, x->out, x->d_model, x->ld_out, 0, x->d_model, 0);
     if ((rc = nsa_linear_few(o, (int64_t)H * dv, x->Z, H * dv, &out, 1, x->dtype, stream))) return rc;
   }

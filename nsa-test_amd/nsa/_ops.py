@@ -350,11 +350,20 @@ def decode_attn(q, kv, n_cmp: int, indices, gates, gate_act: int, t: int, scale:
 
 
 # Rows up to which linear_few stands for torch's GEMMs: 64 (the kernel's most) for a token's
-# eight projections in one launch, 16 for a single layer.  Measured in bf16, launch against
-# F.linear: 17408 x 2560 weights (as one layer) 1 / 16 / 32 / 64 rows 17 / 25 / 43 / 70 us against 35 /
-# 35 / 19 / 19 us, where eight layers take eight such GEMMs and six cache copies; 2560 x 8192
-# 13 / 20 / 26 / 38 us against 19 us; 2304 x 512 6 us against 19 us (its host time).
-LINEAR_FEW_ROWS, LINEAR_ONE_ROWS = 64, 16
+# eight projections in one launch: bf16 17408 x 2560 weights (as one layer) 1 / 16 / 32 / 64 rows
+# 17 / 25 / 43 / 70 us, where eight layers take eight GEMMs of 19 us and six cache copies.
+LINEAR_FEW_ROWS = 64
+# rows x out x in features up to which it stands for a single F.linear, whose call takes the host
+# 19 us at any of these sizes.  bf16 1 / 16 / 32 / 64 rows: 2560 x 8192 14 / 20 / 26 / 38 us, 2560 x
+# 4096 8 / 12 / 15 / 21, 1024 x 2048 6 / 7 / 10 / 12, 192 x 1280 6 / 7 / 7 / 11; fp32 2560 x 4096 15 / 21 /
+# 28 / 46, 1024 x 2048 8 / 12 / 15 / 23, 192 x 1280 6 / 8 / 11 / 17.
+LINEAR_ONE_WORK = {torch.bfloat16: 320 << 20, torch.float32: 80 << 20}
+
+
+def linear_one(rows: int, n: int, k: int, dtype: torch.dtype) -> bool:
+    """Whether linear_few runs one layer of [n, k] weights over `rows` rows at least as fast as
+    F.linear."""
+    return rows <= LINEAR_FEW_ROWS and rows * n * k <= LINEAR_ONE_WORK.get(dtype, 0)
 
 
 def linear_few(x, jobs) -> None:

@@ -999,13 +999,17 @@ class NSAAttention(torch.nn.Module):
             return None
         projs, bufs, (g0, g2) = few
         x2 = _ops._rows(x.reshape(B, D))
-        out = x.new_empty(B, 1, D)
+        # a large output projection over many rows is F.linear's: the step then ends with the heads
+        one = _ops.linear_one(B, D, H * dv, x.dtype)
+        out = x.new_empty(B, 1, D if one else H * dv)
         n_act = (t + 1 - c.l) // c.d + 1 if t + 1 >= c.l else 0  # blocks once the token is in
         np_ = _n_pad(max(n_act, 1))
         a = _lib.DecodeStepArgs()
-        a.x, a.ld_x, a.out, a.ld_out = x2.data_ptr(), x2.stride(0), out.data_ptr(), D
+        a.x, a.ld_x, a.out, a.ld_out = x2.data_ptr(), x2.stride(0), out.data_ptr(), out.shape[-1]
         ps = [m._parameters for m in (self._modules["q_proj"], *projs, g0, g2, o_proj)]
         a.w[:] = [p["weight"].data_ptr() for p in ps]
+        if not one:
+            a.w[9] = None
         a.bias[:] = [None if p["bias"] is None else p["bias"].data_ptr() for p in ps]
         a.ldw[:] = [D, D, D, D, D, D, D, D, g0.out_features, H * dv]
         a.cache[:] = [b.data_ptr() for b in bufs]
@@ -1031,7 +1035,7 @@ class NSAAttention(torch.nn.Module):
         a.phases = 2 if new_block else 3
         _lib.call("nsa_decode_step", p, wp, nb, stream)
         cache.length = t + 1
-        return out
+        return out if one else o_proj(out)
 
     def _decode_inputs(self, x: torch.Tensor, cache: NSAKVCache):
         """The token x [B,1,D] joins the cache; returns its queries [B,H,1,dk] and gate logits
@@ -1102,7 +1106,7 @@ class NSAAttention(torch.nn.Module):
             os_ = [o.to(cdt).contiguous() for o in (o_c, o_s, o_w)]
             o = _mix_fwd(os_, gate_logits.to(cdt), GATE_ACT[c.gate_mode]).to(q.dtype)
         of = o.transpose(1, 2).reshape(B, H * dv)
-        if (B <= _ops.LINEAR_ONE_ROWS and H * dv * of.element_size() % 16 == 0
+        if (_ops.linear_one(B, D, H * dv, of.dtype) and H * dv * of.element_size() % 16 == 0
                 and _plain_linears(of, (self.o_proj, H * dv, D))):
             out = x.new_empty(B, 1, D)
             _ops.linear_few(of, [(self.o_proj.weight, self.o_proj.bias, out, D, 0, D, 0)])

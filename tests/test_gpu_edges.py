@@ -357,6 +357,27 @@ def test_selection_dq_workgroup_order(dev, B, G, hpg, T):
     assert ((acc.double() - want).abs() <= 2 ** -8 * (want.abs() + dq.double().abs()) + 1e-6).all()
 
 
+@pytest.mark.parametrize("rows,own", [(32, True), (33, False)])
+def test_decode_output_projection_rule(dev, rows, own, monkeypatch):
+    """The output projection of a decode step is F.linear's from the size on at which it is the
+    faster one (the rule's line moved to 32 rows of a small layer), with and without a bias, in
+    the whole step and in its parts alike."""
+    cfg = NSAConfig(d_model=64, head_dim_qk=64, head_dim_v=64, n_heads=8, n_kv_groups=2, l_prime=32, n=4, w=48,
+                    use_bias=rows == 33)
+    monkeypatch.setitem(_ops.LINEAR_ONE_WORK, torch.bfloat16, 32 * 64 * 512)
+    torch.manual_seed(rows)
+    m = NSAAttention(cfg).to(dev, torch.bfloat16).eval()
+    x = torch.randn(rows, 45, 64, device=dev).to(torch.bfloat16)
+    real, calls, res = torch.nn.functional.linear, [], []
+    for parts in (False, True):
+        cache = NSAKVCache(cfg, rows, 45, dev, torch.bfloat16)
+        m.prefill(x[:, :40], cache)
+        monkeypatch.setattr(torch.nn.functional, "linear", lambda *a: (calls.append(a[1].shape), real(*a))[1])
+        res.append(torch.cat([m.decode(x[:, t:t + 1], cache, output_attentions=parts)[0] for t in range(40, 45)], 1))
+        monkeypatch.setattr(torch.nn.functional, "linear", real)
+    assert calls == ([] if own else 10 * [(64, 512)]) and torch.equal(*res)
+
+
 # the whole decode step in one call against its parts (taken when the attention details are
 # asked for): the same kernels, so the same bits, with blocks completing on the way, before the
 # first block, with every gate mode, with and without fixed blocks, after a prompt and from empty
