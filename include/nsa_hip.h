@@ -442,7 +442,8 @@ int nsa_compress_pool_bwd(const void* Y, const void* C, const void* dR, const vo
  * (forward) and dR = dK W2, dk = dY W1[:, :dk] (backward), which the caller's GEMMs form.
  * Forward: C [l,W] = E W1[:, dk:]^T + b1, R (pooled, as nsa_compress_pool_fwd), K [Z,G,n_pad,dk]
  * = R W2^T + b2 and V_cmp [Z,G,n_pad,dv], the blocks from n_act on zero; W = 2 dk, R
- * [Z,G,n_pad,W] (rows from n_act on not written).  Backward, from X = k, dK, dV_cmp and dR (the
+ * [Z,G,n_pad,W] (rows from n_act on not written).  With W2 and K null the output layer is the
+ * caller's GEMM too, and those rows of R are zeros.  Backward, from X = k, dK, dV_cmp and dR (the
  * layouts of K, V_cmp, R): dY and dV (the layouts of Y, V), dW1, db1, dW2, db2, dE (each may be
  * null); sums over rows in fp32 in a fixed order.  All tensors compact, 16-byte aligned,
  * one dtype; token_major as above; b1 / b2 may be null.  dk a multiple of 64, l at most 64;

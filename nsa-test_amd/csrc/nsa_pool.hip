@@ -258,9 +258,10 @@ __global__ __launch_bounds__(256) void pool_fwd_vec_kernel(const typename Store<
   const int pc = threadIdx.x % ppt;
   if (threadIdx.x >= bpw * ppt || i >= np) return;
   const int64_t bg = blockIdx.y;
-  if (i >= n_act) {  // padding blocks: zero compressed keys and values (R is not read there)
+  if (i >= n_act) {  // padding blocks: zero compressed keys (without Kc zero R) and values
     const int c = pc * EPF;
-    if (c < dk) *reinterpret_cast<uint4*>(Kc + (bg * np + i) * dk + c) = make_uint4(0, 0, 0, 0);
+    if (Kc && c < dk) *reinterpret_cast<uint4*>(Kc + (bg * np + i) * dk + c) = make_uint4(0, 0, 0, 0);
+    if (!Kc && c < W) *reinterpret_cast<uint4*>(R + (bg * np + i) * W + c) = make_uint4(0, 0, 0, 0);
     if (c >= W) *reinterpret_cast<uint4*>(Vc + (bg * np + i) * dv + c - W) = make_uint4(0, 0, 0, 0);
     return;
   }
@@ -300,7 +301,7 @@ __global__ __launch_bounds__(256) void pool_fwd_vec_kernel(const typename Store<
 }
 
 // R / V_cmp of blocks 0 .. n_act - 1 of every (b, g), np block rows apart.  With np > n_act
-// (vectorised form only) the padding rows of Vc and of Kc [B,G,np,dk] are zeroed.
+// (vectorised form only) the padding rows of Vc and of Kc [B,G,np,dk] (null: of R) are zeroed.
 template <typename T>
 static void pool_fwd(const void* Y, const void* C, const void* V, void* R, void* Vc, void* Kc, int dk, int Z, int G,
                      int n_ctx, int W, int dv, int l, int d, int n_act, int np, int tm, hipStream_t st) {
@@ -421,7 +422,8 @@ extern "C" int nsa_compress_pool_bwd(const void* Y, const void* C, const void* d
 }
 
 // ---- compress_tokens around the two token-wise GEMMs (Y = k W1k^T, dR = dK W2) ----
-static int check_compress(const nsa_compress_args* x) {
+// (fwd: a null W2 and K leave the output layer to the caller)
+static int check_compress(const nsa_compress_args* x, bool fwd) {
   if (!x) return set_error(NSA_ERR_INVALID, "args is null");
   if (x->dtype != NSA_F32 && x->dtype != NSA_BF16) return set_error(NSA_ERR_INVALID, "dtype not supported");
   const int epf = x->dtype == NSA_F32 ? 4 : 8, W = 2 * x->head_dim_qk;
@@ -431,14 +433,14 @@ static int check_compress(const nsa_compress_args* x) {
   if (x->l > 64 || x->l % epf || x->head_dim_qk <= 0 || x->head_dim_qk % 64 || x->head_dim_v <= 0 ||
       x->head_dim_v % epf || (W + x->head_dim_v) / epf > 256)
     return set_error(NSA_ERR_UNSUPPORTED, "compress_tokens: widths without a kernel");
-  const void* in[] = {x->Y, x->C, x->V, x->R, x->K, x->V_cmp, x->E, x->W1, x->W2};
-  for (const void* p : in)
-    if (!p || (uintptr_t)p % 16) return set_error(NSA_ERR_LAYOUT, "compress_tokens: tensors must be 16-byte aligned");
+  const void* in[] = {x->Y, x->C, x->V, x->R, x->V_cmp, x->E, x->W1, x->K, x->W2};
+  for (int i = 0; i < (fwd && !x->W2 && !x->K ? 7 : 9); ++i)
+    if (!in[i] || (uintptr_t)in[i] % 16) return set_error(NSA_ERR_LAYOUT, "compress_tokens: tensors must be 16-byte aligned");
   return NSA_OK;
 }
 
 extern "C" int nsa_compress_fwd(const nsa_compress_args* x, nsa_stream_t stream) {
-  int rc = check_compress(x);
+  int rc = check_compress(x, true);
   if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
   const int dk = x->head_dim_qk, W = 2 * dk, esz = x->dtype == NSA_F32 ? 4 : 2, BG = x->Z * x->n_kv_groups;
@@ -451,12 +453,16 @@ extern "C" int nsa_compress_fwd(const nsa_compress_args* x, nsa_stream_t stream)
     fn(x->Y, x->C, x->V, x->R, x->V_cmp, x->K, dk, x->Z, x->n_kv_groups, x->n_ctx, W, x->head_dim_v, x->l, x->d,
        x->n_act, x->n_pad, x->token_major ? 1 : 0, st);
   }
+  if (!x->W2) {
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? NSA_OK : set_error(NSA_ERR_HIP, hipGetErrorString(e));
+  }
   nsa_linear_job k{x->W2, x->b2, x->K, W, dk, 0, dk, dk, 0};
   return launch_linear_rows(x->R, W, x->n_act, W, BG, (int64_t)x->n_pad * W, (int64_t)x->n_pad * dk, k, x->dtype, st);
 }
 
 extern "C" size_t nsa_compress_bwd_workspace_size(const nsa_compress_args* x) {
-  if (check_compress(x)) return 0;
+  if (check_compress(x, false)) return 0;
   const int dk = x->head_dim_qk, W = 2 * dk, BG = x->Z * x->n_kv_groups;
   const size_t a = wgrad_bytes(BG * x->n_act, dk, W), b = wgrad_bytes(BG * x->n_ctx, W, dk);
   return (size_t)x->l * W * 4 + (a > b ? a : b);
@@ -464,7 +470,7 @@ extern "C" size_t nsa_compress_bwd_workspace_size(const nsa_compress_args* x) {
 
 extern "C" int nsa_compress_bwd(const nsa_compress_args* x, const nsa_compress_grads* g, void* ws, size_t ws_bytes,
                                 nsa_stream_t stream) {
-  int rc = check_compress(x);
+  int rc = check_compress(x, false);
   if (rc) return rc;
   if (!g || !g->X || !g->dK || !g->dV_cmp || !g->dR || !g->dY || !g->dV)
     return set_error(NSA_ERR_INVALID, "compress_tokens: null gradient");

@@ -560,6 +560,13 @@ class _CompressTokens(torch.autograd.Function):
     padding; the pooling's and all weights' gradients).  keys / values [B,G,T,*], or [B,T,G,*]
     with tm.  Returns (K_cmp as [B,G,Np,dk], V_cmp [B,G,Np,dv])."""
 
+    # Multiply-adds of the output layer (block rows x 2 dk x dk) up to which the HIP call runs it:
+    # past them its re-reads of the rows cost more than a GEMM and the clearing of the padding.
+    # Call's kernel / GEMM in us, bf16: dk 192 2044 rows 13 / 7, 8188 33 / 11, 32764 127 / 20; dk 64
+    # 16376 15 / 7; fp32: dk 192 2044 14 / 9, 8188 39 / 16; the clearing 4, both launches 30 of the host.
+    # Whole forward, bf16 G4 dk 192: T16384 94 / 109 us, T32768 145 / 126, B4 T32768 540 / 441.
+    OWN_OUT = 320 << 20
+
     @staticmethod
     def usable(keys, values, W1, b1, W2, b2, E, l) -> bool:
         """Whether the HIP calls take these: fp32 / bf16 on the GPU outside autocast, dk a multiple
@@ -583,12 +590,16 @@ class _CompressTokens(torch.autograd.Function):
         Y = torch.mm(keys.view(-1, dk), W1[:, :dk].t())
         C = torch.empty(l, W, device=dev, dtype=dt)
         R = torch.empty(B, G, n_pad, W, device=dev, dtype=dt)
-        K = torch.empty(B, G, n_pad, dk, device=dev, dtype=dt)
+        own = B * G * n_act * W * dk <= _CompressTokens.OWN_OUT
+        K = torch.empty(B, G, n_pad, dk, device=dev, dtype=dt) if own else None
         V = torch.empty(B, G, n_pad, dv, device=dev, dtype=dt)
         ctx.dims = (B, G, T, dk, dv, l, d, n_act, n_pad, int(tm), _ops._dtype_code(dt))
         ctx.has_b = (b1 is not None, b2 is not None)
-        a = _CompressTokens._args(ctx.dims, Y, C, values, R, K, V, E, W1, b1, W2, b2)
+        a = _CompressTokens._args(ctx.dims, Y, C, values, R, K, V, E, W1, b1, W2 if own else None, b2)
         _lib.call("nsa_compress_fwd", ctypes.byref(a), _ops._stream(dev))
+        if not own:
+            K = F.linear(R, W2, b2)
+            K[:, :, n_act:].zero_()
         ctx.save_for_backward(keys, Y, C, R, W1, W2, E)
         return K, V
 

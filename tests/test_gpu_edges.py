@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from nsa import NSAAttention, NSAConfig, NSAKVCache, _ops
-from nsa.kernels import score_and_select
+from nsa.kernels import _CompressTokens, score_and_select
 from test_gpu_branches import _check, _make
 
 pytestmark = pytest.mark.gpu
@@ -272,7 +272,7 @@ def test_sliding_chunks_out_of_sight(dev, B, G, hpg, T, w, dtype, dk, dv):
     (1, 1, 8, 64, 8, 8, 8, False), (1, 2, 32, 64, 64, 32, 16, True), (2, 3, 177, 128, 40, 32, 16, True),
     (2, 2, 95, 192, 128, 32, 32, False), (1, 4, 1056, 192, 128, 32, 16, True), (3, 1, 130, 64, 128, 64, 16, False)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-def test_compress_tokens_edges(dev, B, G, T, dk, dv, l, d, major, dtype):
+def test_compress_tokens_edges(dev, B, G, T, dk, dv, l, d, major, dtype, monkeypatch):
     cfg = NSAConfig(d_model=64, head_dim_qk=dk, head_dim_v=dv, n_heads=G, n_kv_groups=G, l=l, d=d, l_prime=64 if 64 % d == 0
                     else d)
     torch.manual_seed(T)
@@ -306,6 +306,13 @@ def test_compress_tokens_edges(dev, B, G, T, dk, dv, l, d, major, dtype):
     assert max(err(kc[..., :n].transpose(-1, -2), rk), err(vc[:, :, :n], rv)) < (1e-2 if bf else 1e-5)
     errs = {x: err(a, b) for x, a, b in zip(("k", "v") + names, got, want)}
     assert max(errs.values()) < (6e-2 if bf else 1e-5), errs
+    # the output layer as a GEMM of the caller's (many rows): the same pooled rows, the same zeros
+    monkeypatch.setattr(_CompressTokens, "OWN_OUT", 0)
+    gc, gvc, _, _ = m.compress_tokens(k, v)
+    assert torch.equal(gvc, vc) and not gc[..., n:].any() and err(gc[..., :n].transpose(-1, -2), rk) < (1e-2 if bf else 1e-5)
+    for a, b in zip(torch.autograd.grad([gc, gvc], [k, v, *ps], [gk, gv]), got):
+        assert torch.equal(a, b)
+    monkeypatch.undo()
     # frozen layers: the other gradients are the same
     for p in ps[2:]:
         p.requires_grad_(False)
