@@ -445,7 +445,7 @@ int nsa_compress_pool_bwd(const void* Y, const void* C, const void* dR, const vo
  * [Z,G,n_pad,W] (rows from n_act on not written).  With W2 and K null the output layer is the
  * caller's GEMM too, and those rows of R are zeros.  Backward, from X = k, dK, dV_cmp and dR (the
  * layouts of K, V_cmp, R): dY and dV (the layouts of Y, V), dW1, db1, dW2, db2, dE (each may be
- * null); sums over rows in fp32 in a fixed order.  All tensors compact, 16-byte aligned,
+ * null; X null leaves dW1[:, :dk] to the caller); sums over rows in fp32 in a fixed order.  All tensors compact, 16-byte aligned,
  * one dtype; token_major as above; b1 / b2 may be null.  dk a multiple of 64, l at most 64;
  * l and dv whole 16-byte pieces, (W + dv) at most 256 of them. */
 typedef struct nsa_compress_args {

@@ -472,7 +472,7 @@ extern "C" int nsa_compress_bwd(const nsa_compress_args* x, const nsa_compress_g
                                 nsa_stream_t stream) {
   int rc = check_compress(x, false);
   if (rc) return rc;
-  if (!g || !g->X || !g->dK || !g->dV_cmp || !g->dR || !g->dY || !g->dV)
+  if (!g || !g->dK || !g->dV_cmp || !g->dR || !g->dY || !g->dV)
     return set_error(NSA_ERR_INVALID, "compress_tokens: null gradient");
   if (((uintptr_t)g->X | (uintptr_t)g->dK | (uintptr_t)g->dV_cmp | (uintptr_t)g->dR | (uintptr_t)g->dY |
        (uintptr_t)g->dV) % 16)
@@ -495,7 +495,7 @@ extern "C" int nsa_compress_bwd(const nsa_compress_args* x, const nsa_compress_g
   const unsigned blocks = (l * W + W + 255) / 256 + (l * l * 64 + 255) / 256;
   if (x->dtype == NSA_F32) hipLaunchKernelGGL(compress_pos_grad_kernel<float>, dim3(blocks), dim3(256), 0, st, dC, a);
   else hipLaunchKernelGGL(compress_pos_grad_kernel<bf16>, dim3(blocks), dim3(256), 0, st, dC, a);
-  if (g->dW1)
+  if (g->dW1 && g->X)
     launch_wgrad(x->dtype, g->dY, W, g->X, dk, BG * x->n_ctx, BG * x->n_ctx, BG * x->n_ctx, W, dk, g->dW1, dk + l,
                  nullptr, part, st);
   hipError_t e = hipGetLastError();

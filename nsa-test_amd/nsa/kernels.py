@@ -443,6 +443,17 @@ def _wgrad_hip(dy2, x2, W) -> bool:
             and dy2.stride(0) >= W.shape[0] and x2.stride(0) >= W.shape[1])
 
 
+def _split_rows_wgrad(dy2, x2):
+    """dy2^T x2 as one batched GEMM over up to 64 row chunks with fp32 partials, then summed."""
+    rows, S = x2.shape[0], 64
+    while S > 1 and (rows % S or rows // S < 256):
+        S //= 2
+    if S > 1 and dy2.is_cuda:
+        return torch.bmm(dy2.view(S, rows // S, -1).transpose(1, 2), x2.view(S, rows // S, -1),
+                         out_dtype=torch.float32).sum(0)
+    return dy2.t() @ x2
+
+
 class _LinearSplitK(torch.autograd.Function):
     """y = x W^T (+ b) whose weight gradient is a reduction over every row of x (all
     B*G*T tokens for the compression MLP, against a 384 x 192 output): a single GEMM of
@@ -475,15 +486,7 @@ class _LinearSplitK(torch.autograd.Function):
                           W.shape[1], _ops._ptr(dW), dW.stride(0), _lib.NSA_BF16, _ops._ptr(ws), ws.numel(),
                           _ops._stream(W.device))
             else:
-                S = 64
-                while S > 1 and (rows % S or rows // S < 256):
-                    S //= 2
-                if S > 1 and dy2.is_cuda:
-                    part = torch.bmm(dy2.view(S, rows // S, -1).transpose(1, 2), x2.view(S, rows // S, -1),
-                                     out_dtype=torch.float32)
-                    dW = part.sum(0).to(W.dtype)
-                else:
-                    dW = dy2.t() @ x2
+                dW = _split_rows_wgrad(dy2, x2).to(W.dtype)
         if ctx.has_b and ctx.needs_input_grad[2]:
             db = dy2.sum(0)
         return dx, dW, db
@@ -566,6 +569,11 @@ class _CompressTokens(torch.autograd.Function):
     # 16376 15 / 7; fp32: dk 192 2044 14 / 9, 8188 39 / 16; the clearing 4, both launches 30 of the host.
     # Whole forward, bf16 G4 dk 192: T16384 94 / 109 us, T32768 145 / 126, B4 T32768 540 / 441.
     OWN_OUT = 320 << 20
+    # Rows x 2 dk of dY up to which the call forms dW1[:, :dk] in fp32 too (in bf16 always): its tiles
+    # of 64 output rows reach 60 to 70 TFLOP/s there, the batched GEMM 120, in two launches more.
+    # Kernel / GEMM and sum in us: dk 192 32768 rows 79 / 55, 131072 300 / 180; dk 64 65536 42 / 29,
+    # 262144 158 / 50.
+    OWN_WGRAD32 = 12 << 20
 
     @staticmethod
     def usable(keys, values, W1, b1, W2, b2, E, l) -> bool:
@@ -624,13 +632,16 @@ class _CompressTokens(torch.autograd.Function):
         db1 = W1.new_empty(2 * dk) if ctx.has_b[0] and need[3] else None
         db2 = W2.new_empty(dk) if ctx.has_b[1] and need[5] else None
         # (values, K, V_cmp and the biases are forward operands: any aligned address stands in)
+        own = Y.dtype != torch.float32 or Y.numel() <= _CompressTokens.OWN_WGRAD32
         a = _CompressTokens._args(ctx.dims, Y, C, keys, R, dK, dV, E, W1, None, W2, None)
         g = _lib.CompressGrads(*[None if t is None else t.data_ptr()
-                                 for t in (keys, dK, dV, dR, dY, dval, dW1, db1, dW2, db2, dE)])
+                                 for t in (keys if own else None, dK, dV, dR, dY, dval, dW1, db1, dW2, db2, dE)])
         ws = torch.empty(_lib.size_of("nsa_compress_bwd_workspace_size", a, ctx.dims), device=Y.device,
                          dtype=torch.uint8)
         _lib.call("nsa_compress_bwd", ctypes.byref(a), ctypes.byref(g), _ops._ptr(ws), ws.numel(),
                   _ops._stream(Y.device))
+        if dW1 is not None and not own:
+            dW1[:, :dk] = _split_rows_wgrad(dY.view(-1, 2 * dk), keys.view(-1, dk))
         dkeys = torch.mm(dY, W1[:, :dk]).view(keys.shape) if need[0] else None
         return dkeys, dval if need[1] else None, dW1, db1, dW2, db2, dE, None, None, None, None, None
 

@@ -312,6 +312,11 @@ def test_compress_tokens_edges(dev, B, G, T, dk, dv, l, d, major, dtype, monkeyp
     assert torch.equal(gvc, vc) and not gc[..., n:].any() and err(gc[..., :n].transpose(-1, -2), rk) < (1e-2 if bf else 1e-5)
     for a, b in zip(torch.autograd.grad([gc, gvc], [k, v, *ps], [gk, gv]), got):
         assert torch.equal(a, b)
+    # and, in fp32, the token half of the first layer's weight gradient
+    monkeypatch.setattr(_CompressTokens, "OWN_WGRAD32", 0)
+    gc, gvc, _, _ = m.compress_tokens(k, v)
+    for x, a, b, w in zip(("k", "v") + names, torch.autograd.grad([gc, gvc], [k, v, *ps], [gk, gv]), got, want):
+        assert torch.equal(a, b) if bf or x != names[0] else err(a, w) < 1e-5, x
     monkeypatch.undo()
     # frozen layers: the other gradients are the same
     for p in ps[2:]:
