@@ -985,8 +985,10 @@ class NSAAttention(torch.nn.Module):
                 or type(self)._project_kv is not NSAAttention._project_kv or dk % 16 or dv % 16):
             return None
         g0, act, g2 = gm._modules.values()
+        gd, ad, sd = gm.__dict__, act.__dict__, self.__dict__
         if (type(g0) is not torch.nn.Linear or type(act) is not torch.nn.ReLU
-                or any(m.__dict__[h] for m in (gm, act) for h in ("_forward_hooks", "_forward_pre_hooks"))):
+                or gd["_forward_hooks"] or gd["_forward_pre_hooks"] or ad["_forward_hooks"] or ad["_forward_pre_hooks"]
+                or "forward" in gd or "forward" in ad or "prefill" in sd or "_project_kv" in sd):
             return None
         hw = g0.out_features
         projs = (md["k_compress"], md["v_compress"], md["k_select"], md["v_select"], md["k_sliding"], md["v_sliding"])

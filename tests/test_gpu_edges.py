@@ -369,6 +369,26 @@ def test_selection_dq_workgroup_order(dev, B, G, hpg, T):
     assert ((acc.double() - want).abs() <= 2 ** -8 * (want.abs() + dq.double().abs()) + 1e-6).all()
 
 
+@pytest.mark.parametrize("what", ["gate_mlp", "gate_mlp.1", "k_select", "prefill", "_project_kv"])
+def test_decode_runs_what_was_replaced(dev, what):
+    """A forward replaced on a module's instance, or a method on the layer's, runs in a decode step
+    (which otherwise passes the modules by), with the step's own result."""
+    cfg = NSAConfig(d_model=64, head_dim_qk=64, head_dim_v=64, n_heads=8, n_kv_groups=2, l_prime=32, n=4, w=40)
+    torch.manual_seed(0)
+    m = NSAAttention(cfg).to(dev, torch.bfloat16).eval()
+    x = torch.randn(2, 37, 64, device=dev).to(torch.bfloat16)
+    calls, res = [], []
+    for replaced in (False, True):
+        c = NSAKVCache(cfg, 2, 40, dev, torch.bfloat16)
+        m.prefill(x[:, :35], c)
+        if replaced:
+            owner, name = (m, what) if hasattr(type(m), what) else (m.get_submodule(what), "forward")
+            real = getattr(owner, name)
+            setattr(owner, name, lambda *a: (calls.append(1), real(*a))[1])
+        res.append(torch.cat([m.decode(x[:, t:t + 1], c)[0] for t in (35, 36)], 1).double())
+    assert len(calls) == 2 and (res[0] - res[1]).norm() < 1e-2 * res[0].norm()
+
+
 @pytest.mark.parametrize("rows,own", [(32, True), (33, False)])
 def test_decode_output_projection_rule(dev, rows, own, monkeypatch):
     """The output projection of a decode step is F.linear's from the size on at which it is the
