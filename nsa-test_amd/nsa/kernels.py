@@ -586,7 +586,8 @@ class _CompressTokens(torch.autograd.Function):
         ts = [values, W1, W2, E] + [b for b in (b1, b2) if b is not None]
         return (all(t.dtype == dt and t.device == keys.device for t in ts) and dk % 64 == 0 and dv % epf == 0
                 and l <= 64 and l % epf == 0 and (2 * dk + dv) // epf <= 256 and W1.shape == (2 * dk, dk + l)
-                and W2.shape == (dk, 2 * dk) and E.shape == (l, l))
+                and W2.shape == (dk, 2 * dk) and E.shape == (l, l) and (b1 is None or b1.shape == (2 * dk,))
+                and (b2 is None or b2.shape == (dk,)))
 
     @staticmethod
     def forward(ctx, keys, values, W1, b1, W2, b2, E, l, d, n_act, n_pad, tm):

@@ -327,6 +327,26 @@ def test_compress_tokens_edges(dev, B, G, T, dk, dv, l, d, major, dtype, monkeyp
         assert torch.equal(a, b)
 
 
+def test_compress_tokens_broadcast_bias(dev):
+    """A bias of one element broadcasts, as in F.linear (the one-call form reads whole biases)."""
+    cfg = NSAConfig(d_model=64, head_dim_qk=64, head_dim_v=64, n_heads=2, n_kv_groups=2)
+    torch.manual_seed(0)
+    m = NSAAttention(cfg).to(dev)
+    k, v = (torch.randn(1, 2, 100, 64, device=dev) for _ in range(2))
+    res = []
+    for one in (True, False):
+        for lay in (m.compress_mlp[0], m.compress_mlp[2]):
+            b = torch.full((1,), 0.3, device=dev)
+            lay.bias = torch.nn.Parameter(b if one else b.expand(lay.out_features).clone())
+        assert _CompressTokens.usable(k, v, m.compress_mlp[0].weight, m.compress_mlp[0].bias, m.compress_mlp[2].weight,
+                                      m.compress_mlp[2].bias, m.pos_embed.weight, cfg.l) is not one
+        kc = m.compress_tokens(k, v)[0]
+        kc.square().sum().backward()
+        res.append((kc.double(), *(lay.bias.grad.double().sum() for lay in (m.compress_mlp[0], m.compress_mlp[2]))))
+    for a, b in zip(*res):
+        assert ((a - b).norm() / b.norm()).item() < 1e-5
+
+
 # the 32-column selection forward: one timestep a wave (32 to 96 heads a group, from 2048 waves on,
 # from 4096 where all of more than 512 keys' blocks fit the slots: the rule's edges from both
 # sides; a partly filled last workgroup; five rows: a lone key has an exact dQ of zero, so no relative error), several that
