@@ -351,8 +351,11 @@ int nsa_sliding_window_fwd_noalloc(const void* Q, const void* K, const void* V, 
                                    int dtype, nsa_stream_t stream);
 
 /* ---- dK/dV schedule query (no reference counterpart: introspection for tests) --
- * The number of dK/dV work items per (batch, KV group) and the query-segment length
- * (128 or 256 entries) the backward entry points launch with for this shape. */
+ * The number of dK/dV work items per (batch, KV group) and the query-segment length (32 to
+ * 256 entries; the whole query span of a key tile where items own their tiles) the backward
+ * entry points launch with for this shape.  Compression: the work list is cut on the device
+ * from the block ends, into at most that many items, of that length or longer (from 32 entries
+ * on where the partials are fp32: segment below 128, or at most 512 items in all). */
 int nsa_bwd_dkdv_plan(int branch, int Z, int H, int n_kv_groups, int n_ctx_q, int n_ctx_kv, int n_slots,
                       int block_size_selection, int window_size, int* items_per_bg, int* segment);
 

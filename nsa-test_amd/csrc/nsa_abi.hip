@@ -88,6 +88,14 @@ struct Shape {
     return best;
   }
   int items_per_bg() const { return items_for(seg()); }
+  // bf16: the items' partials in fp32 where items are shorter than 128 entries, or where the
+  // compression work list may cut them shorter (cmp_plan_kernel): a key's sum over them then
+  // has no more bf16 roundings than with 128 entries (none).  Small launches only, where the
+  // partials are: at 512 items of 128 keys, dk + dv = 256, 67 MB
+  bool part32() const {
+    return dtype == NSA_BF16 && !direct() &&
+           (seg() < kSegTMax / 2 || (br == kCompression && (int64_t)Z * G * items_per_bg() <= kPart32Items));
+  }
   // selection backward with stored dS (bf16, whole 16-head groups, 64-key sub-blocks):
   // the dK/dV kernel runs first and stores dS, the dQ kernel reads it
   // (selection); sliding window / compression: bf16, whole 16-head groups, dS stored per
@@ -160,7 +168,7 @@ Layout make_layout(const Shape& s, bool bwd) {
   }
   if (bwd && s.br != kSelection && s.stored_ds()) L.ds = take(s.ds_bytes());
   if (bwd && s.br == kCompression) L.plan = take(((size_t)2 * s.key_tiles() + 2) * 4);
-  if (bwd && !s.direct()) L.partial = take(BG * s.items_per_bg() * dkdv_keys(s.br) * (size_t)(s.dk + s.dv) * s.esz());
+  if (bwd && !s.direct()) L.partial = take(BG * s.items_per_bg() * dkdv_keys(s.br) * (size_t)(s.dk + s.dv) * (s.part32() ? 4 : s.esz()));
   L.total = off;
   return L;
 }
@@ -415,6 +423,7 @@ int run_bwd(const Shape& s, const BwdIO& io, float scale, int window, const int3
   a.items_per_bg = s.items_per_bg();
   a.seg = s.seg();
   a.direct = s.direct() ? 1 : 0;
+  a.part32 = s.part32() ? 1 : 0;
   a.partial = at<char>(ws, L.partial);
 
   launch_repack_kv(s.dtype, io.K, io.sk, s.dk, const_cast<void*>(a.krf), const_cast<void*>(a.kcf), io.V, io.sv,

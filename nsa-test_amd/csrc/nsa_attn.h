@@ -23,9 +23,11 @@ constexpr int kRowChunk = 32;
 // Compression dQ from the stored dS keeps the block end of every 32-key chunk's first key
 // in LDS; the host stores dS for compression only up to this many chunks (65536 blocks).
 constexpr int kDqCbeMax = 2048;
-// Query entries (timesteps; selection: CSR entries) per dK/dV work item: 32 to 256,
-// chosen per launch, at most kSegTMax.
-constexpr int kSegTMax = 256;
+// Query entries (timesteps; selection: CSR entries) per dK/dV work item: kSegTMin to kSegTMax
+// (up to a whole row chunk of the same), chosen per launch.
+constexpr int kSegTMin = 32, kSegTMax = 256;
+// compression dK/dV items of a launch up to which their bf16 partials are kept in fp32
+constexpr int kPart32Items = 512;
 // dK/dV key tiles (all batches and groups) from which the sliding-window backward gives
 // each tile all its query rows in one work item (one item per CU or more)
 constexpr int kDkdvDirectItems = 256;
@@ -80,7 +82,8 @@ struct AttnArgs {
   int64_t sdk_b, sdk_g, sdk_t, sdk_d;
   void* dv;
   int64_t sdv_b, sdv_g, sdv_t, sdv_d;
-  void* partial;  // [items][keys][DK+DV] partial sums, fp32 (bf16 for bf16 inputs)
+  void* partial;  // [items][keys][DK+DV] partial sums, fp32 (bf16 for bf16 inputs without part32)
+  int part32;     // partials of bf16 inputs in fp32
   int items_per_bg;
   int q0;  // absolute position of query row 0 (0 unless a caller decodes past a cache)
   int seg;  // query entries per dK/dV work item

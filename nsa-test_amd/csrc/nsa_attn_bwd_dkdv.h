@@ -609,10 +609,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(DK <= 64 &&
     for (int j = 0; j < DV / 16; ++j) add4<T>(vp, (int64_t)(j * 16 + 4 * g4), a.sdv_d, dva[j]);
     return;
   }
-  // ---- write this item's partial (in the element type: the reduce sums the items' partials
-  // in fp32): lane holds dK^T[d = 16j + 4*g4 + i][key = mykey] ----
-  S* pp = reinterpret_cast<S*>(a.partial) + ((int64_t)bg * a.items_per_bg + item) * KEYS * (DK + DV) +
-          (int64_t)(wave * 16 + c16) * (DK + DV);
+  // ---- write this item's partial (in the element type, or fp32: the reduce sums the items'
+  // partials in fp32): lane holds dK^T[d = 16j + 4*g4 + i][key = mykey] ----
+  const int64_t pe = ((int64_t)bg * a.items_per_bg + item) * KEYS * (DK + DV) + (int64_t)(wave * 16 + c16) * (DK + DV);
+  if (sizeof(S) == 2 && a.part32) {
+    float* pf = reinterpret_cast<float*>(a.partial) + pe;
+#pragma unroll
+    for (int j = 0; j < DK / 16; ++j) store4<float>(pf + j * 16 + 4 * g4, dka[j] * a.scale);
+#pragma unroll
+    for (int j = 0; j < DV / 16; ++j) store4<float>(pf + DK + j * 16 + 4 * g4, dva[j]);
+    return;
+  }
+  S* pp = reinterpret_cast<S*>(a.partial) + pe;
 #pragma unroll
   for (int j = 0; j < DK / 16; ++j) store4<T>(pp + j * 16 + 4 * g4, dka[j] * a.scale);
 #pragma unroll

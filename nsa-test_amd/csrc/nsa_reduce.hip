@@ -38,21 +38,20 @@ bool dispatch_attn_bwd_dkdv(int dtype, int dk, int dv, int br, const AttnArgs& a
 // keys is seen from its earliest block end on, so the tiles' row spans shrink along the
 // sequence and end with the padding tiles' empty ones: cut at fixed rows for every tile, half
 // the items were empty, each still loading its keys and writing a partial of zeros, and the
-// busy ones filled their last round of CUs partly.  Here the segment length is the smallest
-// multiple of a row chunk with which the visible spans take at most max_items items.
-// dK/dV at B2 H32 G2 T5003 dk = dv = 128: 228 -> 115-136 us; H64 G4 T8192 dk = 192: 366 -> 322 us (with
-// 3 us more in the reduce and 4-7 us for this launch).
-__global__ __launch_bounds__(256) void cmp_plan_kernel(const int* block_ends, int Tkv, int Tq, int hpg, int seg_max,
-                                                       int max_items, int* plan) {
-  __shared__ int s_total, s_best;
+// busy ones filled their last round of CUs partly.  Here the segment is the multiple of a row
+// chunk, from seg_min on, with which the visible spans take the fewest entry-steps per CU
+// (rounds of 256 items x (segment + 16), as the host counts) in at most max_items items; of equal
+// ones the longest, for the fewest partials.  seg_min is the launch's own segment, so that no
+// key's sum has more bf16 partials than with fixed cuts, or kSegTMin where they are fp32.
+__global__ __launch_bounds__(256) void cmp_plan_kernel(const int* block_ends, int Tkv, int Tq, int hpg, int nbg,
+                                                       int seg_min, int seg_max, int max_items, int* plan) {
+  __shared__ unsigned long long s_best;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   constexpr int KEYS = dkdv_keys(kCompression);
   const int ntiles = (Tkv + KEYS - 1) / KEYS;
   int* so = plan + 1;
   int* ts = so + ntiles + 1;
-  if (tid == 0) s_total = 0, s_best = 255;
-  __syncthreads();
-  int mine = 0;
+  if (tid == 0) s_best = ~0ull;
   for (int k = wave; k < ntiles; k += 4) {
     int m = 0x7fffffff;
     for (int i = lane; i < KEYS; i += 64)
@@ -60,19 +59,19 @@ __global__ __launch_bounds__(256) void cmp_plan_kernel(const int* block_ends, in
     m = wave_butterfly(m, [](int x, int y) { return min(x, y); });
     m = min(max(m, 0), Tq);
     if (lane == 0) ts[k] = m;
-    mine += Tq - m;
   }
-  if (lane == 0) atomicAdd(&s_total, mine);
-  __syncthreads();  // ts and the total (at most ntiles x Tq rows) are written
-  // candidate i: (lo + i) row chunks; seg_max, among them, always fits
-  const int step = max(1, 32 / hpg);
-  const int lo = max(1, (s_total / max(max_items, 1) + step - 1) / step);
-  const int sg = min((lo + tid) * step, seg_max);
+  __syncthreads();  // ts is written
+  // candidate tid: tid row chunks past seg_min; the last one is seg_max, which always fits
+  const int step = max(1, kRowChunk / hpg);
+  const int sg = min((seg_min + step - 1) / step * step + tid * step, seg_max);
   int n = 0;
   for (int k = 0; k < ntiles && n <= max_items; ++k) n += (Tq - ts[k] + sg - 1) / sg;
-  if (n <= max_items) atomicMin(&s_best, tid);
+  if (n <= max_items) {
+    const unsigned long long cost = ((unsigned long long)n * nbg + 255) / 256 * (sg + 16);
+    atomicMin(&s_best, cost * 512 + (511 - sg));
+  }
   __syncthreads();
-  const int best = min((lo + s_best) * step, seg_max);
+  const int best = 511 - (int)(s_best & 511);
   if (tid == 0) plan[0] = best;
   if (wave == 0) {  // item prefix of the tiles
     int carry = 0;
@@ -93,11 +92,12 @@ __global__ __launch_bounds__(256) void cmp_plan_kernel(const int* block_ends, in
 }
 
 void launch_cmp_plan(const AttnArgs& a, int* plan, hipStream_t st) {
-  hipLaunchKernelGGL(cmp_plan_kernel, dim3(1), dim3(256), 0, st, a.block_ends, a.Tkv, a.Tq, a.hpg, a.seg,
-                     a.items_per_bg, plan);
+  hipLaunchKernelGGL(cmp_plan_kernel, dim3(1), dim3(256), 0, st, a.block_ends, a.Tkv, a.Tq, a.hpg, a.B * a.G,
+                     a.part32 ? kSegTMin : a.seg, std::max(a.seg, kSegTMax), a.items_per_bg, plan);
 }
 
-template <typename T>
+// P: the type of the partials
+template <typename T, typename P>
 __global__ __launch_bounds__(256) void partial_reduce_kernel(AttnArgs a, int DK, int DV, int br, int split) {
   using S = typename Store<T>::type;
   const int bg = blockIdx.y;
@@ -130,12 +130,15 @@ __global__ __launch_bounds__(256) void partial_reduce_kernel(AttnArgs a, int DK,
     step = nsubblk;
   }
   if ((count == 0 && !a.dkdv_ow) || key0 >= key_hi) return;
-  const S* base = reinterpret_cast<const S*>(a.partial) + (int64_t)bg * a.items_per_bg * keys * width;
+  const P* base = reinterpret_cast<const P*>(a.partial) + (int64_t)bg * a.items_per_bg * keys * width;
   const int64_t istride = (int64_t)step * keys * width;  // elements between consecutive items
-  // each thread sums a group of NE consecutive elements (16 bytes of every partial: DK
-  // and DV are multiples of NE, so a group never straddles dK / dV); blockIdx.z splits
-  // the tile's keys x width elements over `split` workgroups
-  constexpr int NE = 16 / sizeof(S);
+  // each thread sums a group of NE consecutive elements (16 bytes of the result, NP 16-byte
+  // pieces of every partial: DK and DV are multiples of NE, so a group never straddles dK /
+  // dV); blockIdx.z splits the tile's keys x width elements over `split` workgroups
+  constexpr int NE = 16 / sizeof(S), NP = NE * sizeof(P) / 16;
+  struct Piece {
+    uint4 v[NP];
+  };
   const int ng = keys * width / NE;
   const int per = (ng + split - 1) / split;
   const int g_end = min(ng, (int)(blockIdx.z + 1) * per);
@@ -161,36 +164,44 @@ __global__ __launch_bounds__(256) void partial_reduce_kernel(AttnArgs a, int DK,
     if (vec && !ow) old = *reinterpret_cast<const uint4*>(p);
     // the items' partials in item order (fixed: reproducible), eight (then four) loads in
     // flight; each partial is read once, so the loads stream past the caches
-    const S* src = base + (int64_t)first * keys * width + e;
-    auto ld = [&](int k) -> uint4 {
-      return __builtin_bit_cast(uint4, __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + k * istride)));
+    const P* src = base + (int64_t)first * keys * width + e;
+    auto ld = [&](int k) -> Piece {
+      Piece r;
+#pragma unroll
+      for (int j = 0; j < NP; ++j)
+        r.v[j] = __builtin_bit_cast(
+            uint4, __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + k * istride) + j));
+      return r;
     };
     float sum[NE];
 #pragma unroll
     for (int u = 0; u < NE; ++u) sum[u] = 0.f;
-    auto add = [&](const uint4& v) {
-      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-      if constexpr (NE == 8) {
+    auto add = [&](const Piece& r) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          sum[2 * u] += __uint_as_float(w[u] << 16);
-          sum[2 * u + 1] += __uint_as_float(w[u] & 0xffff0000u);
+      for (int j = 0; j < NP; ++j) {
+        const uint32_t w[4] = {r.v[j].x, r.v[j].y, r.v[j].z, r.v[j].w};
+        if constexpr (sizeof(P) == 2) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            sum[2 * u] += __uint_as_float(w[u] << 16);
+            sum[2 * u + 1] += __uint_as_float(w[u] & 0xffff0000u);
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) sum[4 * j + u] += __uint_as_float(w[u]);
         }
-      } else {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) sum[u] += __uint_as_float(w[u]);
       }
     };
     int k = 0;
     for (; k + 8 <= count; k += 8) {
-      uint4 v[8];
+      Piece v[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) v[u] = ld(k + u);
 #pragma unroll
       for (int u = 0; u < 8; ++u) add(v[u]);
     }
     for (; k + 4 <= count; k += 4) {
-      uint4 v[4];
+      Piece v[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) v[u] = ld(k + u);
 #pragma unroll
@@ -259,10 +270,10 @@ void launch_partial_reduce(int dtype, int dk, int dv, int br, const AttnArgs& a,
   int split = (int)std::min<int64_t>(std::max<int64_t>(kReduceSplit, (2048 + tb - 1) / tb), (n4 + 255) / 256);
   split = std::max(split, 1);
   dim3 grid(tiles, a.B * a.G, split);
-  if (dtype == kF32)
-    hipLaunchKernelGGL(partial_reduce_kernel<float>, grid, dim3(256), 0, st, a, dk, dv, br, split);
-  else
-    hipLaunchKernelGGL(partial_reduce_kernel<bf16>, grid, dim3(256), 0, st, a, dk, dv, br, split);
+  auto fn = dtype == kF32 ? partial_reduce_kernel<float, float>
+            : a.part32    ? partial_reduce_kernel<bf16, float>
+                          : partial_reduce_kernel<bf16, uint16_t>;
+  hipLaunchKernelGGL(fn, grid, dim3(256), 0, st, a, dk, dv, br, split);
 }
 
 }  // namespace nsa

@@ -247,6 +247,33 @@ def test_compression_work_list(dev, B, G, hpg, T, l, d, dtype, dk, dv):
     _check(_ops.COMPRESSION, q, kp, v, do, 1 / math.sqrt(dk), dtype, block_ends=be.to(dev))
 
 
+# dK/dV items of less than 128 entries (small launches) keep their partials in fp32: 128 rows of 16
+# heads whose dO, multiples of 1/128 that one key (selection: one block of 16, of weight 1/16 each)
+# takes whole, cancel but for one entry.  All sums are exact in fp32; a sum of 32 rows is not in bf16
+@pytest.mark.parametrize("branch", [_ops.SLIDING, _ops.COMPRESSION, _ops.SELECTION])
+def test_small_launch_partials_are_fp32(dev, branch):
+    T, hpg, d = 128, 16, 64
+    g = torch.Generator().manual_seed(branch)
+    half = torch.randint(-128, 129, (T * hpg // 2, d), generator=g).double() / 128
+    do = torch.cat([half, -half[torch.randperm(len(half), generator=g)]])
+    do[7] = 0
+    want = do.sum(0)
+    do = do.view(T, hpg, d).permute(1, 0, 2).unsqueeze(0).to(torch.bfloat16).to(dev)
+    n = {_ops.SLIDING: T, _ops.COMPRESSION: 1, _ops.SELECTION: 16}[branch]
+    k = torch.zeros(1, 1, n, d, device=dev, dtype=torch.bfloat16)
+    q = torch.zeros(1, hpg, T, d, device=dev, dtype=torch.bfloat16)
+    if branch == _ops.SLIDING:  # scores 32 for key 0, -32 for the others
+        q[..., 0], k[..., 0] = 16, -16
+        k[:, :, 0, 0] = 16
+    v = torch.zeros(1, 1, n, d, device=dev, dtype=torch.bfloat16)
+    kw = {_ops.SLIDING: dict(window=T), _ops.COMPRESSION: dict(block_ends=torch.zeros(1, dtype=torch.int32, device=dev)),
+          _ops.SELECTION: dict(indices=torch.zeros(1, 1, T, 1, dtype=torch.int64, device=dev), lprime=16, causal=False)}
+    out, L, M = _ops.attn_fwd(branch, q, k, v, 0.125, **kw[branch])
+    _, _, dv = _ops.attn_bwd(branch, q, k, v, out, do, L, M, 0.125, **kw[branch])
+    want = (want / 16 if branch == _ops.SELECTION else want).to(torch.bfloat16).double()
+    assert want.abs().max() > 0 and torch.equal(dv[0, 0, 0].double().cpu(), want)
+
+
 # sliding-window dK/dV: a wave whose 16 keys no row of a chunk sees skips it.  Windows below, at
 # and past a wave's keys and a row chunk, shorter and longer than the sequence; chunks of less
 # than a timestep to 32 of them; with and without stored dS; one item per key tile (256 tiles).

@@ -182,6 +182,22 @@ def test_dkdv_direct_mode(dev):
     _sampled_check(_ops.SLIDING, q, kp, v, do, np.arange(T), 1 / math.sqrt(d), window=w)
 
 
+def _compression_segment(plan, B, H, G, T, Tkv, block_ends):
+    """The segment length the compression work list takes (chosen on the device from the block
+    ends; the plan's is the host's own, the shortest it may take with bf16 partials): the rows
+    that see each 128-key tile in at most items_per_bg items of the fewest entry-steps per CU."""
+    first = [min(int(block_ends[k:k + 128].min()), T) for k in range(0, Tkv, 128)]
+    lo = 32 if plan["segment"] < 128 or plan["items_per_bg"] * B * G <= 512 else plan["segment"]
+    step = max(1, 32 // (H // G))
+    lo = -(-lo // step) * step
+
+    def items(sg):
+        return sum(-(-(T - t) // sg) for t in first)
+
+    cand = [sg for sg in {min(lo + i * step, 256) for i in range(256)} if items(sg) <= plan["items_per_bg"]]
+    return min(cand, key=lambda sg: (-(-items(sg) * B * G // 256) * (sg + 16), -sg))
+
+
 # ------------------------------------------- 256-entry dK/dV query segments at small T
 SEG_CASES = [
     # kind, B, H, G, T, dk, dv, extra
@@ -208,6 +224,7 @@ def test_dkdv_256_segments(dev, kind, B, H, G, T, dk, dv, extra):
     kw = dict(extra)
     if kind == _ops.COMPRESSION:
         kp, v, kw["block_ends"] = _compressed(c, 510, dev)
+        assert _compression_segment(plan, B, H, G, T, Tkv, kw["block_ends"]) == 256
     if kind == _ops.SELECTION:
         rng = np.random.default_rng(7)
         idx = rng.integers(0, (T + lp - 1) // lp, size=(B, G, T, n))
@@ -220,9 +237,13 @@ def test_dkdv_256_segments(dev, kind, B, H, G, T, dk, dv, extra):
 
 # ------------------------- dK/dV query segments between 128 and 256 entries
 # Small launches take the segment length in [128, 256] (a multiple of 32) that needs the
-# fewest entry-steps per CU; these shapes land on 160, 192 and 224.
+# fewest entry-steps per CU; these shapes land on 160, 192 and 224.  The compression's work list
+# then chooses its own by the rows that see each tile: 128 (with fp32 partials), 208 and 248 here.
+COMPRESSION_SEG = {(2, 3000): 128, (5, 3500): 208, (4, 3000): 248}
 MID_SEG_CASES = [
     # kind, B, H, G, T, dk, dv, extra, segment
+    (_ops.COMPRESSION, 5, 16, 4, 3500, 64, 64, {}, 192),
+    (_ops.COMPRESSION, 4, 16, 4, 3000, 64, 64, {}, 128),
     (_ops.SLIDING, 1, 64, 4, 3000, 64, 64, dict(window=300), 224),
     (_ops.COMPRESSION, 2, 16, 4, 3000, 64, 64, {}, 192),
     (_ops.SELECTION, 4, 64, 4, 700, 64, 64, dict(lprime=64, n=8), 160),
@@ -244,6 +265,7 @@ def test_dkdv_mid_segments(dev, kind, B, H, G, T, dk, dv, extra, segment):
     kw = dict(extra)
     if kind == _ops.COMPRESSION:
         kp, v, kw["block_ends"] = _compressed(c, 710, dev)
+        assert _compression_segment(plan, B, H, G, T, Tkv, kw["block_ends"]) == COMPRESSION_SEG[B, T]
     if kind == _ops.SELECTION:
         rng = np.random.default_rng(8)
         idx = rng.integers(0, (T + lp - 1) // lp, size=(B, G, T, n))
