@@ -91,7 +91,8 @@ struct Shape {
   // bf16: the items' partials in fp32 where items are shorter than 128 entries, or where the
   // compression work list may cut them shorter (cmp_plan_kernel): a key's sum over them then
   // has no more bf16 roundings than with 128 entries (none).  Small launches only, where the
-  // partials are: at 512 items of 128 keys, dk + dv = 256, 67 MB
+  // partials are: at 512 items of 128 keys, dk + dv = 256, 67 MB (reduce at H64 G4 T2048 dk 192 10.6 ->
+  // 13.4 us; error of its dK / dV against 64 bits 3.04e-3 / 2.87e-3 -> 2.56e-3 / 2.30e-3)
   bool part32() const {
     return dtype == NSA_BF16 && !direct() &&
            (seg() < kSegTMax / 2 || (br == kCompression && (int64_t)Z * G * items_per_bg() <= kPart32Items));

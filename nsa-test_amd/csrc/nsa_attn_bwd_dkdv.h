@@ -25,16 +25,17 @@
 // Compression items come from a work list built from the block ends (cmp_plan_kernel): only
 // the rows that see a tile's keys, cut into equal segments over all tiles.
 //
-// Bound by LDS reads (each wave reads the chunk's rows twice, busy 50 % of the cycles) and by
-// their latency at two waves per SIMD: the S and dP products of all row subtiles are therefore
-// one straight run of independent accumulator chains, and the mask stands under one branch on
-// scalar values (with the subtiles one after the other and a branch per masked element, T 8192
-// H64 G4 dk 192: sliding window 630 -> 547 us; compression, T 5003 H32 G2 dk 128, 124 -> 113-120;
-// selection 1061 -> 1023 alone, 1.2 ms either way within a long run: it takes 6.2 GB through
-// the memory side).
+// Bound by latency at two waves per SIMD (LDS busy 50 % of the cycles, but a quarter of its
+// reads, or 44 % fewer L2 misses, changed nothing): the S and dP products of all row subtiles are
+// therefore one straight run of independent accumulator chains, and the mask stands under one
+// branch on scalar values (with the subtiles one after the other and a branch per masked element,
+// T 8192 H64 G4 dk 192: sliding window 630 -> 547 us; compression, T 5003 H32 G2 dk 128, 124 ->
+// 113-120; selection 1061 -> 1023 alone, 1.2 ms either way within a long run: it takes 6.2 GB
+// through the memory side).
 //
-// Every item writes its fp32 dK/dV partial for its keys; a reduce kernel sums the
-// segments of each key tile in a fixed order and accumulates into the caller's dK/dV.
+// Every item writes its dK/dV partial for its keys, in the element type or, where items are
+// short, in fp32 (part32); a reduce kernel sums the segments of each key tile in fp32 in a
+// fixed order and accumulates into the caller's dK/dV.
 // Direct mode (sliding window with at least kDkdvDirectItems key tiles over all batches
 // and groups, so one item per tile still fills the machine): the item's segment is the
 // tile's whole query span and it adds its sums into dK/dV itself, with no partials and

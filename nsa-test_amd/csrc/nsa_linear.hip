@@ -7,7 +7,9 @@
 // workgroup takes 16 features for all rows (W rows as the A operand of 16 x 16 x 32 MFMAs, the
 // token rows as B); its eight waves take the K chunks in turn (together 512 contiguous bytes
 // of each weight row), kLinU loads per wave in flight, and add their sums in wave order
-// through LDS: fp32 throughout, rounded once.
+// through LDS: fp32 throughout, rounded once.  Every 16 features read the rows once more (from
+// L2), so past some rows x weights a library GEMM is faster: the callers say where (linear_one,
+// OWN_OUT).
 #include <stdio.h>
 
 #include "../../include/nsa_hip.h"

@@ -975,8 +975,9 @@ class NSAAttention(torch.nn.Module):
     def _decode_few(self, x: torch.Tensor, cache: NSAKVCache):
         """(the projections of the caches in order, the caches, the gate's layers) where the few-row
         kernels may run the token's layers on x [B,1,D], else None: plain layers (see
-        _plain_linears) over at most 64 rows, caches of x's dtype with unit-stride features, and
-        room for the token."""
+        _plain_linears), nothing replaced on the gate's modules or on this one's prefill /
+        _project_kv, at most 64 rows, caches of x's dtype with unit-stride features, and room for
+        the token."""
         c, md = self.config, self._modules
         B, _, D = x.shape
         H, G, dk, dv = c.n_heads, c.n_kv_groups, c.head_dim_qk, c.head_dim_v
@@ -1007,7 +1008,7 @@ class NSAAttention(torch.nn.Module):
         """The whole decode step in one library call (nsa_decode_step; two when the token completes
         a compression block): the output [B,1,D] before dropout, or None where it does not
         apply (see _decode_few; also plain output projection, compiled head widths, every
-        cache row 16-byte aligned).  A step is bound by the host: projections, scoring,
+        cache row 16-byte aligned; a large output projection over many rows is F.linear's).  A step is bound by the host: projections, scoring,
         attention and output as calls of their own took 155 us of it, this takes about 75."""
         c = self.config
         B, _, D = x.shape
@@ -1095,9 +1096,11 @@ class NSAAttention(torch.nn.Module):
     def decode(self, hidden_states: torch.Tensor, cache: NSAKVCache, output_attentions: bool = False):
         """One decode step (not in the reference): hidden_states [B,1,D] is the token at
         position t = cache.length.  Its keys / values join the cache, then the three
-        branches, the gates and the mix run for its query alone at absolute position t,
-        through the HIP kernels' decode extensions (scoring, attention forward with
-        q_offset = t).  Returns (out [B,1,D], info) as forward does for that row."""
+        branches, the gates and the mix run for its query alone at absolute position t:
+        plain layers as one library call (_decode_step); others through the modules, with the
+        scoring and attention kernels that read the cache in place, or the forward kernels
+        (q_offset = t) where its layout is another.  Returns (out [B,1,D], info) as forward
+        does for that row."""
         c = self.config
         B, T, D = hidden_states.shape
         if T != 1:
