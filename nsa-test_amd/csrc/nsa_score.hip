@@ -250,9 +250,18 @@ __global__ __launch_bounds__(256) void score_logits_kernel(ScoreArgs a) {
 // operands straight into registers, all of its loads in flight at once.  The four lanes of
 // a row load the same 16-byte pieces (one request) and each picks the elements of its k
 // slot.  Every column tile is computed, visible or not: the rows kernel masks.
-// Up to kLgFewRows query rows of a group (four row tiles, each reading K once more; the
-// 128-row tile is at least half padding there).  Bound by launch and load latency.
+// Bound by launch and load latency.  Where it runs (score_few): always for one row tile (the
+// 128-row tile would be 7/8 padding); up to kLgFewRows query rows of a group, four row tiles that
+// each read K once more, while the launch is small: 8192 waves in bf16, 2048 in fp32 (twice the
+// loads).  Call, tiled -> few rows in us: bf16 64 rows dk 64, 2048 blocks: 8192 waves 47 -> 36, 32768
+// 66 -> 89; 32 rows dk 128 16384 waves 135 -> 108, 64 rows 63 -> 79; fp32 64 rows dk 64: 2048 waves
+// 26 -> 21, 8192 39 -> 50, 32768 67 -> 143.
 constexpr int kLgFewRows = 64;
+__host__ inline bool score_few(int dtype, int rows, int NB, int ncs, int64_t nbg) {
+  if (rows > kLgFewRows || NB <= 0) return false;
+  const int64_t waves = (int64_t)(ncs / 16) * ((rows + 15) / 16) * nbg;
+  return rows <= 16 || waves <= (dtype == kF32 ? 2048 : 8192);
+}
 
 template <typename S>
 __global__ __launch_bounds__(256) void score_logits_few_kernel(ScoreArgs a) {
@@ -676,7 +685,7 @@ int launch_score_topn(int dtype, ScoreArgs a, hipStream_t st) {
   if (a.NB > kMaxCols || a.hpg > kMaxRows) return 1;
   a.ncs = score_ncs(a.NB);
   const int Rall = a.T * a.hpg;
-  if (Rall <= kLgFewRows && a.NB > 0) {
+  if (score_few(dtype, Rall, a.NB, a.ncs, (int64_t)a.B * a.G)) {
     const dim3 grid(a.ncs / 64, (Rall + 15) / 16, a.B * a.G);
     if (dtype == kF32) hipLaunchKernelGGL(score_logits_few_kernel<float>, grid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL(score_logits_few_kernel<uint16_t>, grid, dim3(256), 0, st, a);

@@ -37,14 +37,17 @@ def test_selection_bitmap_edges(dev, hpg, T, lp, n, dtype, dk, dv):
 
 
 # scoring with few rows (one MFMA tile per wave) and few timesteps (heads across waves): rows
-# about 16 / 64 (the tile and the rule's edge), 1 / 3 / 20 heads a group, block counts at the
+# about 16 / 64 (the tile and the rule's edge; past 16 rows 2048 / 2112 and 8192 / 8704 waves: the
+# other edges), 1 / 3 / 20 heads a group, block counts at the
 # 256-block pieces and 64-block tiles, both remaps (l/d = 2, l'/d = 4 and another), dk with a
 # remainder piece; indices and scores bit for bit
 @pytest.mark.parametrize("B,G,hpg,T,N,dk,l,lp", [(1, 2, 16, 1, 255, 64, 32, 64), (2, 2, 3, 5, 257, 40, 32, 64),
                                                  (1, 1, 16, 4, 64, 192, 32, 64), (1, 1, 13, 5, 65, 96, 32, 64),
                                                  (1, 2, 20, 3, 1030, 64, 32, 64), (3, 1, 4, 17, 600, 128, 64, 32),
                                                  (1, 2, 1, 64, 70, 64, 32, 64), (1, 1, 2, 1024, 100, 32, 32, 64),
-                                                 (1, 1, 2, 1025, 100, 32, 32, 64), (1, 1, 64, 1, 4096, 32, 32, 64)])
+                                                 (1, 1, 2, 1025, 100, 32, 32, 64), (1, 1, 64, 1, 4096, 32, 32, 64),
+                                                 (2, 4, 4, 8, 2048, 32, 32, 64), (2, 4, 4, 8, 2049, 32, 32, 64),
+                                                 (8, 4, 4, 16, 1024, 32, 32, 64), (8, 4, 4, 16, 1025, 32, 32, 64)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_score_few_rows(dev, B, G, hpg, T, N, dk, l, lp, dtype):
     g = torch.Generator().manual_seed(N + T)
