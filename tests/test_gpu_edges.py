@@ -377,6 +377,25 @@ def test_compress_tokens_broadcast_bias(dev):
         assert ((a - b).norm() / b.norm()).item() < 1e-5
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_compress_tokens_backward_under_autocast(dev, dtype):
+    """A backward that runs inside an autocast region (the forward outside) takes its products in
+    the tensors' own type: autocast's float16 ones would be read as another type by the call."""
+    cfg = NSAConfig(d_model=64, head_dim_qk=64, head_dim_v=64, n_heads=2, n_kv_groups=2)
+    torch.manual_seed(0)
+    m = NSAAttention(cfg).to(dev, dtype)
+    k, v = (torch.randn(2, 2, 177, 64, device=dev, dtype=dtype, requires_grad=True) for _ in range(2))
+    ps = [k, v, *m.compress_mlp.parameters(), m.pos_embed.weight]
+    gs, res = None, []
+    for on in (False, True):
+        kc, vc, _, _ = m.compress_tokens(k, v)
+        gs = gs or [torch.randn_like(kc), torch.randn_like(vc)]
+        with torch.autocast("cuda", dtype=torch.float16, enabled=on):
+            res.append(torch.autograd.grad([kc, vc], ps, gs))
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+
+
 # the 32-column selection forward: one timestep a wave (32 to 96 heads a group, from 2048 waves on,
 # from 4096 where all of more than 512 keys' blocks fit the slots: the rule's edges from both
 # sides; a partly filled last workgroup; five rows: a lone key has an exact dQ of zero, so no relative error), several that
