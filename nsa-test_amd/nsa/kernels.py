@@ -1139,7 +1139,7 @@ class NSAAttention(torch.nn.Module):
         of = o.transpose(1, 2).reshape(B, H * dv)
         if (_ops.linear_one(B, D, H * dv, of.dtype) and H * dv * of.element_size() % 16 == 0
                 and _plain_linears(of, (self.o_proj, H * dv, D))):
-            out = x.new_empty(B, 1, D)
+            out = of.new_empty(B, 1, D)
             _ops.linear_few(of, [(self.o_proj.weight, self.o_proj.bias, out, D, 0, D, 0)])
         else:
             out = self.o_proj(of.view(B, 1, H * dv))

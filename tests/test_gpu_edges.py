@@ -458,6 +458,30 @@ def test_decode_runs_what_was_replaced(dev, what):
     assert len(calls) == 2 and (res[0] - res[1]).norm() < 1e-2 * res[0].norm()
 
 
+def test_decode_output_in_the_layers_type(dev):
+    """Projections that cast an fp32 token to bf16 before a plain bf16 output projection: the output
+    is of that projection's type, as F.linear's is."""
+    class Cast(torch.nn.Linear):
+        def forward(self, x):
+            return super().forward(x.to(self.weight.dtype))
+
+    cfg = NSAConfig(d_model=64, head_dim_qk=64, head_dim_v=64, n_heads=8, n_kv_groups=2, l_prime=32, n=4, w=40)
+    torch.manual_seed(0)
+    m = NSAAttention(cfg).to(dev, torch.bfloat16).eval()
+    x = torch.randn(2, 37, 64, device=dev).to(torch.bfloat16)
+    res = []
+    for dt in (torch.bfloat16, torch.float32):
+        cache = NSAKVCache(cfg, 2, 40, dev, torch.bfloat16)
+        if dt == torch.float32:
+            for name in ("q_proj", "k_compress", "v_compress", "k_select", "v_select", "k_sliding", "v_sliding"):
+                getattr(m, name).__class__ = Cast
+            m.gate_mlp[0].__class__ = Cast
+        m.prefill(x[:, :35].to(dt), cache)
+        res.append(torch.cat([m.decode(x[:, t:t + 1].to(dt), cache)[0] for t in (35, 36)], 1))
+    assert res[1].dtype == torch.bfloat16
+    assert (res[0].double() - res[1].double()).norm() < 1e-2 * res[0].double().norm()
+
+
 @pytest.mark.parametrize("rows,own", [(32, True), (33, False)])
 def test_decode_output_projection_rule(dev, rows, own, monkeypatch):
     """The output projection of a decode step is F.linear's from the size on at which it is the
