@@ -623,7 +623,8 @@ class _CompressTokens(torch.autograd.Function):
         if torch.is_autocast_enabled("cuda"):  # the call reads the products as tensors of dK's type
             with torch.autocast("cuda", enabled=False):
                 return _CompressTokens.backward(ctx, dK, dV)
-        keys, Y, C, R, W1, W2, E = ctx.saved_tensors
+        # (saved-tensor hooks may hand back other strides or alignments)
+        keys, Y, C, R, W1, W2, E = (_compact(t) for t in ctx.saved_tensors)
         B, G, T, dk, dv, l, d, n_act, n_pad, tm, _ = ctx.dims
         need = ctx.needs_input_grad
         dK, dV = _compact(dK), _compact(dV)

@@ -396,6 +396,33 @@ def test_compress_tokens_backward_under_autocast(dev, dtype):
         assert torch.equal(a, b)
 
 
+def test_compress_tokens_saved_tensor_hooks(dev):
+    """Saved tensors that a hook hands back with other strides (each element twice as far apart)
+    or off their 16-byte alignment give the same gradients."""
+    cfg = NSAConfig(d_model=64, head_dim_qk=64, head_dim_v=64, n_heads=2, n_kv_groups=2)
+    torch.manual_seed(0)
+    m = NSAAttention(cfg).to(dev, torch.bfloat16)
+    k, v = (torch.randn(2, 2, 177, 64, device=dev, dtype=torch.bfloat16, requires_grad=True) for _ in range(2))
+    ps = [k, v, *m.compress_mlp.parameters(), m.pos_embed.weight]
+
+    def strided(x):
+        return torch.stack([x, torch.zeros_like(x)], -1)[..., 0]
+
+    def shifted(x):
+        y = x.new_empty(x.numel() + 1)[1:].view(x.shape)
+        return y.copy_(x)
+
+    gs, res = None, []
+    for unpack in (lambda x: x, strided, shifted):
+        with torch.autograd.graph.saved_tensors_hooks(lambda x: x.detach(), unpack):
+            kc, vc, _, _ = m.compress_tokens(k, v)
+        gs = gs or [torch.randn_like(kc), torch.randn_like(vc)]
+        res.append(torch.autograd.grad([kc, vc], ps, gs))
+    for other in res[1:]:
+        for a, b in zip(other, res[0]):
+            assert torch.equal(a, b)
+
+
 # the 32-column selection forward: one timestep a wave (32 to 96 heads a group, from 2048 waves on,
 # from 4096 where all of more than 512 keys' blocks fit the slots: the rule's edges from both
 # sides; a partly filled last workgroup; five rows: a lone key has an exact dQ of zero, so no relative error), several that
