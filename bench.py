@@ -1,8 +1,8 @@
 #!/usr/bin/env python3
-"""NSA fwd+bwd throughput on one MI355X (BASELINE.json metric).
+"""NSA fwd+bwd throughput on one MI355X.
 
 One step = one forward + backward pass of the NSA attention core at the paper
-configuration (B=1, H=64, G=4, T=8192, dk=192, dv=128, bf16; BASELINE configs[2]):
+configuration (B=1, H=64, G=4, T=8192, dk=192, dv=128, bf16):
 compress_tokens (MLP pooling of K, mean pooling of V), the fused Eq. 8 -> 10 top-n
 selection (l=32, d=16, l'=64, n=16 with 3 fixed blocks), the compression / selection /
 sliding-window (w=512) HIP attention branches, the sigmoid-gated mix, and the backward
@@ -10,9 +10,8 @@ of all of it.  Inputs (q, k, v, dO ~ N(0,1)/sqrt(d), gate logits, N(0,0.02) MLP
 weights) are synthetic, in the layouts NSAAttention's projections produce ([B,H,T,d]
 views of [B,T,H,d] storage), and resident in HBM before the timed region.
 
-The JSON line also carries the long-context configuration (T=32768, configs[3]) as
-`secondary`, the sliding-window branch alone at configs[1] as `config2_sliding`, a
-per-kernel breakdown, per-branch fwd and fwd+bwd tokens/s, the roofline of the dominant kernel (timed with
+The JSON line also carries the long-context configuration (T=32768) as `secondary`, the
+sliding-window branch alone (B=2, H=8, T=4096, dk=dv=64) as `config2_sliding`, a per-kernel breakdown, per-branch fwd and fwd+bwd tokens/s, the roofline of the dominant kernel (timed with
 HIP events inside the timed region) and a CPU baseline (the C oracle on all host cores,
 one thread each, on a sample of query rows, extrapolated linearly: each row's work is
 independent).

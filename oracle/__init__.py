@@ -1,7 +1,7 @@
 """CPU oracle for the NSA hot path -- TEST INFRASTRUCTURE ONLY.
 
 Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may import this
-package, and only as the checker of the HIP path.  The product (the `nsa` package and
+package, and only to compare the HIP path with.  The product (the `nsa` package and
 libnsa_hip.so) never imports or calls it.
 
 Contents

@@ -1,7 +1,7 @@
 /*
  * CPU ORACLE FOR TESTS ONLY.  This file is test infrastructure: it is compiled into
  * oracle/liboracle.so and used by tests/, __graft_entry__.smoke() and the
- * cpu_baseline leg of bench.py as the checker of the HIP path.  The product
+ * cpu_baseline leg of bench.py to compare the HIP path with.  The product
  * (libnsa_hip.so and the nsa package) never links, loads or calls it.
  *
  * It restates, in plain C, the semantics of the reference's NSA hot path:

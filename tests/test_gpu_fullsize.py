@@ -162,7 +162,7 @@ def test_fullsize_selection(dev, name):
 
 
 def test_config2_sliding(dev):
-    """Benchmark config 2: sliding window alone, B=2, H=8,
+    """Benchmark configuration 2: sliding window alone, B=2, H=8,
     G=2, T=4096, dk=dv=64, w=512, bf16; 320 sampled rows per batch entry."""
     c = dict(B=2, H=8, G=2, T=4096, dk=64, dv=64)
     q, kp, v, do = _inputs(c, 400, dev)

@@ -1,4 +1,4 @@
-"""CPU tests pinning the oracle (the checker of the HIP path).
+"""CPU tests pinning the oracle.
 
 Each oracle function is checked against something independent of its own code:
 golden vectors written by the reference implementation (tests/golden), known-answer
